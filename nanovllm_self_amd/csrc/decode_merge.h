@@ -44,61 +44,94 @@ struct DecodeArgs {
 // First tile of decode group k of Kw over T tiles.
 __device__ __forceinline__ int group_start(int T, int Kw, int k) { return (int)((int64_t)k * T / Kw); }
 
-// Heads c0 + lane / 16 + 4 i (i < NH) of the row: NH head passes at once,
-// so a group of more than four heads waits for its partials' loads once
-// rather than once per four heads.
+// The merge's state of head c0 + lane / 16 + 4 i (i < NH) of a row: running
+// max, sum and the lane's eight output elements, 8 (lane % 16) .. + 7.  NH
+// head passes at once, so a group of more than four heads waits for its
+// partials' loads once rather than once per four heads.
 template <int NH>
-__device__ __forceinline__ void merge_heads(const DecodeArgs& a, int h, int k, int k_last, int slot_k, int q_row,
-                                            int c0, int lane) {
+struct MergeState {
+  float M[NH], L[NH];
+  f32x4 o0[NH], o1[NH];
+};
+
+template <int NH>
+__device__ __forceinline__ void merge_clear(MergeState<NH>& s) {
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    s.M[i] = -INFINITY;
+    s.L[i] = 0.0f;
+    s.o0[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    s.o1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
+// Adds the partial (m, l, o0, o1) to head pass i.
+template <int NH>
+__device__ __forceinline__ void merge_add(MergeState<NH>& s, int i, float m, float l, f32x4 o0, f32x4 o1) {
+  const float m_new = fmaxf(s.M[i], m);
+  const float al = s.M[i] == -INFINITY ? 0.0f : fast_exp2(s.M[i] - m_new);
+  const float be = m == -INFINITY ? 0.0f : fast_exp2(m - m_new);
+  s.M[i] = m_new;
+  s.L[i] = s.L[i] * al + l * be;
+  s.o0[i] = s.o0[i] * al + o0 * be;
+  s.o1[i] = s.o1[i] * al + o1 * be;
+}
+
+// A row split across groups k .. k_last: output row, the slot of group k's
+// partial (the others' is 0).
+struct MergeRow {
+  int k, h, k_last, slot_k, q_row;
+};
+
+// Partials whose loads are in flight together (a run).
+constexpr int kMergeRun = 4;
+
+// Adds the partials of groups first .. k_last in runs, the next run starting
+// `stride` groups after the last one's start.
+template <int NH>
+__device__ __forceinline__ void merge_partials(const DecodeArgs& a, const MergeRow& r, int first, int stride, int c0,
+                                               int lane, MergeState<NH>& s) {
   const int j = lane & 15;
   int cc[NH];
-  bool use[NH];
-  float M[NH], L[NH];
-  f32x4 acc0[NH], acc1[NH];
 #pragma unroll
   for (int i = 0; i < NH; ++i) {
     const int c = c0 + (lane >> 4) + 4 * i;
-    use[i] = c < a.g;
-    cc[i] = use[i] ? c : 0;
-    M[i] = -INFINITY;
-    L[i] = 0.0f;
-    acc0[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    acc1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    cc[i] = c < a.g ? c : 0;
   }
-  for (int x0 = k; x0 <= k_last; x0 += 4) {
-    f32x2 ml[4][NH];
-    f32x4 o0[4][NH], o1[4][NH];
+  for (int x0 = first; x0 <= r.k_last; x0 += stride) {
+    f32x2 ml[kMergeRun][NH];
+    f32x4 o0[kMergeRun][NH], o1[kMergeRun][NH];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int x = min(x0 + u, k_last);
+    for (int u = 0; u < kMergeRun; ++u) {
+      const int x = min(x0 + u, r.k_last);
 #pragma unroll
       for (int i = 0; i < NH; ++i) {
-        const int64_t base = (((int64_t)x * a.Hkv + h) * 2 + (x == k ? slot_k : 0)) * a.g + cc[i];
+        const int64_t base = (((int64_t)x * a.Hkv + r.h) * 2 + (x == r.k ? r.slot_k : 0)) * a.g + cc[i];
         ml[u][i] = *reinterpret_cast<const f32x2*>(a.ws_ml + base * 2);
         o0[u][i] = *reinterpret_cast<const f32x4*>(a.ws_o + base * kHeadDim + 8 * j);
         o1[u][i] = *reinterpret_cast<const f32x4*>(a.ws_o + base * kHeadDim + 8 * j + 4);
       }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (x0 + u > k_last) break;
+    for (int u = 0; u < kMergeRun; ++u) {
+      if (x0 + u > r.k_last) break;
 #pragma unroll
-      for (int i = 0; i < NH; ++i) {
-        const float m_new = fmaxf(M[i], ml[u][i][0]);
-        const float al = M[i] == -INFINITY ? 0.0f : fast_exp2(M[i] - m_new);
-        const float be = ml[u][i][0] == -INFINITY ? 0.0f : fast_exp2(ml[u][i][0] - m_new);
-        M[i] = m_new;
-        L[i] = L[i] * al + ml[u][i][1] * be;
-        acc0[i] = acc0[i] * al + o0[u][i] * be;
-        acc1[i] = acc1[i] * al + o1[u][i] * be;
-      }
+      for (int i = 0; i < NH; ++i) merge_add<NH>(s, i, ml[u][i][0], ml[u][i][1], o0[u][i], o1[u][i]);
     }
   }
+}
+
+// Normalises and writes the row's heads.
+template <int NH>
+__device__ __forceinline__ void merge_write(const DecodeArgs& a, const MergeRow& r, int c0, int lane,
+                                            const MergeState<NH>& s) {
+  const int j = lane & 15;
 #pragma unroll
   for (int i = 0; i < NH; ++i) {
-    if (!use[i]) continue;
-    const float inv = L[i] > 0.0f ? 1.0f / L[i] : 0.0f;
-    const f32x4 x0 = acc0[i] * inv, x1 = acc1[i] * inv;
+    const int c = c0 + (lane >> 4) + 4 * i;
+    if (c >= a.g) continue;
+    const float inv = s.L[i] > 0.0f ? 1.0f / s.L[i] : 0.0f;
+    const f32x4 x0 = s.o0[i] * inv, x1 = s.o1[i] * inv;
     u32x4 v;
     if (a.f16) {
       v[0] = pack_f16x2(x0[0], x0[1]);
@@ -111,35 +144,130 @@ __device__ __forceinline__ void merge_heads(const DecodeArgs& a, int h, int k, i
       v[2] = pack_bf16x2(x1[0], x1[1]);
       v[3] = pack_bf16x2(x1[2], x1[3]);
     }
-    *reinterpret_cast<u32x4*>(a.out + (int64_t)q_row * a.out_ts + (int64_t)(h * a.g + cc[i]) * a.out_hs + 8 * j) = v;
+    *reinterpret_cast<u32x4*>(a.out + (int64_t)r.q_row * a.out_ts + (int64_t)(r.h * a.g + c) * a.out_hs + 8 * j) = v;
   }
 }
 
-// Log-sum-exp merge of the rows split across groups.  Wave k Hkv + h owns kv
-// head h of the row recorded by decode wave k Hkv + h (the row that crosses
-// the boundary after group k and starts inside group k's range); its
-// partials sit in wave k Hkv + h (the recorded slot) and in waves x Hkv + h
-// for groups x = k + 1 .. k_last (slot 0).  Lane l serves head 4 p + l / 16
-// of the group (pass p) and head_dim elements 8 (l % 16) .. + 7; one pass
-// over the partials keeps a running max, sum and output, with the loads of
-// four partials in flight at a time, for up to two head passes together.
-__device__ __forceinline__ void merge_split_row(const DecodeArgs& a, int unit, int lane) {
-  const int k = unit / a.Hkv, h = unit - k * a.Hkv;
+template <int NH>
+__device__ __forceinline__ void merge_heads(const DecodeArgs& a, const MergeRow& r, int c0, int lane) {
+  MergeState<NH> s;
+  merge_clear<NH>(s);
+  merge_partials<NH>(a, r, r.k, kMergeRun, c0, lane, s);
+  merge_write<NH>(a, r, c0, lane, s);
+}
+
+// A merge work-group is sixteen waves, one unit each.  A row of up to
+// kMergeAlone partials (a run or two) is merged by its wave; the longer
+// ones by teams of waves, the work-group's waves shared evenly among up to
+// kMergeTeams of them at a time.
+constexpr int kMergeWaves = 16;
+constexpr int kMergeAlone = 8;
+constexpr int kMergeTeams = 4;
+
+struct MergeLds {
+  MergeRow rows[kMergeWaves];  // k_last < 0: not a row for a team
+  f32x2 ml[kMergeWaves][64];
+  f32x4 o[kMergeWaves][2][64];
+};
+
+// Work-groups of a merge launch of `units` groups and kv heads.
+inline int merge_wgs(int units, int Hkv) { return (units / Hkv + kMergeWaves - 1) / kMergeWaves * Hkv; }
+
+// One head pass c0 .. c0 + 4 NH - 1 of the row r by `waves` waves (this wave
+// the `part`-th of them, w among the work-group's): each takes every
+// waves-th run of partials, and the first adds the others' states
+// through LDS and writes.  Every wave of the work-group calls it (two
+// barriers a head); r.k_last < 0 adds and writes nothing.
+template <int NH>
+__device__ __forceinline__ void merge_pass(const DecodeArgs& a, const MergeRow& r, int w, int part, int waves, int c0,
+                                           int lane, MergeLds& lds) {
+  MergeState<NH> s;
+  merge_clear<NH>(s);
+  if (r.k_last >= 0) merge_partials<NH>(a, r, r.k + kMergeRun * part, kMergeRun * waves, c0, lane, s);
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    lds.ml[w][lane] = f32x2{s.M[i], s.L[i]};
+    lds.o[w][0][lane] = s.o0[i];
+    lds.o[w][1][lane] = s.o1[i];
+    __syncthreads();
+    if (part == 0 && r.k_last >= 0)
+      for (int y = 1; y < waves; ++y) {
+        const f32x2 ml = lds.ml[w + y][lane];
+        merge_add<NH>(s, i, ml[0], ml[1], lds.o[w + y][0][lane], lds.o[w + y][1][lane]);
+      }
+    __syncthreads();
+  }
+  if (part == 0 && r.k_last >= 0) merge_write<NH>(a, r, c0, lane, s);
+}
+
+// The row merge unit `unit` = k Hkv + h owns: kv head h of the row recorded
+// by decode wave k Hkv + h (the row that crosses the boundary after group k
+// and starts inside group k's range); its partials sit in wave k Hkv + h
+// (the recorded slot) and in waves x Hkv + h for groups x = k + 1 .. k_last
+// (slot 0).  k_last = -1: none.
+__device__ __forceinline__ MergeRow merge_row(const DecodeArgs& a, int unit, int units) {
+  MergeRow r = {0, 0, -1, 0, 0};
+  if (unit >= units) return r;
+  r.k = unit / a.Hkv;
+  r.h = unit - r.k * a.Hkv;
   // Groups k >= Kw - 1 merge nothing (a launch may hold more merge waves
   // than the decode had groups; their records are not this call's).
-  const int Kw = __builtin_amdgcn_readfirstlane(a.ws_rec[1]);
-  if (k >= Kw - 1) return;
+  const int T = __builtin_amdgcn_readfirstlane(a.ws_rec[0]), Kw = __builtin_amdgcn_readfirstlane(a.ws_rec[1]);
+  if (r.k >= Kw - 1) return r;
   const int32_t* rec = a.ws_rec + 4 + 4 * unit;
-  if (__builtin_amdgcn_readfirstlane(rec[3]) == 0) return;
-  const int T = __builtin_amdgcn_readfirstlane(a.ws_rec[0]);
-  const int q_row = __builtin_amdgcn_readfirstlane(rec[0]);
-  const int last = group_start(T, Kw, k + 1) - 1 + __builtin_amdgcn_readfirstlane(rec[1]);  // the row's last tile
-  const int k_last = (int)(((int64_t)(last + 1) * Kw - 1) / T);
-  const int slot_k = __builtin_amdgcn_readfirstlane(rec[2]);
-  if (a.g <= 4) {
-    merge_heads<1>(a, h, k, k_last, slot_k, q_row, 0, lane);
-  } else {
-    for (int c0 = 0; c0 < a.g; c0 += 8) merge_heads<2>(a, h, k, k_last, slot_k, q_row, c0, lane);
+  if (__builtin_amdgcn_readfirstlane(rec[3]) == 0) return r;
+  r.q_row = __builtin_amdgcn_readfirstlane(rec[0]);
+  r.slot_k = __builtin_amdgcn_readfirstlane(rec[2]);
+  const int last = group_start(T, Kw, r.k + 1) - 1 + __builtin_amdgcn_readfirstlane(rec[1]);  // the row's last tile
+  r.k_last = (int)(((int64_t)(last + 1) * Kw - 1) / T);
+  return r;
+}
+
+// Log-sum-exp merge of the rows split across groups, by work-group `wg`
+// (every wave of the work-group calls it): kv head wg % Hkv of the sixteen
+// groups from 16 (wg / Hkv), one a wave, so the kv heads of one row fall to
+// different work-groups and a work-group reads neighbouring groups'
+// partials.  Lane l
+// serves head 4 p + l / 16 of the group (pass p) and head_dim elements
+// 8 (l % 16) .. + 7; a pass over the partials keeps a running max, sum and
+// output, for up to two head passes together.
+// What bounds it is the chain of dependent loads, about 2 us a run of four
+// partials.  With one wave a row throughout, a single conversation of 20 011
+// keys, whose row is split across all 156 groups, took 62.6 us here (now
+// 8.7), 48 rows of 256 .. 32 768 keys with 8 heads a group 14.2 us (12.9).
+// A team costs two barriers: rows of up to eight partials stay with one wave
+// (64 rows of 2 .. 8 K keys: 7.1 us; 12.5 with teams from five partials on;
+// the 48 rows: 16.0 us with teams only from thirteen on).
+__device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units, int wg, MergeLds& lds) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int k = wg / a.Hkv * kMergeWaves + w;
+  MergeRow r = merge_row(a, k * a.Hkv + wg % a.Hkv, units);
+  if (r.k_last >= 0 && r.k_last - r.k < kMergeAlone) {
+    if (a.g <= 4) {
+      merge_heads<1>(a, r, 0, lane);
+    } else {
+      for (int c0 = 0; c0 < a.g; c0 += 8) merge_heads<2>(a, r, c0, lane);
+    }
+    r.k_last = -1;
+  }
+  if (lane == 0) lds.rows[w] = r;
+  __syncthreads();
+  // The longer rows, the same for every wave: one bit a unit.
+  uint32_t rest = (uint32_t)__ballot(lane < kMergeWaves && lds.rows[lane & (kMergeWaves - 1)].k_last >= 0);
+  while (rest) {
+    const int n = __popc(rest);
+    const int waves = n == 1 ? kMergeWaves : n == 2 ? kMergeWaves / 2 : kMergeWaves / kMergeTeams;
+    const int team = w / waves;
+    MergeRow x = {0, 0, -1, 0, 0};
+    for (int t = 0; t < kMergeWaves / waves && rest; ++t) {
+      if (t == team) x = lds.rows[__ffs(rest) - 1];
+      rest &= rest - 1;
+    }
+    if (a.g <= 4) {
+      merge_pass<1>(a, x, w, w % waves, waves, 0, lane, lds);
+    } else {
+      for (int c0 = 0; c0 < a.g; c0 += 8) merge_pass<2>(a, x, w, w % waves, waves, c0, lane, lds);
+    }
   }
 }
 

@@ -76,13 +76,12 @@ void paged_decode_kernel(DecodeArgs a, const int32_t* __restrict__ bt, const int
 // The merge of split rows as a launch of its own (decode-only calls, and
 // after a prefill launch that streamed the decode rows); calls whose decode
 // has a launch of its own beside prefill rows run it in the plan launch
-// (merge_split_row).
+// (merge_split_rows).
 // Sixteen merge waves a work-group: a launch of a few large work-groups
 // is dispatched sooner than one of many single-wave ones.
-constexpr int kMergeWaves = 16;
 __global__ __launch_bounds__(64 * kMergeWaves) void decode_merge_kernel(DecodeArgs a, int units) {
-  const int unit = (int)blockIdx.x * kMergeWaves + (int)(threadIdx.x >> 6);
-  if (unit < units) merge_split_row(a, __builtin_amdgcn_readfirstlane(unit), threadIdx.x & 63);
+  __shared__ MergeLds lds;
+  merge_split_rows(a, units, (int)blockIdx.x, lds);
 }
 
 int64_t decode_workspace_bytes(int max_waves, int group) {
@@ -114,8 +113,7 @@ DecodeArgs decode_args(const AttnParams& P, int max_waves, void* partials) {
 int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream) {
   if (groups <= 1) return NVS_OK;
   const int units = (groups - 1) * a.Hkv;
-  hipLaunchKernelGGL(decode_merge_kernel, dim3((units + kMergeWaves - 1) / kMergeWaves), dim3(64 * kMergeWaves), 0,
-                     stream, a, units);
+  hipLaunchKernelGGL(decode_merge_kernel, dim3(merge_wgs(units, a.Hkv)), dim3(64 * kMergeWaves), 0, stream, a, units);
   return check_launch("decode_merge");
 }
 

@@ -94,6 +94,7 @@ __device__ __forceinline__ void row_work(const PlanArgs& a, int b, bool& dec, in
 
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanWaves = kPlanThreads / 64;
+static_assert(kPlanWaves == kMergeWaves, "a work-group of the plan launch holds the merge's waves");
 
 // Sums of three floats per thread over the 1024-thread work-group (every
 // thread gets them).  Two barriers.
@@ -160,14 +161,17 @@ struct PlanRows {
 // launch left its merge to this one) merge the decode rows split across
 // groups, one merge wave per wave.
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeArgs m, int merge_units) {
+  __shared__ union Lds {
+    struct { int scan[kPlanWaves]; float sum[kPlanWaves][3]; PlanRows rows; } plan;
+    MergeLds merge;
+  } lds;
   if (blockIdx.x > 0) {
-    const int unit = (blockIdx.x - 1) * kPlanWaves + (threadIdx.x >> 6);
-    if (unit < merge_units) merge_split_row(m, __builtin_amdgcn_readfirstlane(unit), threadIdx.x & 63);
+    merge_split_rows(m, merge_units, (int)blockIdx.x - 1, lds.merge);
     return;
   }
-  __shared__ int scan_lds[kPlanWaves];
-  __shared__ float sum_lds[kPlanWaves][3];
-  __shared__ PlanRows rows;
+  int* scan_lds = lds.plan.scan;
+  float (*sum_lds)[3] = lds.plan.sum;
+  PlanRows& rows = lds.plan.rows;
   const int tid = threadIdx.x;
   const Plan& pl = a.plan;
   if (tid < 8) pl.hdr->prefill_next[tid] = 0;
@@ -331,7 +335,7 @@ int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t s
     m = merge->a;
     units = merge->units;
   }
-  const int grid = 1 + (units + kPlanWaves - 1) / kPlanWaves;
+  const int grid = 1 + (units > 0 ? merge_wgs(units, m.Hkv) : 0);
   hipLaunchKernelGGL(plan_kernel, dim3(grid), dim3(kPlanThreads), 0, stream, a, m, units);
   return check_launch("plan");
 }
