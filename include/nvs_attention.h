@@ -211,6 +211,19 @@ int64_t nvs_attention_workspace_bytes_cache(int num_seqs, int max_seqlen_q,
                                             int block_size, int cache_dtype);
 
 /*
+ * Bytes beyond nvs_attention_workspace_bytes_cache(...) (paged calls) or
+ * nvs_attention_workspace_bytes(...) (varlen calls) with which a call's
+ * prefill rows may be split along their keys, where a batch has too few
+ * query tiles for the chip (a short new turn over a long cached prefix): the
+ * parts' fp32 accumulators, at most 768 slots of 132 KiB.  0 where no split
+ * can help.  Optional: a smaller workspace serves the call unsplit.
+ * num_tokens <= 0: unknown (an upper bound); num_kv_heads <= 0: unknown.
+ */
+int64_t nvs_attention_split_bytes(int num_seqs, int64_t num_tokens,
+                                  int max_seqlen_q, int max_seqlen_k,
+                                  int num_heads, int num_kv_heads);
+
+/*
  * Causal varlen attention over a paged KV cache: the paged call of
  * prefill_flashattn (reference attention.py:356-375,
  * flash_attn_varlen_func(..., block_table=...)) and equally the

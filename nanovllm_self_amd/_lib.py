@@ -49,6 +49,7 @@ SIGNATURES = {
     ),
     "nvs_attention_workspace_bytes": (_L, [_I, _I, _I, _I, _I, _I, _I]),
     "nvs_attention_workspace_bytes_cache": (_L, [_I, _I, _I, _I, _I, _I, _I, _I]),
+    "nvs_attention_split_bytes": (_L, [_I, _L, _I, _I, _I, _I]),
     "nvs_paged_attention": (
         _I,
         [

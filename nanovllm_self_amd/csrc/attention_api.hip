@@ -112,6 +112,30 @@ static bool shadow_serves(const AttnParams& P) {
   return prefill_mx_serves(C);
 }
 
+// The prefill tokens a batch holds at least (a row of one token may be a
+// decode row), as units of the tile-loop kernel: with kSplitMaxUnits of them
+// its entries are not split along the keys, and no room is asked for.
+static bool may_split(int num_seqs, int64_t num_tokens, int units, int pbm) {
+  return (num_tokens - num_seqs) / pbm * units < kSplitMaxUnits;
+}
+
+// Entries of a call served by the tile-loop kernel split along their keys,
+// if the workspace holds their slots after `offset` bytes; job->slots = 0 if
+// not.
+static SplitJob split_job(const AttnParams& P, const Plan& plan, int64_t offset, int wgs) {
+  SplitJob job = {};
+  const int units = prefill_mx_units(P.Hq, P.Hkv);
+  const int64_t slots = split_slots(P.B, plan.ntq, P.max_seqlen_k, units);
+  offset = align256(offset);
+  if (slots <= 0 || !may_split(P.B, P.T, units, plan.pbm) ||
+      P.ws_bytes < offset + split_bytes(P.B, plan.ntq, slots))
+    return job;
+  job.at = split_at((char*)P.ws + offset, P.B, plan.ntq);
+  job.slots = (int)slots;
+  job.wgs = wgs;
+  return job;
+}
+
 // Work-groups of a prefill launch that also streams the call's decode rows
 // (0: the decode keeps a launch of its own): every work-group slot of the
 // device, when the tile-loop kernel serves the prefill rows (from the cache,
@@ -174,6 +198,18 @@ extern "C" int64_t nvs_attention_workspace_bytes_cache(int num_seqs, int max_seq
       num_heads % num_kv_heads != 0)
     return base;
   return align256(base) + shadow_bytes(num_seqs, max_seqlen_k, num_kv_heads);
+}
+
+extern "C" int64_t nvs_attention_split_bytes(int num_seqs, int64_t num_tokens, int max_seqlen_q, int max_seqlen_k,
+                                             int num_heads, int num_kv_heads) {
+  if (num_seqs <= 0 || num_heads <= 0 || max_seqlen_q <= 1) return 0;
+  const bool known = num_kv_heads > 0 && num_heads % num_kv_heads == 0;
+  const int units = known ? prefill_mx_units(num_heads, num_kv_heads) : num_heads;
+  const int pbm = known ? prefill_mx_positions(num_heads / num_kv_heads) : prefill_mx_positions(8);
+  if (num_tokens > 0 && !may_split(num_seqs, num_tokens, units, pbm)) return 0;
+  const int ntq = prefill_tiles(max_seqlen_q, pbm);
+  const int64_t slots = split_slots(num_seqs, ntq, max_seqlen_k, units);
+  return slots > 0 ? 256 + split_bytes(num_seqs, ntq, slots) : 0;
 }
 
 static int check_workspace(const AttnParams& P, const char* who) {
@@ -252,19 +288,21 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
     co.kv = P.cache_dtype;
     co.groups = std::min(8 * ((co_wgs / 2) / P.Hkv), max_waves / P.Hkv);
     co.wgs = co_wgs;
+    const int64_t base = align256(attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv));
+    const SplitJob split =
+        split_job(P, plan, base + (shadow ? shadow_bytes(P.B, P.max_seqlen_k, P.Hkv) : 0), co_wgs);
+    const SplitJob* sp = split.slots > 0 ? &split : nullptr;
     if (!shadow) {
-      rc = launch_plan(P, plan, /*paged=*/true, s, nullptr, nullptr, &co);
+      rc = launch_plan(P, plan, /*paged=*/true, s, nullptr, nullptr, &co, sp);
       if (rc != NVS_OK) return rc;
-      rc = launch_prefill_mx(P, plan, s, &co);
+      rc = launch_prefill_mx(P, plan, s, &co, sp);
       if (rc != NVS_OK) return rc;
-      return launch_decode_merge(co.a, co.groups, s);
+      return launch_decode_merge(co.a, co.groups, s, &P, &plan, sp);
     }
     // Code cache: the prefill reads the bf16 copy, the decode waves the
     // codes; they run whichever prefill kernel the plan lets serve.
-    const ShadowLayout sh = shadow_at((char*)workspace + align256(attention_workspace_bytes(
-                                          P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv)),
-                                      P.B, P.max_seqlen_k, P.Hkv);
-    rc = launch_plan(P, plan, /*paged=*/true, s, &sh, nullptr, &co);
+    const ShadowLayout sh = shadow_at((char*)workspace + base, P.B, P.max_seqlen_k, P.Hkv);
+    rc = launch_plan(P, plan, /*paged=*/true, s, &sh, nullptr, &co, sp);
     if (rc != NVS_OK) return rc;
     rc = launch_shadow_fill(P, plan, sh, s);
     if (rc != NVS_OK) return rc;
@@ -272,7 +310,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
     C.kc = sh.k; C.vc = sh.v; C.cache_dtype = NVS_DTYPE_BF16; C.ks = nullptr; C.vs = nullptr;
     C.bt = sh.table; C.bt_stride = sh.ST; C.bs = kShadowTile; C.NB = sh.cap;
     C.gate = &plan.hdr->shadow_on; C.gate_run = 1;
-    rc = launch_prefill_mx(C, plan, s, &co);
+    rc = launch_prefill_mx(C, plan, s, &co, sp);
     if (rc != NVS_OK) return rc;
     if ((int64_t)sh.cap < (int64_t)P.B * sh.ST) {
       AttnParams F = P;
@@ -280,7 +318,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
       rc = launch_prefill(F, plan, s);
       if (rc != NVS_OK) return rc;
     }
-    return launch_decode_merge(co.a, co.groups, s);
+    return launch_decode_merge(co.a, co.groups, s, &P, &plan, sp);
   }
   // With prefill rows the plan launch also merges the split decode rows.
   MergeJob merge;
@@ -415,9 +453,18 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
   if (rc != NVS_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
   const Plan plan = make_plan(workspace, P);
-  rc = launch_plan(P, plan, /*paged=*/false, s);
+  if (!prefill_mx_serves(P)) {
+    rc = launch_plan(P, plan, /*paged=*/false, s);
+    return rc != NVS_OK ? rc : launch_prefill(P, plan, s);
+  }
+  const SplitJob split = split_job(P, plan, attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv),
+                                   prefill_mx_wgs(P, plan));
+  const SplitJob* sp = split.slots > 0 ? &split : nullptr;
+  rc = launch_plan(P, plan, /*paged=*/false, s, nullptr, nullptr, nullptr, sp);
   if (rc != NVS_OK) return rc;
-  return launch_prefill_any(P, plan, s);
+  rc = launch_prefill_mx(P, plan, s, nullptr, sp);
+  if (rc != NVS_OK) return rc;
+  return sp ? launch_decode_merge(DecodeArgs{}, 0, s, &P, &plan, sp) : NVS_OK;
 }
 
 extern "C" int nvs_varlen_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride,

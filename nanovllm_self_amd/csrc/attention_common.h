@@ -10,6 +10,8 @@ constexpr int kHeadDim = 128;    // head_dim served by the attention kernels
 #define NVS_DECODE_WAVES_PER_EU 2
 #endif
 constexpr int kDecodeWavesPerEU = NVS_DECODE_WAVES_PER_EU;  // decode waves per SIMD
+inline int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
+
 constexpr int kDecodeTile = 32;         // keys per decode tile (one unit of decode work)
 constexpr int kDecodeMaxWaves = 2048;   // decode waves per call at most (256 CUs x 8)
 constexpr int kDecodeMinUnits = 4;      // fewest tiles a decode group is given
@@ -99,21 +101,25 @@ struct PlanHeader {
   int shadow_tiles;     // code caches: 64-key tiles of the prefill rows' bf16 copy
   int shadow_on;        // 1: the copy fits and the tile-loop kernel serves the prefill
   int dec_wgs;          // work-groups of the prefill launch that stream the decode rows first
-  int pad[52];          // keeps the list 256-byte aligned
+  int n_split;          // list entries split along the keys (SplitRow records)
+  int pad[51];          // keeps the list 256-byte aligned
 };
 static_assert(sizeof(PlanHeader) == 256, "plan header is one 256-byte line");
 
 // What a work-group of the MFMA prefill kernel needs to start a list entry,
-// in one 64-byte load: the entry, its sequence's query and key ranges,
+// in one 64-byte load: the entry's first partial slot (-1: the entry covers
+// all its rows' keys and writes the output), its sequence's query and key ranges,
 // (paged) the block ids of its first three 64-key tiles (-1: missing), and
 // what the kernel derives from them per entry: the entry's first query
 // position p0, the 64-key tiles its rows see, the key rows its fills may
 // read (local mode: never past the k / v tensors), K - L, the first key row
-// clamped into the local k / v, the sequence and the bytes of its
-// block-table row the kernel may read.
+// clamped into the local k / v, the sequence, the bytes of its block-table
+// row the kernel may read and the byte in it of the entry's first block.  An
+// entry of a part of the keys (64 t0 ..) is an entry over the keys from there
+// on: its tiles, blocks, kf, off and k0c count from key 64 t0.
 struct PlanRecord {
-  int item, q0, L, k0, K, blk0, blk1, blk2;
-  int p0, ntiles, kf, off, k0c, b, bt_bytes, pad;
+  int part, q0, L, k0, K, blk0, blk1, blk2;
+  int p0, ntiles, kf, off, k0c, b, bt_bytes, bt_off;
 };
 static_assert(sizeof(PlanRecord) == 64, "plan record is 64 bytes");
 
@@ -125,7 +131,62 @@ struct Plan {
   int pbm;          // query positions per prefill tile
 };
 
-inline int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
+// ---------------------------------------------------------------------------
+// Prefill entries split along the keys (the tile-loop kernel): where a batch
+// has fewer units than the chip has work-groups, or few and uneven ones (a
+// short new turn over a long cached prefix), the deepest unit alone bounds
+// the call.  The plan then cuts the entries into parts of about equal numbers
+// of key tiles; a part's units leave their accumulators, running max and sum
+// (fp32) in a slot of the workspace each, and the launch that merges the
+// split decode rows merges them too.
+// ---------------------------------------------------------------------------
+constexpr int kSplitSlots = 768;        // partial slots at most: three rounds of the chip's work-groups
+constexpr int kSplitMaxUnits = 1024;    // units from which a batch fills the chip without parts
+constexpr int kSplitMaxEntries = 1024;  // list entries the plan weighs, one a thread
+constexpr int kSplitMinTiles = 8;       // fewest key tiles a part is given
+constexpr int kPartWaveBytes = 33792;   // one wave's part of a slot: O (64 rows x 128), m, l in fp32
+constexpr int kPartBytes = 4 * kPartWaveBytes;
+
+// A split entry for the merge: its first slot, parts (slots apart: the units
+// of an entry), first query row, new tokens and first query position.
+struct SplitRow {
+  int slot, parts, q0, L, p0;
+};
+
+struct SplitLayout {
+  PlanRecord* rec;  // the list's records, with room for the parts
+  SplitRow* rows;   // [kSplitMaxEntries]
+  char* slots;      // [kSplitSlots] of kPartBytes
+};
+
+// Slots a batch can use: none where no row can hold two parts.
+inline int64_t split_slots(int B, int ntq, int max_seqlen_k, int units_per_entry) {
+  const int64_t tiles = ((int64_t)max_seqlen_k + 63) / 64;
+  if (tiles < 2 * kSplitMinTiles || tiles > (1 << 20) || (int64_t)B * ntq > (1 << 16)) return 0;
+  const int64_t most = (int64_t)B * ntq * units_per_entry * (tiles / kSplitMinTiles);
+  return most < kSplitSlots ? most : kSplitSlots;
+}
+inline int64_t split_bytes(int B, int ntq, int64_t slots) {
+  if (slots <= 0) return 0;
+  return align256(((int64_t)B * ntq + kSplitSlots) * (int64_t)sizeof(PlanRecord)) +
+         align256(kSplitMaxEntries * (int64_t)sizeof(SplitRow)) + slots * kPartBytes;
+}
+inline SplitLayout split_at(void* p, int B, int ntq) {
+  SplitLayout s;
+  char* c = (char*)p;
+  s.rec = (PlanRecord*)c;
+  c += align256(((int64_t)B * ntq + kSplitSlots) * (int64_t)sizeof(PlanRecord));
+  s.rows = (SplitRow*)c;
+  s.slots = c + align256(kSplitMaxEntries * (int64_t)sizeof(SplitRow));
+  return s;
+}
+
+// What the plan, the prefill launch and the merge need of it.
+struct SplitJob {
+  SplitLayout at;
+  int slots;  // 0: entries are not split
+  int wgs;    // work-groups of the prefill launch
+};
 
 // Decode waves a call may use: Hkv per group, at most kDecodeMaxWaves in
 // all, and no more groups than the tiles there can be (B rows x
@@ -265,7 +326,7 @@ struct CoDecode;
 // decode waves' header.
 int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t stream,
                 const ShadowLayout* shadow = nullptr, const MergeJob* merge = nullptr,
-                const CoDecode* co = nullptr);
+                const CoDecode* co = nullptr, const SplitJob* split = nullptr);
 // Rates the plan sizes the co-scheduled decode with: decode bytes per
 // second of one CU beside the prefill and of the whole chip, prefill FLOP
 // per second of one CU, and the fraction of the call by which the decode
@@ -285,17 +346,22 @@ int launch_decode(const AttnParams& P, int max_waves, int waves, void* partials,
 // and the merge of rows split across `groups` decode groups as a launch.
 struct DecodeArgs;
 DecodeArgs decode_args(const AttnParams& P, int max_waves, void* partials);
-int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream);
+// With `split`, the same launch merges the prefill rows' parts.
+int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream, const AttnParams* P = nullptr,
+                        const Plan* plan = nullptr, const SplitJob* split = nullptr);
 int launch_prefill(const AttnParams& P, const Plan& plan, hipStream_t stream);
 // The MFMA tile-loop prefill kernel (paged_prefill_mx.hip): whether it serves
 // a call, its query positions per work item for a group of g query heads,
 // and its launch.
 bool prefill_mx_serves(const AttnParams& P);
 int prefill_mx_positions(int g);
+int prefill_mx_units(int Hq, int Hkv);  // units of a list entry
+int prefill_mx_wgs(const AttnParams& P, const Plan& plan);  // work-groups of a launch without decode rows
 // With `co`, the launch's first work-groups stream the call's decode rows
 // before they join the prefill (co->kv: the cache type of the decode rows,
 // which a code cache's prefill reads through its bf16 copy); the plan has
 // sized their number for co->wgs work-groups.
-int launch_prefill_mx(const AttnParams& P, const Plan& plan, hipStream_t stream, const CoDecode* co = nullptr);
+int launch_prefill_mx(const AttnParams& P, const Plan& plan, hipStream_t stream, const CoDecode* co = nullptr,
+                      const SplitJob* split = nullptr);
 
 }  // namespace nvs

@@ -70,6 +70,7 @@ class Sim:
         self.slots = {}  # ring slot register base -> (region, content)
         self.claim_lds = {}
         self.counter = 3
+        self.parts = []  # partial stores: (slot part's base, offset, bytes)
         self.qk, self.pv = [], []  # operand contents of QK / PV MFMAs
 
     # ---------------------------------------------------------- registers
@@ -409,9 +410,17 @@ class Sim:
             nrec = self.s[r0 + 2]
             assert args[-1].endswith("lds"), ln
             self.lds_fill(self.m0, (base, nrec) if nrec else ("zero",))
-        elif op == "buffer_store_dwordx4":
-            self.check_rsrc(args[2])
+        elif op in ("buffer_store_dwordx4", "buffer_store_dword"):
+            r0 = self.check_rsrc(args[2])
             self.vmq.append({"pos": self.pos, "done": None, "region": None})
+            if self.s[r0 + 2] == G.PART_WAVE:  # a wave's part of a partial slot
+                size = 16 if op.endswith("x4") else 4
+                off = self.sget(args[3].split()[0]) + self.off(args)
+                voff = self.vget(args[1])
+                if voff != [size * x for x in range(64)]:
+                    self.fail("partial store: lane offsets")
+                base = self.s[r0] | ((self.s[r0 + 1] & 0xFFFF) << 32)
+                self.parts.append((base, off, 64 * size))
         elif op == "global_atomic_add":
             self.vmq.append({"pos": self.pos, "done": None, "region": None})
             assert self.exec1
@@ -437,8 +446,12 @@ class Sim:
 
 
 # ------------------------------------------------------------------ model
-def plan_records(seqs, pbm, ntq, paged, bs, bt_stride, Tk, cu_k0, bt_rows):
-    recs = []
+def plan_records(seqs, pbm, ntq, paged, bs, bt_stride, Tk, cu_k0, rng, pe):
+    """The list's records (as the plan kernel's) and each one's row, query
+    tile, first key tile and tiles.  Some entries are cut into parts of
+    whole blocks, every row of the entry seeing a key of every part."""
+    recs, where = [], []
+    slot = 0
     q0 = 0
     for b, (L, K, blks) in enumerate(seqs):
         np_ = min((L + pbm - 1) // pbm, ntq)
@@ -456,38 +469,42 @@ def plan_records(seqs, pbm, ntq, paged, bs, bt_stride, Tk, cu_k0, bt_rows):
                 nblk = min((K + bs - 1) // bs, bt_stride)
                 x = blks[lb] if lb < nblk else -1
                 return x if 0 <= x < NB else -1  # the plan's check against the pool
-            if paged:
-                k0c, kf = 0, K
-                btb = 4 * min((K + bs - 1) // bs, bt_stride)
-                bb = (tb(0), tb(1), tb(2))
-            else:
-                k0c = min(max(k0, 0), Tk)
-                kf = max(0, min(K, Tk - k0c))
-                btb = 0
-                bb = (-1, -1, -1)
-            recs.append([b * ntq + qt, q0, L, k0, K, *bb, p0, nt, kf, off, k0c, b, btb, 0])
+            step = bs // 64 if paged else 1
+            starts = [0]
+            if rng.random() < 0.5:
+                each = step * rng.randint(1, 4)
+                starts += [t for t in range(each, nt, each) if 64 * t <= p0 + off]
+            for t0, t1 in zip(starts, starts[1:] + [nt]):
+                if paged:
+                    k0c, kf = 0, K - 64 * t0
+                    bto = 4 * (64 * t0 // bs)
+                    btb = 4 * min((K + bs - 1) // bs, bt_stride) - bto
+                    bb = tuple(tb(t0 + t) for t in range(3))
+                else:
+                    c = min(max(k0, 0), Tk)
+                    k0c, kf = c + 64 * t0, max(0, min(K, Tk - c)) - 64 * t0
+                    bto = btb = 0
+                    bb = (-1, -1, -1)
+                part = slot if len(starts) > 1 else -1
+                slot += pe if len(starts) > 1 else 0
+                recs.append([part, q0, L, k0, K, *bb, p0, t1 - t0, kf, off - 64 * t0, k0c, b, btb, bto])
+                where.append((b, qt, t0, t1 - t0))
         q0 += L
-    return recs
+    return recs, where
 
 
-def unit_tiles(u, recs, a, seqs, NB):
+def unit_tiles(u, recs, where, a, seqs, NB):
     """(K tiles, V tiles) of unit u as (address, bytes) with bytes > 0 only."""
     pe = a["Hkv"] * a["hgroups"]
     idx, rem = divmod(u, pe)
     hkv, hg = divmod(rem, a["hgroups"])
-    item, q0, L, k0, K = recs[idx][:5]
-    b, qt = divmod(item, a["ntq"])
-    p0 = qt * a["pbm"]
-    nt = 0
-    if p0 < L:
-        p_last = min(L, p0 + a["pbm"]) - 1
-        kv_end = min(K, p_last + (K - L) + 1)
-        nt = (kv_end + 63) // 64 if kv_end > 0 else 0
+    q0, L, k0, K = recs[idx][1:5]
+    b, qt, t0, nt = where[idx]
     out = ([], [])
     M48 = (1 << 48) - 1
     # a unit of one tile runs the QK^T of tile 1 too (its scores unused)
-    for t in range(nt + (1 if nt == 1 else 0)):
-        phantom = t >= nt
+    for t in range(t0, t0 + nt + (1 if nt == 1 else 0)):
+        phantom = t >= t0 + nt
         if a["paged"]:
             krow = a["Hkv"] * 256
             lb = 64 * t // a["bs"]
@@ -558,8 +575,8 @@ def check_case(rng, paged, slow_p):
              bt_stride=bt_stride, Tk=Tk, kc=base(), vc=base(), k=base(), v=base(), k_ts=Hkv * 128,
              v_ts=Hkv * 128, k_hs=128, v_hs=128, q=base(), q_ts=Hq * 128, q_hs=128, out=base(),
              out_ts=Hq * 128, out_hs=128, bt=base())
-    recs = plan_records(seqs, pbm, ntq, paged, bs, bt_stride, Tk, cu_k0, None)
     pe = Hkv * hgroups
+    recs, where = plan_records(seqs, pbm, ntq, paged, bs, bt_stride, Tk, cu_k0, rng, pe)
     units = len(recs) * pe
     lines = G.program(paged)
     w = rng.randrange(4)
@@ -610,6 +627,8 @@ def check_case(rng, paged, slow_p):
     vals[22] = a["out_hs"] * 2
     put64(23, a["bt"] if paged else 0)
     vals[25] = 4 * bt_stride if paged else 0
+    parts = base()
+    put64(26, parts + w * G.PART_WAVE)
     for k, x in vals.items():
         bank[k] = x & M32
     sim.v[G.BANKC] = bank
@@ -627,7 +646,7 @@ def check_case(rng, paged, slow_p):
     order = [u for u in order if u < units]
     expk, expv = [], []
     for u in order:
-        kt, vt = unit_tiles(u, recs, a, seqs, NB)
+        kt, vt = unit_tiles(u, recs, where, a, seqs, NB)
         expk += kt
         expv += vt
     gotk = [c[1] for c in groups(sim.qk, "QK") if c[1] != ("zero",)]
@@ -638,6 +657,15 @@ def check_case(rng, paged, slow_p):
     if gotv != expv:
         raise Fail(f"V tile sequence differs: got {len(gotv)} want {len(expv)}; first diff at "
                    f"{next((i for i, (x, y) in enumerate(zip(gotv, expv)) if x != y), min(len(gotv), len(expv)))}")
+    # each partial unit's slot written once, whole (O, then m and l)
+    want = []
+    for u in order:
+        idx, rem = divmod(u, pe)
+        if recs[idx][0] >= 0:
+            at = parts + w * G.PART_WAVE + (recs[idx][0] + rem) * G.PART_BYTES & ((1 << 48) - 1)
+            want += [(at, 32768 + 256 * k, 256) for k in range(4)] + [(at, 1024 * k, 1024) for k in range(32)]
+    if sim.parts != want:
+        raise Fail(f"partial stores differ: got {len(sim.parts)} want {len(want)}")
     return len(order)
 
 

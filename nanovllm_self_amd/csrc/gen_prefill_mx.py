@@ -41,6 +41,11 @@ u+1's first tiles are in opposite buffers.  A unit of one tile, a unit
 without a visible key and the work-group's last unit end the pipeline: the
 last PV and the output, then the next unit starts afresh.
 
+A unit may cover a part of its rows' keys (its record's tiles, blocks and
+causal offset count from the part's first key): it leaves its accumulators
+with m and l in its slot of the workspace instead of its output (chainp,
+transp, drainp), for the merge launch.
+
 Units are claimed three ahead: when unit u starts, wave 0 claims unit u+3
 (published in LDS before u's first barrier, read by every wave when u ends)
 and every wave loads the plan record of unit u+2 (a vector load into VREC,
@@ -170,6 +175,7 @@ BANKC_OUT = (19, 20)
 BANKC_ORTS, BANKC_OHS = 21, 22
 BANKC_BT = (23, 24)   # block tables (paged)
 BANKC_BTS = 25        # bytes between block-table rows
+BANKC_PART = (26, 27) # partials of the wave: slot 0, lo / hi
 
 # bank lanes: a unit's descriptor
 BANK_EX, BANK_NT, BANK_JM, BANK_KF = 0, 1, 2, 3
@@ -238,7 +244,15 @@ LDS_V0 = 32768      # V buffer 0 (K buffers at 0 and 16384; V buffers 1 and 2 fo
 TILE = 16384        # bytes of one 64-key bf16 tile
 NVBUF = 3           # V buffers: the tile of iteration g in buffer g % 3
 S_VB = "s100"       # offset from V buffer 0 of the buffer of the current iteration's tile
+BANK_PART = 36       # the unit's partial slot (negative: the unit is a whole one and writes its output)
+BANK_BTO = 37        # bytes from the row's first block-table entry to the unit's first
 BANK_NV0 = (34, 35)  # the unit's value tile 0: lo, hi (its bytes are key tile 0's)
+# A unit that covers a part of its rows' keys leaves a partial in its slot of
+# the workspace: per wave the O^T accumulators as they are (32 KiB, the 64
+# lanes' 16 bytes of four registers together), then m of both q-blocks and l
+# of both, one dword a lane.
+PART_WAVE = 33792
+PART_BYTES = 4 * PART_WAVE
 RSRC_W3 = "0x20000"  # raw buffer: 32-bit data format, no swizzle, no stride
 
 
@@ -753,6 +767,14 @@ def decode(em, u, paged, bank=None):
     em("s_nop 4")
     em(f"s_lshr_b32 {hkv}, {r}, {tt}")
     em(f"s_and_b32 {hg}, {r}, {tt}")
+    # its partial slot: the entry's first + r
+    pt = t[18]
+    readlanes(em, [(pt, VREC, 0), (t[19], VREC, 15)])
+    em(f"s_add_u32 {r}, {r}, {pt}")
+    em(f"s_cmp_lt_i32 {pt}, 0")
+    em(f"s_cselect_b32 {r}, -1, {r}")
+    em(f"v_writelane_b32 {BANKN}, {r}, {BANK_PART}")
+    em(f"v_writelane_b32 {BANKN}, {t[19]}, {BANK_BTO}")
     # record fields
     q0, L, blk0, blk1, blk2, p0, nt, kf, off, k0c, b, btb = t[6:18]
     readlanes(em, [(q0, VREC, 1), (L, VREC, 2), (blk0, VREC, 5), (blk1, VREC, 6), (blk2, VREC, 7),
@@ -823,11 +845,13 @@ def decode(em, u, paged, bank=None):
             em(f"v_writelane_b32 {BANKN}, {lo}, {BANK_NV0[0]}")
             em(f"v_writelane_b32 {BANKN}, {hi}, {BANK_NV0[1]}")
     # block-table row: bt + b x row bytes
-    readlanes(em, [(c0, BANKC, BANKC_BT[0]), (c1, BANKC, BANKC_BT[1]), (c2, BANKC, BANKC_BTS)])
+    readlanes(em, [(c0, BANKC, BANKC_BT[0]), (c1, BANKC, BANKC_BT[1]), (c2, BANKC, BANKC_BTS), (c3, BANKN, BANK_BTO)])
     em(f"s_mul_i32 {m0}, {b}, {c2}")
     em(f"s_mul_hi_u32 {m1}, {b}, {c2}")
     em(f"s_add_u32 {c0}, {c0}, {m0}")
     em(f"s_addc_u32 {c1}, {c1}, {m1}")
+    em(f"s_add_u32 {c0}, {c0}, {c3}")  # the unit's first block
+    em(f"s_addc_u32 {c1}, {c1}, 0")
     em(f"s_and_b32 {c1}, {c1}, 0xffff")
     em(f"v_writelane_b32 {BANKN}, {c0}, {BANK_RBT[0]}")
     em(f"v_writelane_b32 {BANKN}, {c1}, {BANK_RBT[1]}")
@@ -1079,6 +1103,56 @@ def output_items(bank, lsum, tmp, zero_o, qnext=False):
     return it
 
 
+def partial_resource(bank):
+    """S_RK <- the wave's part of the partial slot of the unit in `bank`."""
+    x0, x1 = S_RV_W[0], S_RV_W[1]
+    return [f"v_readlane_b32 {x0}, {bank}, {BANK_PART}", f"v_readlane_b32 {S_RK_W[0]}, {BANKC}, {BANKC_PART[0]}",
+            f"v_readlane_b32 {S_RK_W[1]}, {BANKC}, {BANKC_PART[1]}", "s_nop 4",
+            f"s_mul_hi_u32 {x1}, {x0}, {PART_BYTES}", f"s_mul_i32 {x0}, {x0}, {PART_BYTES}",
+            f"s_add_u32 {S_RK_W[0]}, {S_RK_W[0]}, {x0}", f"s_addc_u32 {S_RK_W[1]}, {S_RK_W[1]}, {x1}",
+            f"s_and_b32 {S_RK_W[1]}, {S_RK_W[1]}, 0xffff", f"s_mov_b32 {S_RK_W[2]}, {PART_WAVE}",
+            f"s_mov_b32 {S_RK_W[3]}, {RSRC_W3}"]
+
+
+def lane_bytes(reg, shift):
+    """reg <- lane << shift"""
+    return [f"v_mbcnt_lo_u32_b32 {reg}, -1, 0", f"v_mbcnt_hi_u32_b32 {reg}, -1, {reg}",
+            f"v_lshlrev_b32 {reg}, {shift}, {reg}"]
+
+
+def partial_ml(em, bank):
+    """m and l (summed over both key halves) of the unit in `bank` into its
+    partial slot."""
+    emit_items(em, partial_resource(bank) + lane_bytes(TMPV, 2) + [f"s_mov_b32 {S_TMP}, {4 * 8192}"])
+    for k, r in enumerate(MRUN + LRUN):
+        em(f"buffer_store_dword {r}, {TMPV}, {S_RK}, {S_TMP} offen offset:{256 * k}")
+
+
+def partial_items(bank, tmp, zero_o, qnext=False):
+    """O^T of the unit in `bank` into its partial slot, straight from the
+    accumulators (no scaling, no staging: the merge knows their layout), as
+    instruction strings; zero_o and qnext as in output_items.  32 stores a
+    wave."""
+    it = ["s_nop 7", "s_nop 7"] + partial_resource(bank) + lane_bytes(TMPV, 4)
+    zr = tmp[28]
+    if zero_o:
+        it += [f"v_mov_b32 v{zr + k}, 0" for k in range(4)]
+    for n in range(4):
+        for qb in range(2):
+            blk = 2 * n + qb
+            it.append(f"s_mov_b32 {S_TMP}, {4096 * blk}")
+            for k in range(4):
+                a = 64 + 16 * blk + 4 * k
+                it.append(f"buffer_store_dwordx4 a[{a}:{a + 3}], {TMPV}, {S_RK}, {S_TMP} offen offset:{1024 * k}")
+            if zero_o:
+                it += ["s_nop 1", f"{MF} {O(n, qb)}, v[{zr}:{zr + 3}], v[{zr}:{zr + 3}], 0"]
+    if qnext:
+        pre = Items()
+        q_prefetch(pre, BANKN, guard=True)
+        it += pre
+    return it
+
+
 def zero_output(em, bank):
     """A unit whose rows see no key: zeros for its rows (row 4 i + L / 16,
     chunk L % 16 from lane L, i = 0..7)."""
@@ -1135,12 +1209,13 @@ def unit_start(em, lbl, qnext=True):
     em(f"s_cselect_b32 {S_FLAGS}, 0, {S_FLAGS}")
 
 
-def block_iteration(em, paged, par, kind, lbl):
+def block_iteration(em, paged, par, kind, lbl, part=False):
     """Iteration j (parity par) of one of these kinds:
       fresh0  a unit's first tile after a fresh start (no PV),
       chain0  a unit's first tile in a chain: the PV of the previous unit's
               last tile (V and P of parity 1 - par) and its output beside
               this unit's QK^T of tile 1,
+              (part: its partial instead),
       main    a tile between,
       last    a unit's last tile ending the pipeline: no K fill, no QK^T,
       lastc   a unit's last tile chaining into the next: the next unit's
@@ -1189,7 +1264,9 @@ def block_iteration(em, paged, par, kind, lbl):
         b_items += dec
     if kind == "chain0":  # the previous unit's output first: its stores leave early
         pt = 128 + 32 * ppar  # the previous P, read by segment A's PV, is free in segment B
-        b_items = output_items(BANKP, LPREV, list(range(pt, pt + 32)), zero_o=True, qnext=True) + b_items
+        tmp = list(range(pt, pt + 32))
+        b_items = (partial_items(BANKP, tmp, zero_o=True, qnext=True) if part else
+                   output_items(BANKP, LPREV, tmp, zero_o=True, qnext=True)) + b_items
     if not pv:
         emit_items(em, fill)
         emit_items(em, a_items)
@@ -1258,9 +1335,9 @@ def block_iteration(em, paged, par, kind, lbl):
     em(f"s_mov_b32 {S_ROW[0]}, {S_ROW[1]}")
     em(f"s_mov_b32 {S_ROW[1]}, {S_ROW[2]}")
     vb_advance(em)
-    # chain0's output stores and the next unit's query-row copies (its last
-    # 32 vector memory operations) may drain
-    em(f"s_waitcnt vmcnt({32 if kind == 'chain0' else 0})")
+    # chain0's output stores (16, of a partial 32) and the next unit's
+    # query-row copies (16), its last vector memory operations, may drain
+    em(f"s_waitcnt vmcnt({(48 if part else 32) if kind == 'chain0' else 0})")
     mark(em, 3)
     if first:
         claim_publish(em, lbl)
@@ -1355,6 +1432,13 @@ def block_pv_only(em, par):
     em.lds_drain()
 
 
+def partial_branch(em, bank, lbl):
+    """To lbl if the unit in `bank` is a partial one."""
+    readlanes(em, [(S_TMP, bank, BANK_PART)])
+    em(f"s_cmp_lt_i32 {S_TMP}, 0")
+    em(f"s_cbranch_scc0 {lbl}")
+
+
 def claim_slot_read(em):
     """S_U2 <- the unit the current one claimed at its start (its first
     iteration published it; every wave has passed a barrier since)."""
@@ -1417,15 +1501,17 @@ def program(paged):
     em(f"s_mov_b32 {S_J}, 1")
     em(f"s_branch {u}top")
     # ---- a unit in a chain, its first iteration at parity p
-    for p in (0, 1):
-        em(f"{u}chain{p}:")
+    # (after a whole unit; after a partial one: chainp)
+    for p, part in ((0, True), (1, True), (0, False), (1, False)):
+        c = f"{u}{'cp' if part else 'c'}{p}"
+        em(f"{u}chain{'p' if part else ''}{p}:")
         unit_init(em, paged)
-        unit_start(em, f"{u}c{p}", qnext=False)
+        unit_start(em, c, qnext=False)
         em(f"s_cmp_gt_i32 {S_JM}, 0")
-        em(f"s_cbranch_scc1 {u}c{p}nomask")
+        em(f"s_cbranch_scc1 {c}nomask")
         block_mask(em, p)
-        em(f"{u}c{p}nomask:")
-        block_iteration(em, paged, p, "chain0", f"{u}c{p}i")
+        em(f"{c}nomask:")
+        block_iteration(em, paged, p, "chain0", f"{c}i", part)
         em(f"s_mov_b32 {S_J}, 1")
         em(f"s_branch {u}{'top' if p == 0 else 'mid'}")
     # ---- iterations 1, 2, ... (parity 1 at top, 0 at mid)
@@ -1458,6 +1544,7 @@ def program(paged):
     block_slow(em, 0, f"{u}i0")
     for p in (0, 1):
         block_slow(em, p, f"{u}c{p}i")
+        block_slow(em, p, f"{u}cp{p}i")
     for par in (1, 0):
         block_slow(em, par, f"{u}m{par}")
         block_slow(em, par, f"{u}l{par}")
@@ -1475,19 +1562,30 @@ def program(paged):
         em(f"{u}d{par}nonext:")
         block_pv_only(em, par)
         l_sum(em)
+        partial_branch(em, BANKU, f"{u}drainp")
         emit_items(em, output_items(BANKU, LRUN, list(range(32)), zero_o=False))
         em(f"s_branch {u}next")
+    em(f"{u}drainp:")
+    partial_ml(em, BANKU)
+    emit_items(em, partial_items(BANKU, list(range(32)), zero_o=False))
+    em(f"s_branch {u}next")
     # ---- a unit's last iteration chained into the next (its QK^T_0 done,
     # the units moved on beside it)
     for par in (0, 1):
-        em(f"{u}trans{par}:")
-        l_sum(em)
-        em(f"v_mov_b32 {LPREV[0]}, {LRUN[0]}")
-        em(f"v_mov_b32 {LPREV[1]}, {LRUN[1]}")
-        set_lim(em)
-        claim_slot_read(em)
-        em(f"s_add_u32 {S_IT}, {S_IT}, 1")
-        em(f"s_branch {u}chain{1 - par}")
+        for part in (False, True):
+            if not part:
+                em(f"{u}trans{par}:")
+                l_sum(em)
+                partial_branch(em, BANKP, f"{u}transp{par}")
+                em(f"v_mov_b32 {LPREV[0]}, {LRUN[0]}")
+                em(f"v_mov_b32 {LPREV[1]}, {LRUN[1]}")
+            else:
+                em(f"{u}transp{par}:")
+                partial_ml(em, BANKP)
+            set_lim(em)
+            claim_slot_read(em)
+            em(f"s_add_u32 {S_IT}, {S_IT}, 1")
+            em(f"s_branch {u}chain{'p' if part else ''}{1 - par}")
     # ---- a unit whose rows see no key (the pipeline is empty)
     em(f"{u}zero:")
     unit_start(em, f"{u}z")

@@ -43,6 +43,7 @@
 #include "store_common.h"
 #include "decode_merge.h"
 #include "decode_wave.h"
+#include "part_merge.h"
 
 namespace nvs {
 
@@ -79,9 +80,15 @@ void paged_decode_kernel(DecodeArgs a, const int32_t* __restrict__ bt, const int
 // (merge_split_rows).
 // Sixteen merge waves a work-group: a launch of a few large work-groups
 // is dispatched sooner than one of many single-wave ones.
-__global__ __launch_bounds__(64 * kMergeWaves) void decode_merge_kernel(DecodeArgs a, int units) {
+// The work-groups after the first `wgs` merge the parts of prefill entries
+// split along the keys.
+__global__ __launch_bounds__(64 * kMergeWaves) void decode_merge_kernel(DecodeArgs a, int units, int wgs,
+                                                                        PartMergeArgs parts) {
   __shared__ MergeLds lds;
-  merge_split_rows(a, units, (int)blockIdx.x, lds);
+  if ((int)blockIdx.x < wgs)
+    merge_split_rows(a, units, (int)blockIdx.x, lds);
+  else
+    merge_parts(parts, (int)blockIdx.x - wgs);
 }
 
 int64_t decode_workspace_bytes(int max_waves, int group) {
@@ -110,10 +117,29 @@ DecodeArgs decode_args(const AttnParams& P, int max_waves, void* partials) {
   return a;
 }
 
-int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream) {
-  if (groups <= 1) return NVS_OK;
-  const int units = (groups - 1) * a.Hkv;
-  hipLaunchKernelGGL(decode_merge_kernel, dim3(merge_wgs(units, a.Hkv)), dim3(64 * kMergeWaves), 0, stream, a, units);
+int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream, const AttnParams* P, const Plan* plan,
+                        const SplitJob* split) {
+  PartMergeArgs parts = {};
+  if (split && split->slots > 0) {
+    parts.hdr = plan->hdr;
+    parts.rows = split->at.rows;
+    parts.slots = split->at.slots;
+    parts.g = P->Hq / P->Hkv;
+    parts.hpi = 256 / prefill_mx_positions(parts.g);
+    parts.units = prefill_mx_units(P->Hq, P->Hkv);
+    parts.hgroups = parts.units / P->Hkv;
+    parts.out = (uint16_t*)P->out;
+    parts.out_ts = P->out_ts;
+    parts.out_hs = P->out_hs;
+    parts.f16 = P->cache_dtype == NVS_DTYPE_FP16 ? 1 : 0;
+    // Four items a unit, at least two slots an entry; two work-groups a CU.
+    parts.wgs = std::min(2 * split->slots, device_slots(2));
+  }
+  const int units = groups > 1 ? (groups - 1) * a.Hkv : 0;
+  const int wgs = units > 0 ? merge_wgs(units, a.Hkv) : 0;
+  if (wgs + parts.wgs == 0) return NVS_OK;
+  hipLaunchKernelGGL(decode_merge_kernel, dim3(wgs + parts.wgs), dim3(64 * kMergeWaves), 0, stream, a, units, wgs,
+                     parts);
   return check_launch("decode_merge");
 }
 

@@ -87,6 +87,7 @@ struct MxArgs {
   DecodeArgs dec;
   const int32_t* dec_bt;
   int dec_groups;  // decode groups the partial workspace has room for
+  char* parts;     // slots of the units that cover a part of their keys (null: none)
 };
 
 // Tile ring depth of the decode waves in this kernel (one wave per SIMD,
@@ -104,6 +105,14 @@ __host__ __device__ inline int mx_heads_per_item(int g) {
   return h;
 }
 int prefill_mx_positions(int g) { return 256 / mx_heads_per_item(g); }
+int prefill_mx_units(int Hq, int Hkv) {
+  const int g = Hq / Hkv, hpi = mx_heads_per_item(g);
+  return Hkv * ((g + hpi - 1) / hpi);
+}
+int prefill_mx_wgs(const AttnParams& P, const Plan& plan) {
+  const int64_t upper = (((int64_t)P.B * plan.ntq * prefill_mx_units(P.Hq, P.Hkv) + 7) / 8) * 8;
+  return (int)std::max<int64_t>(8, std::min<int64_t>(upper, (int64_t)device_slots(1)) & ~(int64_t)7);
+}
 
 __device__ __forceinline__ int mx_swz(int key) { return ((key & 3) << 2) | ((key >> 2) & 3); }
 
@@ -112,9 +121,12 @@ __device__ __forceinline__ int mx_lane() {
 }
 
 // Persistent, dynamically scheduled over the prefill list: unit u = (list
-// entry, kv head, head group); units with u % 8 == x are claimed from XCD
-// x's counter by the work-groups on XCD x.  The work-group claims its first
-// three units here; one asm statement (gen_prefill_mx.py) runs the rest: it
+// entry, kv head, head group); units with u % 8 == x belong to XCD x and are
+// claimed from its counter by the work-groups on it, except the first three
+// rounds: the work-groups that start on the prefill at once take those by
+// their number, back and forth (claimed one after the other, three to a
+// work-group, 104 units of up to 10 tiles left most of the chip idle: 26.4
+// us, now 22.0).  One asm statement (gen_prefill_mx.py) runs the rest: it
 // claims each further unit three ahead, decodes units from their plan
 // records, and streams their tiles through one pipeline that runs on from
 // one unit into the next.  What it needs from here: lane constants (LDS
@@ -134,8 +146,13 @@ __global__ __launch_bounds__(kMxThreads) __attribute__((amdgpu_waves_per_eu(1, 1
     MxArgs a, const PlanRecord* __restrict__ rec) {
   __shared__ __attribute__((aligned(1024))) char lds[kMxLdsBytes];
   __shared__ int s_claim[3];
+  // Work-groups of this XCD that start on the prefill at once, and this
+  // one's number among them (below 0: it streams decode rows first).
+  int starters = gridDim.x >> 3, number = blockIdx.x >> 3;
   if constexpr (DKV != kNoDecode) {
     const int nd = __builtin_amdgcn_readfirstlane(a.plan.hdr->dec_wgs);
+    starters -= nd >> 3;
+    number -= nd >> 3;
     if ((int)blockIdx.x < nd) {
       const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
       const int lw = 4 * (int)(blockIdx.x >> 3) + wave;  // among the XCD's nd / 2 decode waves
@@ -153,10 +170,12 @@ __global__ __launch_bounds__(kMxThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   const int xcd = blockIdx.x & 7;
   int* counter = a.plan.hdr->prefill_next + xcd;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (threadIdx.x == 0) {
-    s_claim[0] = atomicAdd(counter, 1);
-    s_claim[1] = atomicAdd(counter, 1);
-    s_claim[2] = atomicAdd(counter, 1);
+  if (number < 0) {  // streamed decode rows: joins late
+    if (threadIdx.x == 0)
+      for (int i = 0; i < 3; ++i) s_claim[i] = 3 * starters + atomicAdd(counter, 1);
+  } else if (threadIdx.x < 3) {
+    const int i = threadIdx.x;
+    s_claim[i] = i * starters + (i == 1 ? starters - 1 - number : number);
   }
   __syncthreads();
   const int u0 = __builtin_amdgcn_readfirstlane(8 * s_claim[0] + xcd);
@@ -235,12 +254,14 @@ __global__ __launch_bounds__(kMxThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   put(22, (int)(a.out_hs * 2));
   put64(23, PAGED ? (const void*)a.bt : nullptr);
   put(25, PAGED ? 4 * a.bt_stride : 0);
+  put64(26, a.parts + w * kPartWaveBytes);
 
   const int s_bs = PAGED ? a.bs : 64;
   const int s_nb = PAGED ? a.NB : 0;
   const int s_m0w = (int)lds_base + w * 4096;
   const int s_scale = __float_as_int(a.scale_log2);
   const uint64_t s_cnt = (uint64_t)counter;
+  const int claim0 = xcd + 24 * starters;  // unit of the counter's value 0
   const int s_qst = (int)lds_base + kMxQStage + w * kMxStageBytes;
   const int s_qd = kMxQStage + w * kMxStageBytes;
   const uint32_t mpe = per_entry == 1 ? 0u : (uint32_t)((0x100000000ull + per_entry - 1) / per_entry);
@@ -255,7 +276,7 @@ __global__ __launch_bounds__(kMxThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   : "{v[192:199]}"(kaddr), "{v[208:211]}"(dmak), "{v[212:215]}"(qlane),                                  \
     "{v246}"(ooff), "{v247}"(lanec), "{v248}"(bank), "{v255}"(rl),                                        \
     "{s4}"(krow), "{s5}"(s_bs), "{s6}"(s_nb), "{s7}"(s_m0w), "{s8}"(s_scale), "{s9}"(w),                  \
-    "{s[10:11]}"(s_cnt), "{s12}"(s_qst), "{s13}"(s_qd), "{s14}"(xcd), "{s15}"(units), "{s16}"(s_mpe),       \
+    "{s[10:11]}"(s_cnt), "{s12}"(s_qst), "{s13}"(s_qd), "{s14}"(claim0), "{s15}"(units), "{s16}"(s_mpe),       \
     "{s17}"(per_entry), "{s[18:19]}"(s_rec), "{s20}"(s_q16), "{s21}"(s_slot), "{s22}"(u0), "{s23}"(u1),    \
     "{s37}"(s_pe1), "{s60}"(u2), "{s61}"(4 * orts)                                                        \
   : NVS_PREFILL_MX_CLOBBERS
@@ -301,7 +322,8 @@ bool prefill_mx_serves(const AttnParams& P) {
   return P.NB * (int64_t)P.bs < (1ll << 31) && 4 * P.bt_stride < (1ll << 31);
 }
 
-int launch_prefill_mx(const AttnParams& P, const Plan& plan, hipStream_t stream, const CoDecode* co) {
+int launch_prefill_mx(const AttnParams& P, const Plan& plan, hipStream_t stream, const CoDecode* co,
+                      const SplitJob* split) {
   MxArgs a;
   a.q = (const uint16_t*)P.q; a.q_ts = P.q_ts; a.q_hs = P.q_hs;
   a.kc = (const char*)P.kc; a.vc = (const char*)P.vc;
@@ -330,11 +352,10 @@ int launch_prefill_mx(const AttnParams& P, const Plan& plan, hipStream_t stream,
     set_error("prefill: plan tile of %d positions does not match %d heads per item", plan.pbm, a.hpi);
     return NVS_ERR_INVALID;
   }
-  const int64_t upper = (((int64_t)P.B * plan.ntq * P.Hkv * a.hgroups + 7) / 8) * 8;
-  int64_t wgs = std::min<int64_t>(upper, (int64_t)device_slots(1));
-  wgs = std::max<int64_t>(8, wgs & ~(int64_t)7);
-  if (co) wgs = co->wgs;  // the plan sized the decode part for this many
-  const PlanRecord* rec = plan.rec;
+  // The plan sized the decode part, or the entries' parts, for as many.
+  const int64_t wgs = co ? co->wgs : split ? split->wgs : prefill_mx_wgs(P, plan);
+  a.parts = split ? split->at.slots : nullptr;
+  const PlanRecord* rec = split ? split->at.rec : plan.rec;
   const bool f16 = P.cache_dtype == NVS_DTYPE_FP16;
   const dim3 grid((unsigned)wgs), block(kMxThreads);
   const int dkv = co ? co->kv : kNoDecode;

@@ -3,6 +3,8 @@
 #include "nvs_common.h"
 #include "attention_common.h"
 #include "decode_merge.h"
+#include <climits>
+#include <type_traits>
 
 namespace nvs {
 
@@ -34,6 +36,11 @@ struct PlanArgs {
   float dec_hbm_bps;     // decode bytes per second of the whole chip
   float pre_cu_flops;    // prefill FLOP per second of one CU
   float dec_finish;      // the decode should end by this fraction of the call
+  // Entries split along the keys (split_slots > 0: the slots there are).
+  PlanRecord* rec;  // the list's records
+  SplitRow* split_rows;
+  int split_slots, split_wgs;
+  int units;  // units of an entry
 };
 
 // Tiles of the bf16 copy for a prefill row with kl keys.
@@ -51,16 +58,38 @@ __device__ __forceinline__ int tile_block(const PlanArgs& a, int b, int kl, int 
   return (blk >= 0 && blk < a.NB) ? blk : -1;
 }
 
-// Inclusive scan of one int per thread over the 1024-thread work-group:
-// shuffle scan inside each wave, then the 16 wave totals through LDS.  Also
-// returns the work-group total.  Two barriers.
+// x op the value of the lanes before it, step by step within the wave (data
+// parallel primitives: a step takes a few cycles where a shuffle through LDS
+// takes about a hundred).  Lanes a step does not reach take 0.
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T lanes_before(T x) {
+  return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROWS, 0xf, false));
+}
+template <typename T, typename F>
+__device__ __forceinline__ T wave_scan(T x, F op) {
+  x = op(x, lanes_before<0x111, 0xf>(x));  // row_shr 1, 2, 4, 8 within 16 lanes
+  x = op(x, lanes_before<0x112, 0xf>(x));
+  x = op(x, lanes_before<0x114, 0xf>(x));
+  x = op(x, lanes_before<0x118, 0xf>(x));
+  x = op(x, lanes_before<0x142, 0xa>(x));  // row_bcast 15: rows 1 and 3
+  return op(x, lanes_before<0x143, 0xc>(x));  // row_bcast 31: rows 2 and 3
+}
+__device__ __forceinline__ int wave_scan_add(int x) { return wave_scan(x, [](int p, int q) { return p + q; }); }
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan_add(x), 63); }
+__device__ __forceinline__ int wave_most(int x) {  // of values >= 0
+  return __builtin_amdgcn_readlane(wave_scan(x, [](int p, int q) { return max(p, q); }), 63);
+}
+__device__ __forceinline__ float wave_total(float x) {
+  x = wave_scan(x, [](float p, float q) { return p + q; });
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
+}
+
+// Inclusive scan of one int per thread over the 1024-thread work-group: a
+// scan inside each wave, then the 16 wave totals through LDS.  Also returns
+// the work-group total.  Two barriers.
 __device__ __forceinline__ int block_scan_1024(int v, int* lds, int& total) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(v, off, 64);
-    if (lane >= off) v += t;
-  }
+  v = wave_scan_add(v);
   if (lane == 63) lds[w] = v;
   __syncthreads();
   int before = 0, all = 0;
@@ -101,9 +130,7 @@ static_assert(kPlanWaves == kMergeWaves, "a work-group of the plan launch holds 
 __device__ __forceinline__ void block_sum3_1024(float (&v)[3], float (*lds)[3]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v[i] += __shfl_xor(v[i], off, 64);
+  for (int i = 0; i < 3; ++i) v[i] = wave_total(v[i]);
   if (lane == 0)
     for (int i = 0; i < 3; ++i) lds[w][i] = v[i];
   __syncthreads();
@@ -149,6 +176,81 @@ __device__ int pick_decode_wgs(const PlanArgs& a, float dec_rows, float dec_tile
   return top;
 }
 
+// A row of the batch, as its entries need it.
+struct RowFields {
+  int b, q0, L, k0, K;
+};
+
+// The record of the entry of query tile qt (kv tiles t0 .. t1 of the row's
+// visible ones), from its row.
+__device__ __forceinline__ PlanRecord make_record(const PlanArgs& a, const RowFields& r, bool shadow, const int (&blk)[3],
+                                                  int qt, int t0, int nt, int part) {
+  PlanRecord rec;
+  rec.part = part;
+  rec.q0 = r.q0;
+  rec.L = r.L;
+  rec.k0 = r.k0;
+  rec.K = r.K;
+  rec.blk0 = blk[0];
+  rec.blk1 = blk[1];
+  rec.blk2 = blk[2];
+  rec.off = r.K - r.L - 64 * t0;
+  rec.b = r.b;
+  if (a.paged) {
+    const int tbs = shadow ? kShadowTile : a.bs;
+    const int64_t tst = shadow ? a.shadow_st : a.bt_stride;
+    rec.k0c = 0;
+    rec.kf = r.K - 64 * t0;
+    rec.bt_off = 4 * (64 * t0 / tbs);
+    rec.bt_bytes = 4 * (int)min((int64_t)(r.K + tbs - 1) / tbs, tst) - rec.bt_off;
+  } else {
+    const int64_t k0c = min(max((int64_t)r.k0, (int64_t)0), a.Tk);
+    rec.k0c = (int)k0c + 64 * t0;
+    rec.kf = (int)max((int64_t)0, min((int64_t)r.K, a.Tk - k0c)) - 64 * t0;
+    rec.bt_off = rec.bt_bytes = 0;
+  }
+  rec.p0 = qt * a.plan.pbm;
+  rec.ntiles = nt;
+  return rec;
+}
+
+// Visible key tiles of query tile qt of a row, and those its first position
+// sees a key of.
+__device__ __forceinline__ int entry_tiles(const PlanArgs& a, int L, int K, int qt, int& first_sees) {
+  const int p0 = qt * a.plan.pbm, off = K - L;
+  const int kv_end = min(K, min(L, p0 + a.plan.pbm) + off);
+  first_sees = p0 + off >= 0 ? (p0 + off) / 64 + 1 : 0;
+  return (p0 < L && kv_end > 0) ? (kv_end + 63) / 64 : 0;
+}
+
+__device__ __forceinline__ int decode_wgs(const PlanArgs& a, float dec_rows, float dec_tiles, float pairs,
+                                          float (*lds)[3]) {
+  float sums[3] = {dec_rows, dec_tiles, pairs};
+  block_sum3_1024(sums, lds);
+  return pick_decode_wgs(a, sums[0], sums[1], sums[2]);
+}
+
+// An entry of nt key tiles in parts of at most about C: their tiles each
+// (whole blocks of `step` tiles) and their number.  Every row sees a key of
+// every part (first_sees: tiles the entry's first position sees a key of), so
+// no row of a part stays without a running max.
+__device__ __forceinline__ int part_tiles(int nt, int first_sees, int C, int step, int& parts) {
+  int n = (nt + C - 1) / C;
+  n = max(n, 1);
+  const int each = max(1, ((nt + n - 1) / n + step - 1) / step * step);
+  n = max(1, (nt + each - 1) / each);
+  while (n > 1 && (n - 1) * each >= first_sees) --n;
+  parts = n;
+  return each;
+}
+
+// Tiles a part may have at most, in rising order (8, 10, 12, 14, 16, 20, ..,
+// 80, 96: four steps an octave); the last choice: no parts.  One a wave.
+constexpr int kPartChoices = kPlanWaves;
+__device__ __forceinline__ int part_choice(int i) {
+  return i == kPartChoices - 1 ? INT_MAX / 2 : (4 + (i & 3)) << (1 + (i >> 2));
+}
+
 // What the plan keeps of each row of a 1024-row step in LDS while the
 // step's list entries are written, one entry per thread.
 struct PlanRows {
@@ -157,15 +259,200 @@ struct PlanRows {
   int blk[3][kPlanThreads];
 };
 
+// Entries weighed for a split: row, key tiles, tiles the first position sees
+// (then the first slot, -1: none), tiles of a part and parts; what the
+// buckets of part sizes hold, then their next place in the list; the list's
+// places (entry << 10 | part).
+constexpr int kPartBuckets = 64;
+struct PlanEntries {
+  int row[kSplitMaxEntries], nt[kSplitMaxEntries], sees[kSplitMaxEntries];
+  int each[kSplitMaxEntries], parts[kSplitMaxEntries];
+  int place[kSplitMaxEntries + kSplitSlots];
+  float cost[kPartChoices];
+  int bucket[kPartBuckets];
+  int longest, list, slots, rows;
+};
+
+// Estimated time of the call's prefill with parts of at most C tiles, in key
+// tiles of one work-group (1.2 us, 1.6 with the whole chip busy), by one wave
+// over all entries; infinite where the parts need more slots than there are.
+// Each unit has kPartSetup tiles' worth of set-up and output.  The units of
+// an XCD are dealt to its work-groups longest first, back and forth, three
+// rounds of them (prefill_mx_kernel's first claims): the most a work-group
+// gets is the estimate; past three rounds, the even share and some of the
+// longest.  A part's slot is written and read once (132 KiB each way):
+// kPartMerge.
+constexpr float kPartSetup = 7.0f;
+constexpr float kPartUneven = 0.3f;
+constexpr float kPartMerge = 0.0125f;
+constexpr float kPartLaunch = 1.0f;
+__device__ __forceinline__ float part_cost(const PlanArgs& a, const PlanEntries& ent, int* hist, int entries, int C,
+                                           int step, int wgs, int lane) {
+  int units = 0, slots = 0, longest = 0, tiles = 0;
+  for (int e = lane; e < entries; e += 64) {
+    int parts;
+    const int nt = ent.nt[e], each = part_tiles(nt, ent.sees[e], C, step, parts);
+    units += parts;
+    if (parts > 1) slots += parts;
+    tiles += nt;
+    longest = max(longest, parts > 1 ? max(each, nt - (parts - 1) * each) : nt);
+  }
+  const int pieces = wave_total(units);
+  units = pieces * a.units;
+  slots = wave_total(slots) * a.units;
+  tiles = wave_total(tiles);
+  longest = wave_most(longest);
+  if (slots > a.split_slots) return INFINITY;
+  const float merge = slots > 0 ? kPartLaunch + kPartMerge * slots : 0.0f;
+  const int most = wgs >> 3;  // work-groups of an XCD
+  if (units > 24 * most) {
+    const float one = (float)longest + kPartSetup;
+    return merge + fmaxf(one, ((float)tiles * a.units + kPartSetup * units) / (float)wgs + kPartUneven * one);
+  }
+  // Pieces by size, longest first: 64 buckets, then how many there are up to
+  // each (the wave's own LDS: its operations complete in order).
+  const float scale = 64.0f / (float)(longest + 1);
+  hist[lane] = 0;
+  __builtin_amdgcn_wave_barrier();
+  for (int e = lane; e < entries; e += 64) {
+    int parts;
+    const int nt = ent.nt[e], each = part_tiles(nt, ent.sees[e], C, step, parts);
+    const int last = parts > 1 ? nt - (parts - 1) * each : nt;
+    atomicAdd(&hist[min(63, (int)((float)(longest - last) * scale))], 1);
+    if (parts > 1) atomicAdd(&hist[min(63, (int)((float)(longest - each) * scale))], parts - 1);
+  }
+  __builtin_amdgcn_wave_barrier();
+  const int upto = wave_scan_add(hist[lane]);
+  hist[lane] = upto;
+  __builtin_amdgcn_wave_barrier();
+  float load = 0.0f;
+  for (int i = 0; i < 3; ++i) {
+    const int unit = 8 * (i * most + (i == 1 ? most - 1 - lane : lane));
+    if (lane < most && unit < units) {
+      const int piece = unit / a.units;
+      int b = 0;  // the first bucket that reaches past the piece
+#pragma unroll
+      for (int s = 32; s >= 1; s >>= 1)
+        if (hist[b + s - 1] <= piece) b += s;
+      load += (float)longest - (float)b / scale + kPartSetup;
+    }
+  }
+  return merge + 0.125f * (float)wave_most((int)(8.0f * load));
+}
+
+// Measured (the prefill kernel alone): six turns of 44 .. 294 tokens over
+// 2 .. 16 K cached ones (32 / 8 heads, 144 units of 33 .. 249 tiles) unsplit
+// 302 us, bound by the longest unit; in parts of up to 20, 28, 40, 56 and 92
+// tiles 135, 151, 136, 150 and 139 us, and 14, 12, 9, 6 and 4 us of merge.
+// Four prompts of 0.7 .. 1.2 K over up to 3.8 K cached (488 units of up to 75
+// tiles, fp8): row by row 194 us, longest first 178, in parts of 64 171.  A
+// batch of more than kSplitMaxUnits units keeps the row order: its tail is
+// short, and neighbouring units of a row share its keys in L2.
+// The list of a batch of one step of rows (in `rows`, tot entries), longest
+// units first, its entries split along the keys where that ends sooner.
+// Returns the list's length; every thread calls it.
+__device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& ent, bool shadow, int tot, int wgs) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int step = (a.paged && !shadow) ? a.bs / 64 : 1;
+  int r = 0, qt = 0, nt = 0, sees = 0;
+  if (tid < tot) {
+    int hi = kPlanThreads - 1;
+    while (r < hi) {
+      const int mid = (r + hi) >> 1;
+      if (rows.end[mid] > tid) hi = mid; else r = mid + 1;
+    }
+    qt = rows.end[r] - 1 - tid;
+    nt = entry_tiles(a, rows.L[r], rows.K[r], qt, sees);
+    ent.row[tid] = r;
+    ent.nt[tid] = nt;
+    ent.sees[tid] = sees;
+  }
+  if (tid < kPartBuckets) ent.bucket[tid] = 0;
+  if (tid == kPartBuckets) ent.longest = ent.slots = ent.rows = 0;
+  __syncthreads();
+  {
+    const float c = part_cost(a, ent, ent.place + 64 * w, tot, part_choice(w), step, wgs, lane);
+    if (lane == 0) ent.cost[w] = c;
+  }
+  __syncthreads();
+  int best = kPartChoices - 1;
+  for (int i = kPartChoices - 2; i >= 0; --i)
+    if (ent.cost[i] < ent.cost[best]) best = i;
+  int parts = 0, each = 0;
+  if (tid < tot) {
+    each = part_tiles(nt, sees, part_choice(best), step, parts);
+    if (parts == 1) each = nt;
+    ent.each[tid] = each;
+    ent.parts[tid] = parts;
+    atomicMax(&ent.longest, each);
+    int slot = -1;
+    if (parts > 1) {
+      slot = atomicAdd(&ent.slots, parts) * a.units;
+      a.split_rows[atomicAdd(&ent.rows, 1)] = {slot, parts, rows.q0[r], rows.L[r], qt * a.plan.pbm};
+    }
+    ent.sees[tid] = slot;
+  }
+  __syncthreads();
+  // Places by part size, longest first, to a 64th of the longest.  Which of
+  // two entries of one bucket comes first, and the slots they take, change
+  // with the run; their outputs do not.
+  int bk = 0;
+  if (tid < tot) {
+    bk = (int)((int64_t)(ent.longest - each) * kPartBuckets / (ent.longest + 1));
+    atomicAdd(&ent.bucket[bk], parts);
+  }
+  __syncthreads();
+  if (tid < kPartBuckets) {
+    const int n = ent.bucket[tid], end = wave_scan_add(n);
+    ent.bucket[tid] = end - n;
+    if (tid == kPartBuckets - 1) {
+      ent.list = end;
+      a.plan.hdr->n_split = ent.rows;
+    }
+  }
+  __syncthreads();
+  if (tid < tot) {
+    const int at = atomicAdd(&ent.bucket[bk], parts);
+    for (int c = 0; c < parts; ++c) ent.place[at + c] = tid << 10 | c;
+  }
+  __syncthreads();
+  const int list = ent.list;
+  for (int i = tid; i < list; i += kPlanThreads) {
+    const int e = ent.place[i] >> 10, c = ent.place[i] & 1023;
+    const int b = ent.row[e];
+    const RowFields row = {b, rows.q0[b], rows.L[b], rows.k0[b], rows.K[b]};
+    const int n = ent.parts[e], tiles = ent.each[e], t0 = c * tiles;
+    int blk[3];
+    for (int t = 0; t < 3; ++t) {
+      if (c == 0)
+        blk[t] = rows.blk[t][b];
+      else if (shadow)
+        blk[t] = t0 + t < shadow_row_tiles(a, 1, row.K) ? a.shadow_base[b] + t0 + t : -1;
+      else
+        blk[t] = a.paged ? tile_block(a, b, row.K, t0 + t) : -1;
+    }
+    a.rec[i] = make_record(a, row, shadow, blk, rows.end[b] - 1 - e, t0, c == n - 1 ? ent.nt[e] - t0 : tiles,
+                           n > 1 ? ent.sees[e] + c * a.units : -1);
+  }
+  return list;
+}
+
 // Work-group 0 writes the plan; the others (a paged call whose decode
 // launch left its merge to this one) merge the decode rows split across
 // groups, one merge wave per wave.
+template <bool PARTS, bool MERGE>
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeArgs m, int merge_units) {
+  struct NoEntries {};
   __shared__ union Lds {
-    struct { int scan[kPlanWaves]; float sum[kPlanWaves][3]; PlanRows rows; } plan;
-    MergeLds merge;
+    struct {
+      PlanRows rows;
+      int scan[kPlanWaves];
+      float sum[kPlanWaves][3];
+      std::conditional_t<PARTS, PlanEntries, NoEntries> entries;
+    } plan;
+    std::conditional_t<MERGE, MergeLds, NoEntries> merge;
   } lds;
-  if (blockIdx.x > 0) {
+  if constexpr (MERGE) if (blockIdx.x > 0) {
     merge_split_rows(m, merge_units, (int)blockIdx.x - 1, lds.merge);
     return;
   }
@@ -175,6 +462,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
   const int tid = threadIdx.x;
   const Plan& pl = a.plan;
   if (tid < 8) pl.hdr->prefill_next[tid] = 0;
+  if (!PARTS && tid == 0) pl.hdr->n_split = 0;
   // ---- code caches: the prefill rows' 64-key tiles of the bf16 copy, row
   // by row (an exclusive scan of ceil(k_len / 64)); the copy serves the call
   // if they fit.
@@ -209,6 +497,8 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
   int base = 0;
   // this thread's rows: decode rows and their tiles, prefill query-key pairs
   float dec_rows = 0.0f, dec_tiles = 0.0f, pairs = 0.0f;
+  int dec_wgs = -1;  // picked
+  bool parted = false;
   for (int b0 = 0; b0 < a.B; b0 += kPlanThreads) {
     bool dec;
     int np, q0, kl, tot;
@@ -232,6 +522,19 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
       }
     }
     __syncthreads();
+    if constexpr (PARTS) {
+      if (a.B <= kPlanThreads && tot > 0 && tot <= kSplitMaxEntries && tot * a.units <= kSplitMaxUnits &&
+          (!a.shadow_base || shadow)) {
+        int wgs = a.split_wgs;
+        if (a.co_wgs > 0) {  // the work-groups that stream decode rows join late
+          dec_wgs = decode_wgs(a, dec_rows, dec_tiles, pairs, sum_lds);
+          wgs = max(8, a.co_wgs - dec_wgs);
+        }
+        base = plan_parts(a, rows, lds.plan.entries, shadow, tot, wgs);
+        parted = true;
+        break;
+      }
+    }
     for (int e = tid; e < tot; e += kPlanThreads) {
       int lo = 0, hi = kPlanThreads - 1;  // the first row whose prefix passes e
       while (lo < hi) {
@@ -240,48 +543,21 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
       }
       const int r = lo, rb = b0 + r;
       const int qt = rows.end[r] - 1 - e;  // the row's first entry is its deepest tile
-      PlanRecord rec;
-      rec.q0 = rows.q0[r];
-      rec.L = rows.L[r];
-      rec.k0 = rows.k0[r];
-      rec.K = rows.K[r];
-      rec.blk0 = rows.blk[0][r];
-      rec.blk1 = rows.blk[1][r];
-      rec.blk2 = rows.blk[2][r];
-      // What the MFMA kernel derives per entry.  The table it reads is the
-      // copy's (64-key tiles, shadow_st a row) when the copy serves the call.
-      rec.off = rec.K - rec.L;
-      rec.b = rb;
-      if (a.paged) {
-        rec.k0c = 0;
-        rec.kf = rec.K;
-        const int tbs = shadow ? kShadowTile : a.bs;
-        const int64_t tst = shadow ? a.shadow_st : a.bt_stride;
-        rec.bt_bytes = 4 * (int)min((int64_t)(rec.K + tbs - 1) / tbs, tst);
-      } else {
-        const int64_t k0c = min(max((int64_t)rec.k0, (int64_t)0), a.Tk);
-        rec.k0c = (int)k0c;
-        rec.kf = (int)max((int64_t)0, min((int64_t)rec.K, a.Tk - k0c));
-        rec.bt_bytes = 0;
-      }
-      rec.pad = 0;
-      rec.item = rb * pl.ntq + qt;
-      rec.p0 = qt * pl.pbm;
-      const int p_last = min(rec.L, rec.p0 + pl.pbm) - 1;
-      const int kv_end = min(rec.K, p_last + rec.off + 1);
-      rec.ntiles = (rec.p0 < rec.L && kv_end > 0) ? (kv_end + 63) / 64 : 0;
-      pl.plist[base + e] = rec.item;
-      pl.rec[base + e] = rec;
+      const RowFields row = {rb, rows.q0[r], rows.L[r], rows.k0[r], rows.K[r]};
+      const int blk[3] = {rows.blk[0][r], rows.blk[1][r], rows.blk[2][r]};
+      int sees;
+      pl.plist[base + e] = rb * pl.ntq + qt;
+      a.rec[base + e] = make_record(a, row, shadow, blk, qt, 0, entry_tiles(a, row.L, row.K, qt, sees), -1);
     }
     __syncthreads();  // the next step's rows overwrite the LDS
     base += tot;
   }
   if (tid == 0) pl.hdr->n_prefill = base;
+  if (PARTS && !parted && tid == 0) pl.hdr->n_split = 0;
   if (a.co_wgs > 0) {
     if (tid < 2) a.dec_rec[tid] = 0;
-    float sums[3] = {dec_rows, dec_tiles, pairs};
-    block_sum3_1024(sums, sum_lds);
-    if (tid == 0) pl.hdr->dec_wgs = pick_decode_wgs(a, sums[0], sums[1], sums[2]);
+    if (dec_wgs < 0) dec_wgs = decode_wgs(a, dec_rows, dec_tiles, pairs, sum_lds);
+    if (tid == 0) pl.hdr->dec_wgs = dec_wgs;
   } else if (tid == 0) {
     pl.hdr->dec_wgs = 0;
   }
@@ -302,7 +578,7 @@ int device_slots(int per_cu) {
 }
 
 int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t stream, const ShadowLayout* shadow,
-                const MergeJob* merge, const CoDecode* co) {
+                const MergeJob* merge, const CoDecode* co, const SplitJob* split) {
   PlanArgs a;
   a.cu_q = P.cu_q;
   a.cu_k = P.cu_k;
@@ -318,6 +594,11 @@ int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t s
   a.shadow_cap = shadow ? shadow->cap : 0;
   a.shadow_st = shadow ? shadow->ST : 0;
   a.Tk = P.Tk;
+  a.rec = split ? split->at.rec : plan.rec;
+  a.split_rows = split ? split->at.rows : nullptr;
+  a.split_slots = split ? split->slots : 0;
+  a.split_wgs = split ? split->wgs : 0;
+  a.units = prefill_mx_units(P.Hq, P.Hkv);
   a.co_wgs = co ? co->wgs : 0;
   a.dec_rec = co ? co->a.ws_rec : nullptr;
   a.Hq = P.Hq;
@@ -336,7 +617,12 @@ int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t s
     units = merge->units;
   }
   const int grid = 1 + (units > 0 ? merge_wgs(units, m.Hkv) : 0);
-  hipLaunchKernelGGL(plan_kernel, dim3(grid), dim3(kPlanThreads), 0, stream, a, m, units);
+  if (a.split_slots > 0)
+    hipLaunchKernelGGL((plan_kernel<true, false>), dim3(1), dim3(kPlanThreads), 0, stream, a, m, units);
+  else if (units > 0)
+    hipLaunchKernelGGL((plan_kernel<false, true>), dim3(grid), dim3(kPlanThreads), 0, stream, a, m, units);
+  else
+    hipLaunchKernelGGL((plan_kernel<false, false>), dim3(grid), dim3(kPlanThreads), 0, stream, a, m, units);
   return check_launch("plan");
 }
 

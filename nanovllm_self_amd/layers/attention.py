@@ -30,6 +30,7 @@ _SERVED_CACHE_DTYPES = (torch.bfloat16, torch.float16, torch.int8, torch.float8_
 _QUANT_DTYPE = {"int8_mock": torch.int8, "fp8_e4m3": torch.float8_e4m3fn}
 
 _workspaces: dict = {}
+_kept_workspaces: set = set()  # devices whose workspace was reserved or is in a captured graph
 
 
 def _need_device(t: torch.Tensor, what: str) -> None:
@@ -37,22 +38,30 @@ def _need_device(t: torch.Tensor, what: str) -> None:
         raise RuntimeError(f"{what} must be a GPU tensor for the HIP kernels (got {t.device})")
 
 
-def attention_workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
+def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) -> torch.Tensor | None:
     """Per-device split-K workspace, grown on demand (never inside graph capture).
 
-    Calls that share it must be ordered on one stream."""
+    `optional` bytes more are used where they are there: a buffer that lacks
+    only them is not replaced once it was reserved or handed to a captured
+    graph.  Calls that share it must be ordered on one stream."""
     if nbytes <= 0:
         return None
     key = torch.device(device)
     buf = _workspaces.get(key)
-    if buf is None or buf.numel() < nbytes:
+    have = buf.numel() if buf is not None else 0
+    if optional > 0 and have < nbytes + optional or have < nbytes:
         if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError(
-                "decode workspace too small inside graph capture; call "
-                "reserve_attention_workspace(...) before capturing"
-            )
-        buf = torch.empty(nbytes, dtype=torch.uint8, device=key)
-        _workspaces[key] = buf
+            _kept_workspaces.add(key)
+            if have < nbytes:
+                raise RuntimeError(
+                    "decode workspace too small inside graph capture; call "
+                    "reserve_attention_workspace(...) before capturing"
+                )
+        elif have < nbytes or key not in _kept_workspaces:
+            buf = torch.empty(nbytes + optional, dtype=torch.uint8, device=key)
+            _workspaces[key] = buf
+    elif key not in _kept_workspaces and torch.cuda.is_current_stream_capturing():
+        _kept_workspaces.add(key)
     return buf
 
 
@@ -62,9 +71,12 @@ def reserve_attention_workspace(num_seqs: int, max_seqlen_q: int, max_seqlen_k: 
     before capturing a graph, where it cannot grow).  num_kv_heads = 0 sizes
     for every kv-head count (an upper bound); passing the layer's count
     reserves exactly what its calls need."""
-    n = _lib.load().nvs_attention_workspace_bytes(num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads,
-                                                  128, 0)
-    attention_workspace(torch.device(device), int(n))
+    lib = _lib.load()
+    n = lib.nvs_attention_workspace_bytes(num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, 128, 0)
+    extra = lib.nvs_attention_split_bytes(num_seqs, 0, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads)
+    if n > 0:
+        attention_workspace(torch.device(device), int(n), int(extra))
+        _kept_workspaces.add(torch.device(device))
 
 
 def _quantize(x: torch.Tensor, code_dtype: torch.dtype):
@@ -303,6 +315,10 @@ class PagedAttention(nn.Module):
         lib = _lib.load()
         stream = _lib.stream_of(q)
         max_q, max_k = int(context.max_seqlen_q), int(context.max_seqlen_k)
+        # Room for the parts of prefill rows split along their keys, where
+        # that can help (used if there).
+        extra = int(lib.nvs_attention_split_bytes(
+            B, T, max_q, max_k, self.num_heads, self.num_kv_heads)) if max_q > 1 else 0
         if (context.block_tables is not None and self.k_cache is not None
                 and self.k_cache.dtype in (torch.int8, torch.float8_e4m3fn)):
             # int8 / fp8 caches: room for the bf16 copy of the prefill rows'
@@ -310,10 +326,15 @@ class PagedAttention(nn.Module):
             ws_bytes = int(lib.nvs_attention_workspace_bytes_cache(
                 B, max_q, max_k, self.num_heads, self.num_kv_heads, self.head_dim, 0,
                 _lib.nvs_dtype(self.k_cache.dtype)))
+            if extra > 0 and ws_bytes <= lib.nvs_attention_workspace_bytes(
+                    B, max_q, max_k, self.num_heads, self.num_kv_heads, self.head_dim, 0):
+                extra = 0  # no room for the copy: the kernel without it splits nothing
         else:
             ws_bytes = int(lib.nvs_attention_workspace_bytes(
                 B, max_q, max_k, self.num_heads, self.num_kv_heads, self.head_dim, 0))
-        ws = attention_workspace(q.device, ws_bytes)
+        ws = attention_workspace(q.device, ws_bytes, extra)
+        if ws is not None and extra > 0:
+            ws_bytes = min(ws.numel(), ws_bytes + extra)
         if context.block_tables is None:
             k = k.to(compute) if k.dtype != compute else k
             v = v.to(compute) if v.dtype != compute else v

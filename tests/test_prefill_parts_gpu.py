@@ -1,0 +1,112 @@
+"""Prefill entries split along their keys: short new turns over long cached
+prefixes (and long prompts of one kv head), where a batch has too few units
+for the chip.  The plan cuts their keys into parts, each part's units leave
+fp32 partials in the workspace, and the merge joins them.  Checked against
+the fp32 CPU oracle with the tolerances of tests/gpu_util.py; a batch that
+should be split is also checked to have been (the plan header's count), and
+the same batch in a workspace without room for the parts must agree."""
+import numpy as np
+import pytest
+import torch
+
+from nanovllm_self_amd import workloads as W
+from nanovllm_self_amd.kv_cache import SeqSlice
+from nanovllm_self_amd.layers import attention as LA
+from oracle import attn_oracle as AO
+from tests.gpu_util import bf16_to_np, compare, oracle_seq_rows, say
+
+pytestmark = pytest.mark.gpu
+N_SPLIT = 12  # the plan header's word
+
+
+def _workload(device, spec, Hkv, g, bs, kv, seed):
+    lens = [p + n for p, n in spec]
+    NB = sum((x + bs - 1) // bs for x in lens) + 2
+    gen = torch.Generator().manual_seed(seed)
+    tabs = W._tables(gen, lens, bs, NB)
+    seqs = [SeqSlice(tabs[i], p, n) for i, (p, n) in enumerate(spec)]
+    return W._assemble("parts", seqs, g * Hkv, Hkv, 128, bs, NB, kv, device, gen, seed=seed)
+
+
+def _check(wl, got, spec, quant, what):
+    """Rows of every sequence against the oracle: the first, the last and
+    those around query-tile edges."""
+    for i, (p, n) in enumerate(spec):
+        for r0, r1 in ((0, min(n, 3)), (max(0, min(n, 65) - 3), min(n, 65)), (max(0, n - 2), n)):
+            ref, rows = oracle_seq_rows(wl, i, r0, r1)
+            compare(got[rows], ref, quant, f"{what} row {i} [{r0}, {r1})")
+
+
+@pytest.mark.parametrize("Hkv,g,bs,kv,spec", [
+    (8, 4, 256, "bf16", [(8192, 70), (2048, 3), (4352, 130)]),
+    (8, 4, 256, "bf16", [(6400, 65), (300, 1), (9000, 1), (1000, 33)]),       # decode rows beside them
+    (2, 8, 64, "fp8", [(4160, 40), (1111, 64), (64, 2)]),
+    (2, 8, 64, "int8", [(3000, 1), (5056, 100)]),
+    (1, 16, 128, "bf16", [(7040, 257)]),                                     # two head groups
+    (2, 5, 64, "bf16", [(2752, 31), (1024, 2)]),                             # a head group not full
+    (1, 1, 1024, "bf16", [(8192, 300)]),                                     # blocks of sixteen tiles
+    (4, 3, 64, "fp16", [(3072, 129), (3000, 5)]),
+])
+def test_parts_match_oracle(device, monkeypatch, Hkv, g, bs, kv, spec):
+    say(f"parts: Hkv={Hkv} g={g} block_size={bs} cache={kv} rows (cached, new)={spec}")
+    wl = _workload(device, spec, Hkv, g, bs, kv, 11)
+    out = wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    header = LA._workspaces[wl.q.device][:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) > 0, "the batch was not split"
+    got = bf16_to_np(out)
+    _check(wl, got, spec, kv in ("int8", "fp8"), "parts")
+    again = wl.attn.prefill_flashattn(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again), "two identical calls differ"
+    # No room for the parts: the whole entries, in another order of sums.
+    monkeypatch.setattr(LA._lib.load(), "nvs_attention_split_bytes", lambda *a: 0)
+    whole = wl.attn.prefill_flashattn(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    compare(got, bf16_to_np(whole), kv in ("int8", "fp8"), "parts vs whole")
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp16"])
+def test_local_prompt_parts_match_oracle(device, kv):
+    """A long prompt of one kv head, nothing cached: its deep query tiles
+    are cut into parts, its shallow ones (and the diagonal) are not."""
+    spec = [(0, 3001), (0, 70)]
+    say(f"local parts {kv} {spec}")
+    wl = _workload(device, spec, 1, 8, 64, kv, 5)
+    assert wl.context.block_tables is None
+    out = wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    header = LA._workspaces[wl.q.device][:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) > 0, "the batch was not split"
+    ref = AO.attention_local(*(torch.from_numpy(bf16_to_np(x)) for x in (wl.q, wl.k, wl.v)),
+                             wl.context.cu_seqlens_q.cpu(), 8, 1, 128)
+    compare(bf16_to_np(out), ref.numpy(), False, f"local parts {kv}")
+
+
+def test_parts_in_a_graph(device):
+    """A captured call whose workspace has room for the parts, replayed over
+    changed queries, equals the eager one; the captured workspace stays."""
+    spec = [(4096, 40), (2048, 7), (500, 1)]
+    say(f"parts in a graph {spec}")
+    wl = _workload(device, spec, 8, 4, 256, "bf16", 3)
+    args = (wl.q, wl.k, wl.v, wl.context)
+    wl.attn.forward(*args)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = wl.attn.forward(*args)
+    ws = LA._workspaces[wl.q.device]
+    for step in range(3):
+        wl.q.copy_(torch.randn_like(wl.q))
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = out.clone()
+        eager = wl.attn.forward(*args)
+        torch.cuda.synchronize()
+        assert torch.equal(replayed, eager), f"replay {step} differs"
+    big = _workload(device, [(16384, 20), (16384, 30)], 8, 4, 256, "bf16", 4)
+    big.attn.forward(big.q, big.k, big.v, big.context)
+    torch.cuda.synchronize()
+    need = LA._lib.load().nvs_attention_workspace_bytes(2, 30, 16384 + 30, 32, 8, 128, 0)
+    assert ws.numel() < need or LA._workspaces[wl.q.device] is ws
+    assert np.all(np.isfinite(bf16_to_np(eager)))
