@@ -157,11 +157,12 @@ __device__ __forceinline__ void merge_heads(const DecodeArgs& a, const MergeRow&
 }
 
 // A merge work-group is sixteen waves, one unit each.  A row of up to
-// kMergeAlone partials (a run or two) is merged by its wave; the longer
+// kMergeAlone partials is merged by its wave; the longer
 // ones by teams of waves, the work-group's waves shared evenly among up to
 // kMergeTeams of them at a time.
 constexpr int kMergeWaves = 16;
-constexpr int kMergeAlone = 8;
+template <int NH>
+constexpr int kMergeAlone = 16 / NH;
 constexpr int kMergeTeams = 4;
 
 struct MergeLds {
@@ -210,15 +211,17 @@ __device__ __forceinline__ MergeRow merge_row(const DecodeArgs& a, int unit, int
   if (unit >= units) return r;
   r.k = unit / a.Hkv;
   r.h = unit - r.k * a.Hkv;
-  // Groups k >= Kw - 1 merge nothing (a launch may hold more merge waves
-  // than the decode had groups; their records are not this call's).
-  const int T = __builtin_amdgcn_readfirstlane(a.ws_rec[0]), Kw = __builtin_amdgcn_readfirstlane(a.ws_rec[1]);
-  if (r.k >= Kw - 1) return r;
+  // Header and record in one round trip.  Groups k >= Kw - 1 merge nothing (a
+  // launch may hold more merge waves than the decode had groups; their
+  // records are not this call's).
+  const int T = a.ws_rec[0], Kw = a.ws_rec[1];
   const int32_t* rec = a.ws_rec + 4 + 4 * unit;
-  if (__builtin_amdgcn_readfirstlane(rec[3]) == 0) return r;
-  r.q_row = __builtin_amdgcn_readfirstlane(rec[0]);
-  r.slot_k = __builtin_amdgcn_readfirstlane(rec[2]);
-  const int last = group_start(T, Kw, r.k + 1) - 1 + __builtin_amdgcn_readfirstlane(rec[1]);  // the row's last tile
+  const int rec_row = rec[0], rec_tiles = rec[1], rec_slot = rec[2], rec_on = rec[3];
+  asm volatile("" ::"s"(T), "s"(Kw), "s"(rec_row), "s"(rec_tiles), "s"(rec_slot), "s"(rec_on));
+  if (r.k >= Kw - 1 || rec_on == 0) return r;
+  r.q_row = rec_row;
+  r.slot_k = rec_slot;
+  const int last = group_start(T, Kw, r.k + 1) - 1 + rec_tiles;  // the row's last tile
   r.k_last = (int)(((int64_t)(last + 1) * Kw - 1) / T);
   return r;
 }
@@ -230,24 +233,23 @@ __device__ __forceinline__ MergeRow merge_row(const DecodeArgs& a, int unit, int
 // partials.  Lane l
 // serves head 4 p + l / 16 of the group (pass p) and head_dim elements
 // 8 (l % 16) .. + 7; a pass over the partials keeps a running max, sum and
-// output, for up to two head passes together.
-// What bounds it is the chain of dependent loads, about 2 us a run of four
-// partials.  With one wave a row throughout, a single conversation of 20 011
-// keys, whose row is split across all 156 groups, took 62.6 us here (now
-// 8.7), 48 rows of 256 .. 32 768 keys with 8 heads a group 14.2 us (12.9).
-// A team costs two barriers: rows of up to eight partials stay with one wave
-// (64 rows of 2 .. 8 K keys: 7.1 us; 12.5 with teams from five partials on;
-// the 48 rows: 16.0 us with teams only from thirteen on).
+// output, for NH head passes together (two for groups of more than four).
+// What bounds it is the chain of dependent loads, about 0.7 us a run of four
+// partials (1.3 us with two head passes).  With one wave a row throughout, a
+// single conversation of 20 011 keys, whose row is split across all 156
+// groups, took 62.8 us here (now 9.0), 48 rows of 256 .. 32 768 keys with 8
+// heads a group 14.1 us (13.2).  A team costs about 2 us (barriers, the
+// states' way through LDS): rows of up to sixteen partials (eight with two
+// head passes) stay with one wave (33 rows of up to 14 partials: 8.0 us
+// alone, 9.5 with teams from nine on; 64 rows of about 5: 7.3, 12.5 with
+// teams from five on; the 48 rows: 16.0 with teams only from thirteen on).
+template <int NH>
 __device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units, int wg, MergeLds& lds) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int k = wg / a.Hkv * kMergeWaves + w;
   MergeRow r = merge_row(a, k * a.Hkv + wg % a.Hkv, units);
-  if (r.k_last >= 0 && r.k_last - r.k < kMergeAlone) {
-    if (a.g <= 4) {
-      merge_heads<1>(a, r, 0, lane);
-    } else {
-      for (int c0 = 0; c0 < a.g; c0 += 8) merge_heads<2>(a, r, c0, lane);
-    }
+  if (r.k_last >= 0 && r.k_last - r.k < kMergeAlone<NH>) {
+    for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_heads<NH>(a, r, c0, lane);
     r.k_last = -1;
   }
   if (lane == 0) lds.rows[w] = r;
@@ -263,11 +265,12 @@ __device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units,
       if (t == team) x = lds.rows[__ffs(rest) - 1];
       rest &= rest - 1;
     }
-    if (a.g <= 4) {
-      merge_pass<1>(a, x, w, w % waves, waves, 0, lane, lds);
-    } else {
-      for (int c0 = 0; c0 < a.g; c0 += 8) merge_pass<2>(a, x, w, w % waves, waves, c0, lane, lds);
-    }
+    x.k = __builtin_amdgcn_readfirstlane(x.k);
+    x.h = __builtin_amdgcn_readfirstlane(x.h);
+    x.k_last = __builtin_amdgcn_readfirstlane(x.k_last);
+    x.slot_k = __builtin_amdgcn_readfirstlane(x.slot_k);
+    x.q_row = __builtin_amdgcn_readfirstlane(x.q_row);
+    for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_pass<NH>(a, x, w, w % waves, waves, c0, lane, lds);
   }
 }
 

@@ -82,11 +82,12 @@ void paged_decode_kernel(DecodeArgs a, const int32_t* __restrict__ bt, const int
 // is dispatched sooner than one of many single-wave ones.
 // The work-groups after the first `wgs` merge the parts of prefill entries
 // split along the keys.
+template <int NH>
 __global__ __launch_bounds__(64 * kMergeWaves) void decode_merge_kernel(DecodeArgs a, int units, int wgs,
                                                                         PartMergeArgs parts) {
   __shared__ MergeLds lds;
   if ((int)blockIdx.x < wgs)
-    merge_split_rows(a, units, (int)blockIdx.x, lds);
+    merge_split_rows<NH>(a, units, (int)blockIdx.x, lds);
   else
     merge_parts(parts, (int)blockIdx.x - wgs);
 }
@@ -138,8 +139,11 @@ int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream, con
   const int units = groups > 1 ? (groups - 1) * a.Hkv : 0;
   const int wgs = units > 0 ? merge_wgs(units, a.Hkv) : 0;
   if (wgs + parts.wgs == 0) return NVS_OK;
-  hipLaunchKernelGGL(decode_merge_kernel, dim3(wgs + parts.wgs), dim3(64 * kMergeWaves), 0, stream, a, units, wgs,
-                     parts);
+  const dim3 grid(wgs + parts.wgs), block(64 * kMergeWaves);
+  if (a.g <= 4)
+    hipLaunchKernelGGL(decode_merge_kernel<1>, grid, block, 0, stream, a, units, wgs, parts);
+  else
+    hipLaunchKernelGGL(decode_merge_kernel<2>, grid, block, 0, stream, a, units, wgs, parts);
   return check_launch("decode_merge");
 }
 

@@ -25,8 +25,9 @@ struct PartMergeArgs {
 //
 // A work-group merges one wave's part of one unit (64 rows), its waves
 // taking the (n, qb) blocks' halves, so that a few hundred units fill the
-// chip.  It is bound by the slots' bytes, 132 KiB a part and unit; four
-// parts' loads are in flight at a time.
+// chip.  It is bound by the slots' bytes, 132 KiB a part and unit, and their
+// loads' latency, four parts in flight at a time: 152 slots 3.6 us, 504 slots
+// 9.3 us (7 TB/s) beyond a launch that merges nothing (4.7 us).
 __device__ __forceinline__ void merge_parts(const PartMergeArgs& a, int wg) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int n = w >> 2, qb = (w >> 1) & 1, kh = w & 1, qc = lane & 31, h = lane >> 5;

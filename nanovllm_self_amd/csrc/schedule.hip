@@ -453,7 +453,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
     std::conditional_t<MERGE, MergeLds, NoEntries> merge;
   } lds;
   if constexpr (MERGE) if (blockIdx.x > 0) {
-    merge_split_rows(m, merge_units, (int)blockIdx.x - 1, lds.merge);
+    merge_split_rows<2>(m, merge_units, (int)blockIdx.x - 1, lds.merge);
     return;
   }
   int* scan_lds = lds.plan.scan;

@@ -1,5 +1,5 @@
 """Decode rows split across few, several and very many groups, so that the
-merge of their partials takes each of its routes: one wave alone (up to eight
+merge of their partials takes each of its routes: one wave alone (up to sixteen
 partials), a team of four, eight or sixteen waves, and several rounds of
 teams, for one, a few and all sixteen query heads a kv head, in a decode call
 and in a call with prefill rows (where the merge follows another launch).
