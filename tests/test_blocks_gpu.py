@@ -86,3 +86,25 @@ def test_round_trip_and_errors(device):
         import_kv_blocks(b, b_sc, *export_kv_blocks(a, a_sc, [1]), [40])
     with pytest.raises(RuntimeError, match="no kv_scale_cache"):
         import_kv_blocks(b, None, *export_kv_blocks(a, a_sc, [1]), [3])
+
+
+@pytest.mark.parametrize("planes,nb,copies,block_bytes", [
+    (2, 9, 5, 16), (3, 4, 4, 1008), (2, 3, 2, 1024 + 16), (1, 2, 2, 5 * 1024 - 16),  # remainders of a 1 KiB chunk
+    (1, 70001, 70001, 16), (65537, 1, 1, 16),  # past the grid's copies and planes
+])
+def test_copy_blocks_sizes(device, planes, nb, copies, block_bytes):
+    from nanovllm_self_amd import _lib
+    say(f"copy_blocks {planes} planes {copies} of {nb} blocks of {block_bytes} bytes")
+    gen = torch.Generator().manual_seed(3)
+    src = torch.randint(0, 256, (planes, nb, block_bytes), generator=gen, dtype=torch.uint8)
+    dst = torch.randint(0, 256, (planes, nb + 1, block_bytes), generator=gen, dtype=torch.uint8)
+    sid = torch.randperm(nb, generator=gen)[:copies]
+    did = torch.randperm(nb + 1, generator=gen)[:copies]
+    want = dst.clone()
+    want[:, did] = src[:, sid]
+    s, d = src.to(device), dst.to(device)
+    si, di = sid.to(torch.int32).to(device), did.to(torch.int32).to(device)
+    _lib.check(_lib.load().nvs_copy_blocks(s.data_ptr(), nb, si.data_ptr(), d.data_ptr(), nb + 1, di.data_ptr(), planes,
+                                           block_bytes, copies, _lib.stream_of(s)), "copy_blocks")
+    torch.cuda.synchronize()
+    assert torch.equal(d.cpu(), want)
