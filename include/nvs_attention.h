@@ -385,6 +385,29 @@ int nvs_varlen_attention_dtype(const void* q, int64_t q_tok_stride,
                                int64_t workspace_bytes, void* stream, int dtype);
 
 /*
+ * nvs_store_kvcache (of the step's k and v, dtype both) and then
+ * nvs_varlen_attention_dtype over them, as forward_unified makes them for a
+ * batch without a cached prefix (attention.py:500-546): the same results,
+ * with the write in the attention's planning launch where the batch is
+ * small.  num_tokens rows of q, k and v.
+ */
+int nvs_varlen_attention_store(const void* q, int64_t q_tok_stride,
+                               int64_t q_head_stride, const void* k, const void* v,
+                               int64_t k_tok_stride, int64_t k_head_stride,
+                               int64_t v_tok_stride, int64_t v_head_stride,
+                               const int32_t* slot_mapping, void* k_cache,
+                               void* v_cache, int cache_dtype, float* k_scale,
+                               float* v_scale, int64_t num_blocks, int block_size,
+                               const int32_t* cu_seqlens_q,
+                               const int32_t* cu_seqlens_k, int num_seqs,
+                               int64_t num_tokens, int max_seqlen_q,
+                               int max_seqlen_k, int num_heads, int num_kv_heads,
+                               int head_dim, float softmax_scale, void* out,
+                               int64_t out_tok_stride, int64_t out_head_stride,
+                               void* workspace, int64_t workspace_bytes,
+                               void* stream, int dtype);
+
+/*
  * Step metadata built on the device.  Replaces the per-token loops of
  * ModelRunner.prepare_model_input (reference model_runner.py:461-532) that
  * form cu_seqlens_q/k, context_lens, positions and slot_mapping, and the

@@ -7,6 +7,7 @@
 #include "nvs_common.h"
 #include "attention_common.h"
 #include "decode_merge.h"
+#include "store_rows.h"
 
 using namespace nvs;
 
@@ -220,6 +221,14 @@ static int check_workspace(const AttnParams& P, const char* who) {
   return NVS_OK;
 }
 
+// A call that ended before any launch (nothing to attend, or arguments the
+// attention refuses) still writes the step's k / v.
+static int write_left(const AttnParams& P, int rc, void* stream) {
+  if (!P.store) return rc;
+  const int st = launch_store_job(*P.store, (hipStream_t)stream);
+  return rc != NVS_OK ? rc : st;
+}
+
 // nvs_paged_attention's body; P.kn != null asks the decode kernel to store
 // the step's new tokens itself (decode rows only).
 static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stride, int64_t q_head_stride,
@@ -281,6 +290,13 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
   // too (its first work-groups, before they join the prefill); the merge of
   // split rows follows it.
   const int co_wgs = (shadow || prefill_mx_serves(P)) ? co_decode_wgs(P) : 0;
+  const StoreJob* store = P.store;
+  if (store && !(co_wgs > 0 && plan_launch_stores(*store))) {
+    rc = launch_store_job(*store, s);
+    if (rc != NVS_OK) return rc;
+    store = nullptr;
+  }
+  P.store = nullptr;
   if (co_wgs > 0) {
     CoDecode co;
     co.a = decode_args(P, max_waves, partials);
@@ -293,7 +309,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
         split_job(P, plan, base + (shadow ? shadow_bytes(P.B, P.max_seqlen_k, P.Hkv) : 0), co_wgs);
     const SplitJob* sp = split.slots > 0 ? &split : nullptr;
     if (!shadow) {
-      rc = launch_plan(P, plan, /*paged=*/true, s, nullptr, nullptr, &co, sp);
+      rc = launch_plan(P, plan, /*paged=*/true, s, nullptr, nullptr, &co, sp, store);
       if (rc != NVS_OK) return rc;
       rc = launch_prefill_mx(P, plan, s, &co, sp);
       if (rc != NVS_OK) return rc;
@@ -302,7 +318,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
     // Code cache: the prefill reads the bf16 copy, the decode waves the
     // codes; they run whichever prefill kernel the plan lets serve.
     const ShadowLayout sh = shadow_at((char*)workspace + base, P.B, P.max_seqlen_k, P.Hkv);
-    rc = launch_plan(P, plan, /*paged=*/true, s, &sh, nullptr, &co, sp);
+    rc = launch_plan(P, plan, /*paged=*/true, s, &sh, nullptr, &co, sp, store);
     if (rc != NVS_OK) return rc;
     rc = launch_shadow_fill(P, plan, sh, s);
     if (rc != NVS_OK) return rc;
@@ -400,17 +416,24 @@ extern "C" int nvs_paged_attention_store(const void* q, int64_t q_tok_stride, in
   if (fused) {
     P.kn = k; P.vn = v; P.slots = slot_mapping;
     P.kn_ts = k_tok_stride; P.kn_hs = k_head_stride; P.vn_ts = v_tok_stride; P.vn_hs = v_head_stride;
-  } else {
-    const int rc = nvs_store_kvcache(k, v, src_dtype, k_tok_stride, k_head_stride, v_tok_stride, v_head_stride,
-                                     slot_mapping, num_tokens, k_cache, v_cache, cache_dtype, k_scale, v_scale,
-                                     num_blocks, block_size, num_kv_heads, head_dim, stream);
-    if (rc != NVS_OK) return rc;
   }
-  return paged_attention_impl(P, q, q_tok_stride, q_head_stride, k_cache, v_cache, cache_dtype, k_scale, v_scale,
-                              cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride, num_seqs, num_tokens,
-                              max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim, block_size,
-                              num_blocks, softmax_scale, out, out_tok_stride, out_head_stride, workspace,
-                              workspace_bytes, stream);
+  StoreJob job;
+  if (!fused) {
+    NVS_REQUIRE(num_tokens >= 0, NVS_ERR_INVALID, "store_kvcache: num_tokens < 0");
+    if (num_tokens > 0) {
+      const int rc = make_store_job(job, k, v, src_dtype, k_tok_stride, k_head_stride, v_tok_stride, v_head_stride,
+                                    slot_mapping, num_tokens, k_cache, v_cache, cache_dtype, k_scale, v_scale,
+                                    num_blocks, block_size, num_kv_heads, head_dim);
+      if (rc != NVS_OK) return rc;
+      P.store = &job;
+    }
+  }
+  const int rc =
+      paged_attention_impl(P, q, q_tok_stride, q_head_stride, k_cache, v_cache, cache_dtype, k_scale, v_scale,
+                           cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride, num_seqs, num_tokens, max_seqlen_q,
+                           max_seqlen_k, num_heads, num_kv_heads, head_dim, block_size, num_blocks, softmax_scale, out,
+                           out_tok_stride, out_head_stride, workspace, workspace_bytes, stream);
+  return write_left(P, rc, stream);
 }
 
 static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_head_stride,
@@ -421,8 +444,8 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
                                  int64_t num_kv_tokens, int max_seqlen_q, int max_seqlen_k, int num_heads,
                                  int num_kv_heads, int head_dim, float softmax_scale, void* out,
                                  int64_t out_tok_stride, int64_t out_head_stride,
-                                 void* workspace, int64_t workspace_bytes, void* stream, int dtype) {
-  AttnParams P = {};
+                                 void* workspace, int64_t workspace_bytes, void* stream, int dtype,
+                                 AttnParams& P) {
   P.cache_dtype = dtype;  // the element type of q, k, v and out
   P.ws = workspace; P.ws_bytes = workspace_bytes;
   P.q = q; P.q_ts = q_tok_stride; P.q_hs = q_head_stride;
@@ -453,6 +476,13 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
   if (rc != NVS_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
   const Plan plan = make_plan(workspace, P);
+  const StoreJob* store = P.store;
+  if (store && !(prefill_mx_serves(P) && plan_launch_stores(*store))) {
+    rc = launch_store_job(*store, s);
+    if (rc != NVS_OK) return rc;
+    store = nullptr;
+  }
+  P.store = nullptr;
   if (!prefill_mx_serves(P)) {
     rc = launch_plan(P, plan, /*paged=*/false, s);
     return rc != NVS_OK ? rc : launch_prefill(P, plan, s);
@@ -460,7 +490,7 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
   const SplitJob split = split_job(P, plan, attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv),
                                    prefill_mx_wgs(P, plan));
   const SplitJob* sp = split.slots > 0 ? &split : nullptr;
-  rc = launch_plan(P, plan, /*paged=*/false, s, nullptr, nullptr, nullptr, sp);
+  rc = launch_plan(P, plan, /*paged=*/false, s, nullptr, nullptr, nullptr, sp, store);
   if (rc != NVS_OK) return rc;
   rc = launch_prefill_mx(P, plan, s, nullptr, sp);
   if (rc != NVS_OK) return rc;
@@ -477,11 +507,12 @@ extern "C" int nvs_varlen_attention(const void* q, int64_t q_tok_stride, int64_t
                                     int64_t out_tok_stride, int64_t out_head_stride,
                                     void* workspace, int64_t workspace_bytes, void* stream) {
   clear_error();
+  AttnParams P = {};
   return varlen_attention_impl(q, q_tok_stride, q_head_stride, k, v, k_tok_stride, k_head_stride, v_tok_stride,
                                v_head_stride, cu_seqlens_q, cu_seqlens_k, num_seqs, num_tokens, num_kv_tokens,
                                max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, out,
                                out_tok_stride, out_head_stride, workspace, workspace_bytes, stream,
-                               NVS_DTYPE_BF16);
+                               NVS_DTYPE_BF16, P);
 }
 
 extern "C" int nvs_varlen_attention_dtype(const void* q, int64_t q_tok_stride, int64_t q_head_stride,
@@ -494,8 +525,37 @@ extern "C" int nvs_varlen_attention_dtype(const void* q, int64_t q_tok_stride, i
                                           void* out, int64_t out_tok_stride, int64_t out_head_stride,
                                           void* workspace, int64_t workspace_bytes, void* stream, int dtype) {
   clear_error();
+  AttnParams P = {};
   return varlen_attention_impl(q, q_tok_stride, q_head_stride, k, v, k_tok_stride, k_head_stride, v_tok_stride,
                                v_head_stride, cu_seqlens_q, cu_seqlens_k, num_seqs, num_tokens, num_kv_tokens,
                                max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim, softmax_scale, out,
-                               out_tok_stride, out_head_stride, workspace, workspace_bytes, stream, dtype);
+                               out_tok_stride, out_head_stride, workspace, workspace_bytes, stream, dtype, P);
+}
+
+extern "C" int nvs_varlen_attention_store(const void* q, int64_t q_tok_stride, int64_t q_head_stride, const void* k,
+                                          const void* v, int64_t k_tok_stride, int64_t k_head_stride,
+                                          int64_t v_tok_stride, int64_t v_head_stride, const int32_t* slot_mapping,
+                                          void* k_cache, void* v_cache, int cache_dtype, float* k_scale, float* v_scale,
+                                          int64_t num_blocks, int block_size, const int32_t* cu_seqlens_q,
+                                          const int32_t* cu_seqlens_k, int num_seqs, int64_t num_tokens,
+                                          int max_seqlen_q, int max_seqlen_k, int num_heads, int num_kv_heads,
+                                          int head_dim, float softmax_scale, void* out, int64_t out_tok_stride,
+                                          int64_t out_head_stride, void* workspace, int64_t workspace_bytes,
+                                          void* stream, int dtype) {
+  clear_error();
+  AttnParams P = {};
+  StoreJob job;
+  NVS_REQUIRE(num_tokens >= 0, NVS_ERR_INVALID, "store_kvcache: num_tokens < 0");
+  if (num_tokens > 0) {
+    const int rc = make_store_job(job, k, v, dtype, k_tok_stride, k_head_stride, v_tok_stride, v_head_stride,
+                                  slot_mapping, num_tokens, k_cache, v_cache, cache_dtype, k_scale, v_scale,
+                                  num_blocks, block_size, num_kv_heads, head_dim);
+    if (rc != NVS_OK) return rc;
+    P.store = &job;
+  }
+  const int rc = varlen_attention_impl(
+      q, q_tok_stride, q_head_stride, k, v, k_tok_stride, k_head_stride, v_tok_stride, v_head_stride, cu_seqlens_q,
+      cu_seqlens_k, num_seqs, num_tokens, num_tokens, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, head_dim,
+      softmax_scale, out, out_tok_stride, out_head_stride, workspace, workspace_bytes, stream, dtype, P);
+  return write_left(P, rc, stream);
 }

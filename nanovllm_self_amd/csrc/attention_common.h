@@ -222,6 +222,8 @@ inline Plan plan_at(void* ws, int B, int ntq, int pbm) {
 // `per_cu` resident work-groups per CU (CU count cached per device).
 int device_slots(int per_cu);
 
+struct StoreJob;
+
 // Validated launch parameters of one attention call.
 struct AttnParams {
   const void* q;
@@ -250,6 +252,9 @@ struct AttnParams {
   const void* vn;
   int64_t kn_ts, kn_hs, vn_ts, vn_hs;
   const int32_t* slots;
+  // The write of the step's k / v that comes before the attention, until a
+  // launch has made it (null: none is left to make).
+  const StoreJob* store;
   int64_t T;   // query / output rows
   int64_t Tk;  // rows of the local k/v (varlen mode)
   int max_seqlen_q, max_seqlen_k;
@@ -320,13 +325,16 @@ int64_t attention_workspace_bytes(int num_seqs, int max_seqlen_q, int max_seqlen
 int decode_launch_waves(int max_waves, int Hkv);
 struct MergeJob;
 struct CoDecode;
+struct StoreJob;
 // The plan kernel; with `merge` it also runs the decode launch's merge of
 // split rows (extra work-groups beside the plan's); with `co` it sizes the
 // decode part of the prefill launch (PlanHeader::dec_wgs) and clears the
 // decode waves' header.
 int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t stream,
                 const ShadowLayout* shadow = nullptr, const MergeJob* merge = nullptr,
-                const CoDecode* co = nullptr, const SplitJob* split = nullptr);
+                const CoDecode* co = nullptr, const SplitJob* split = nullptr, const StoreJob* store = nullptr);
+// Whether the plan launch can make this write of the step's k / v too.
+bool plan_launch_stores(const StoreJob& job);
 // Rates the plan sizes the co-scheduled decode with: decode bytes per
 // second of one CU beside the prefill and of the whole chip, prefill FLOP
 // per second of one CU, and the fraction of the call by which the decode

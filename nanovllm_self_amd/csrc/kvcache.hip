@@ -11,6 +11,7 @@
 
 #include "nvs_common.h"
 #include "store_common.h"
+#include "store_rows.h"
 
 namespace nvs {
 
@@ -38,71 +39,11 @@ int check_launch(const char* what) {
 }
 
 // ---------------------------------------------------------------------------
-// KV-cache write.  One thread owns 8 consecutive head_dim elements of one
-// (token, kv_head) row of both K and V; lpr = head_dim / 8 lanes form a row.
-// With IDENT the destination row is the token index itself (used by
-// nvs_quantize_per_token), otherwise slot_mapping[token].
+// KV-cache write as a launch of its own (store_rows.h)
 // ---------------------------------------------------------------------------
-struct StoreArgs {
-  const void* k;
-  const void* v;
-  int64_t k_ts, k_hs, v_ts, v_hs;
-  const int32_t* slots;
-  int64_t rows;         // num_tokens * H
-  int64_t total_slots;  // num_blocks * block_size
-  void* kc;
-  void* vc;
-  float* ks;
-  float* vs;
-  int H, D, lpr_log2;
-};
-
 template <int SRC, int DST, bool IDENT, bool HAS_V>
 __global__ __launch_bounds__(256) void store_kv_kernel(StoreArgs a) {
-  const int lpr = 1 << a.lpr_log2;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t row = gid >> a.lpr_log2;
-  const int c = (int)(gid & (lpr - 1));
-  const bool active = row < a.rows;
-  const int64_t t = active ? row / a.H : 0;
-  const int h = active ? (int)(row - t * a.H) : 0;
-  int64_t slot = -1;
-  if (active) slot = IDENT ? t : (int64_t)a.slots[t];
-  const bool valid = active && slot >= 0 && slot < a.total_slots;
-
-  constexpr int SRC_BYTES = (SRC == NVS_DTYPE_FP32) ? 4 : 2;
-  float xk[8], xv[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) xk[i] = xv[i] = 0.0f;
-  if (valid) {
-    load8<SRC>((const char*)a.k + (t * a.k_ts + h * a.k_hs + c * 8) * SRC_BYTES, xk);
-    if constexpr (HAS_V)
-      load8<SRC>((const char*)a.v + (t * a.v_ts + h * a.v_hs + c * 8) * SRC_BYTES, xv);
-  }
-  const int64_t dst_row = slot * a.H + h;  // (block*bs + off) * H + h
-  const int64_t dst_elem = dst_row * a.D + c * 8;
-
-  if constexpr (DST == NVS_DTYPE_INT8 || DST == NVS_DTYPE_FP8_E4M3) {
-    // All lanes of a row take part in the reduction, valid or not.
-    constexpr float qmax = (DST == NVS_DTYPE_INT8) ? QuantInt8::kQmax : QuantFp8::kQmax;
-    const float sk = quant_scale(row_absmax(xk, lpr), qmax);
-    float sv = 0.0f;
-    if constexpr (HAS_V) sv = quant_scale(row_absmax(xv, lpr), qmax);
-    if (valid) {
-      *reinterpret_cast<u32x2*>((uint8_t*)a.kc + dst_elem) = quant8<DST, SRC != NVS_DTYPE_FP32>(xk, sk);
-      if (c == 0) a.ks[dst_row] = sk;
-      if constexpr (HAS_V) {
-        *reinterpret_cast<u32x2*>((uint8_t*)a.vc + dst_elem) = quant8<DST, SRC != NVS_DTYPE_FP32>(xv, sv);
-        if (c == 0) a.vs[dst_row] = sv;
-      }
-    }
-  } else {
-    constexpr int DST_BYTES = (DST == NVS_DTYPE_FP32) ? 4 : 2;
-    if (valid) {
-      store8_float<DST>((char*)a.kc + dst_elem * DST_BYTES, xk);
-      if constexpr (HAS_V) store8_float<DST>((char*)a.vc + dst_elem * DST_BYTES, xv);
-    }
-  }
+  store_rows<SRC, DST, IDENT, HAS_V>(a, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 static int lpr_log2_for(int D) {
@@ -282,17 +223,11 @@ extern "C" const char* nvs_last_error(void) { return g_err; }
 
 extern "C" int nvs_version(void) { return 100; }
 
-extern "C" int nvs_store_kvcache(const void* k, const void* v, int src_dtype,
-                                 int64_t k_tok_stride, int64_t k_head_stride,
-                                 int64_t v_tok_stride, int64_t v_head_stride,
-                                 const int32_t* slot_mapping, int64_t num_tokens,
-                                 void* k_cache, void* v_cache, int cache_dtype,
-                                 float* k_scale, float* v_scale, int64_t num_blocks,
-                                 int block_size, int num_kv_heads, int head_dim,
-                                 void* stream) {
-  clear_error();
-  NVS_REQUIRE(num_tokens >= 0, NVS_ERR_INVALID, "store_kvcache: num_tokens < 0");
-  if (num_tokens == 0) return NVS_OK;
+int nvs::make_store_job(StoreJob& job, const void* k, const void* v, int src_dtype, int64_t k_tok_stride,
+                        int64_t k_head_stride, int64_t v_tok_stride, int64_t v_head_stride,
+                        const int32_t* slot_mapping, int64_t num_tokens, void* k_cache, void* v_cache, int cache_dtype,
+                        float* k_scale, float* v_scale, int64_t num_blocks, int block_size, int num_kv_heads,
+                        int head_dim) {
   NVS_REQUIRE(k && v && slot_mapping && k_cache && v_cache, NVS_ERR_INVALID,
               "store_kvcache: null tensor pointer");
   NVS_REQUIRE(src_dtype == NVS_DTYPE_BF16 || src_dtype == NVS_DTYPE_FP16 ||
@@ -312,7 +247,9 @@ extern "C" int nvs_store_kvcache(const void* k, const void* v, int src_dtype,
                   (v_tok_stride * sb) % 16 == 0 && (v_head_stride * sb) % 16 == 0 &&
                   ((uintptr_t)k % 16) == 0 && ((uintptr_t)v % 16) == 0,
               NVS_ERR_INVALID, "store_kvcache: k/v rows must be 16-byte aligned");
-  StoreArgs a;
+  StoreArgs& a = job.a;
+  job.src = src_dtype;
+  job.dst = cache_dtype;
   a.k = k; a.v = v;
   a.k_ts = k_tok_stride; a.k_hs = k_head_stride;
   a.v_ts = v_tok_stride; a.v_hs = v_head_stride;
@@ -321,7 +258,29 @@ extern "C" int nvs_store_kvcache(const void* k, const void* v, int src_dtype,
   a.total_slots = num_blocks * (int64_t)block_size;
   a.kc = k_cache; a.vc = v_cache; a.ks = k_scale; a.vs = v_scale;
   a.H = num_kv_heads; a.D = head_dim; a.lpr_log2 = l2;
-  return launch_store<false, true>(a, src_dtype, cache_dtype, (hipStream_t)stream);
+  return NVS_OK;
+}
+
+int nvs::launch_store_job(const StoreJob& job, hipStream_t stream) {
+  return launch_store<false, true>(job.a, job.src, job.dst, stream);
+}
+
+extern "C" int nvs_store_kvcache(const void* k, const void* v, int src_dtype,
+                                 int64_t k_tok_stride, int64_t k_head_stride,
+                                 int64_t v_tok_stride, int64_t v_head_stride,
+                                 const int32_t* slot_mapping, int64_t num_tokens,
+                                 void* k_cache, void* v_cache, int cache_dtype,
+                                 float* k_scale, float* v_scale, int64_t num_blocks,
+                                 int block_size, int num_kv_heads, int head_dim,
+                                 void* stream) {
+  clear_error();
+  NVS_REQUIRE(num_tokens >= 0, NVS_ERR_INVALID, "store_kvcache: num_tokens < 0");
+  if (num_tokens == 0) return NVS_OK;
+  StoreJob job;
+  const int rc = make_store_job(job, k, v, src_dtype, k_tok_stride, k_head_stride, v_tok_stride, v_head_stride,
+                                slot_mapping, num_tokens, k_cache, v_cache, cache_dtype, k_scale, v_scale, num_blocks,
+                                block_size, num_kv_heads, head_dim);
+  return rc != NVS_OK ? rc : launch_store_job(job, (hipStream_t)stream);
 }
 
 extern "C" int nvs_quantize_per_token(const void* x, int src_dtype, int64_t tok_stride,

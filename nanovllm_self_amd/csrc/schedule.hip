@@ -3,6 +3,7 @@
 #include "nvs_common.h"
 #include "attention_common.h"
 #include "decode_merge.h"
+#include "store_rows.h"
 #include <climits>
 #include <type_traits>
 
@@ -437,28 +438,21 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
   return list;
 }
 
-// Work-group 0 writes the plan; the others (a paged call whose decode
-// launch left its merge to this one) merge the decode rows split across
-// groups, one merge wave per wave.
-template <bool PARTS, bool MERGE>
-__global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeArgs m, int merge_units) {
+template <bool PARTS>
+struct PlanLds {
   struct NoEntries {};
-  __shared__ union Lds {
-    struct {
-      PlanRows rows;
-      int scan[kPlanWaves];
-      float sum[kPlanWaves][3];
-      std::conditional_t<PARTS, PlanEntries, NoEntries> entries;
-    } plan;
-    std::conditional_t<MERGE, MergeLds, NoEntries> merge;
-  } lds;
-  if constexpr (MERGE) if (blockIdx.x > 0) {
-    merge_split_rows<2>(m, merge_units, (int)blockIdx.x - 1, lds.merge);
-    return;
-  }
-  int* scan_lds = lds.plan.scan;
-  float (*sum_lds)[3] = lds.plan.sum;
-  PlanRows& rows = lds.plan.rows;
+  PlanRows rows;
+  int scan[kPlanWaves];
+  float sum[kPlanWaves][3];
+  std::conditional_t<PARTS, PlanEntries, NoEntries> entries;
+};
+
+// The plan, by one work-group.
+template <bool PARTS>
+__device__ __forceinline__ void write_plan(const PlanArgs& a, PlanLds<PARTS>& lds) {
+  int* scan_lds = lds.scan;
+  float (*sum_lds)[3] = lds.sum;
+  PlanRows& rows = lds.rows;
   const int tid = threadIdx.x;
   const Plan& pl = a.plan;
   if (tid < 8) pl.hdr->prefill_next[tid] = 0;
@@ -530,7 +524,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
           dec_wgs = decode_wgs(a, dec_rows, dec_tiles, pairs, sum_lds);
           wgs = max(8, a.co_wgs - dec_wgs);
         }
-        base = plan_parts(a, rows, lds.plan.entries, shadow, tot, wgs);
+        base = plan_parts(a, rows, lds.entries, shadow, tot, wgs);
         parted = true;
         break;
       }
@@ -563,6 +557,65 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
   }
 }
 
+// Work-group 0 writes the plan; the others (a paged call whose decode
+// launch left its merge to this one) merge the decode rows split across
+// groups, one merge wave per wave.
+__global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeArgs m, int merge_units) {
+  __shared__ union Lds {
+    PlanLds<false> plan;
+    MergeLds merge;
+  } lds;
+  if (blockIdx.x > 0)
+    merge_split_rows<2>(m, merge_units, (int)blockIdx.x - 1, lds.merge);
+  else
+    write_plan<false>(a, lds.plan);
+}
+
+template <bool PARTS>
+__global__ __launch_bounds__(kPlanThreads) void plan_only_kernel(PlanArgs a) {
+  __shared__ PlanLds<PARTS> lds;
+  write_plan<PARTS>(a, lds);
+}
+
+// The plan by work-group 0 and the write of the step's k / v by the others:
+// neither reads what the other writes, and a small step's write (5 us) and
+// plan (4 .. 13 us) are each mostly latency.  Chosen for writes of up to two
+// work-groups a CU; a long one is bound by HBM and keeps its own launch,
+// whose small work-groups stream faster.
+template <bool PARTS, int SRC, int DST>
+__global__ __launch_bounds__(kPlanThreads) void plan_store_kernel(PlanArgs a, StoreArgs st) {
+  __shared__ PlanLds<PARTS> lds;
+  if (blockIdx.x > 0)
+    store_rows<SRC, DST, false, true>(st, (int64_t)(blockIdx.x - 1) * kPlanThreads + threadIdx.x);
+  else
+    write_plan<PARTS>(a, lds);
+}
+
+// The element types the plan launch writes.
+static bool plan_stores(const StoreJob& job) {
+  const int s = job.src, d = job.dst;
+  return (s == NVS_DTYPE_FP16 && d == NVS_DTYPE_FP16) ||
+         (s == NVS_DTYPE_BF16 && (d == NVS_DTYPE_BF16 || d == NVS_DTYPE_FP8_E4M3 || d == NVS_DTYPE_INT8));
+}
+static int64_t store_wgs(const StoreJob& job) {
+  return ((job.a.rows << job.a.lpr_log2) + kPlanThreads - 1) / kPlanThreads;
+}
+bool plan_launch_stores(const StoreJob& job) { return plan_stores(job) && store_wgs(job) <= device_slots(2); }
+
+template <bool PARTS>
+static void launch_plan_store(const PlanArgs& a, const StoreJob& job, hipStream_t stream) {
+  const dim3 grid((unsigned)(1 + store_wgs(job))), block(kPlanThreads);
+  if (job.src == NVS_DTYPE_FP16)
+    hipLaunchKernelGGL((plan_store_kernel<PARTS, NVS_DTYPE_FP16, NVS_DTYPE_FP16>), grid, block, 0, stream, a, job.a);
+  else if (job.dst == NVS_DTYPE_BF16)
+    hipLaunchKernelGGL((plan_store_kernel<PARTS, NVS_DTYPE_BF16, NVS_DTYPE_BF16>), grid, block, 0, stream, a, job.a);
+  else if (job.dst == NVS_DTYPE_FP8_E4M3)
+    hipLaunchKernelGGL((plan_store_kernel<PARTS, NVS_DTYPE_BF16, NVS_DTYPE_FP8_E4M3>), grid, block, 0, stream, a,
+                       job.a);
+  else
+    hipLaunchKernelGGL((plan_store_kernel<PARTS, NVS_DTYPE_BF16, NVS_DTYPE_INT8>), grid, block, 0, stream, a, job.a);
+}
+
 static int g_cus[64] = {0};
 
 int device_slots(int per_cu) {
@@ -578,7 +631,8 @@ int device_slots(int per_cu) {
 }
 
 int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t stream, const ShadowLayout* shadow,
-                const MergeJob* merge, const CoDecode* co, const SplitJob* split) {
+                const MergeJob* merge, const CoDecode* co, const SplitJob* split,
+                const StoreJob* store) {
   PlanArgs a;
   a.cu_q = P.cu_q;
   a.cu_k = P.cu_k;
@@ -617,12 +671,16 @@ int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t s
     units = merge->units;
   }
   const int grid = 1 + (units > 0 ? merge_wgs(units, m.Hkv) : 0);
-  if (a.split_slots > 0)
-    hipLaunchKernelGGL((plan_kernel<true, false>), dim3(1), dim3(kPlanThreads), 0, stream, a, m, units);
+  const bool parts = a.split_slots > 0;
+  const dim3 one(1), block(kPlanThreads);
+  if (store)
+    parts ? launch_plan_store<true>(a, *store, stream) : launch_plan_store<false>(a, *store, stream);
+  else if (parts)
+    hipLaunchKernelGGL(plan_only_kernel<true>, one, block, 0, stream, a);
   else if (units > 0)
-    hipLaunchKernelGGL((plan_kernel<false, true>), dim3(grid), dim3(kPlanThreads), 0, stream, a, m, units);
+    hipLaunchKernelGGL(plan_kernel, dim3(grid), block, 0, stream, a, m, units);
   else
-    hipLaunchKernelGGL((plan_kernel<false, false>), dim3(grid), dim3(kPlanThreads), 0, stream, a, m, units);
+    hipLaunchKernelGGL(plan_only_kernel<false>, one, block, 0, stream, a);
   return check_launch("plan");
 }
 

@@ -273,7 +273,7 @@ class PagedAttention(nn.Module):
     def _attention(self, q, k, v, context, store_slots=None):
         """One call of the HIP attention over the whole (mixed) batch; with
         store_slots the same call first writes k / v to those cache slots
-        (nvs_paged_attention_store, paged mode only)."""
+        (nvs_paged_attention_store, nvs_varlen_attention_store)."""
         # The kernels compute in bf16 or fp16 (attention_compute_dtype,
         # config.py:33-38; the reference's flash path computes in it,
         # attention.py:326-336): the local mode in attention_compute_dtype,
@@ -342,6 +342,24 @@ class PagedAttention(nn.Module):
                 k = k.contiguous()
             if v.stride(-1) != 1:
                 v = v.contiguous()
+            if store_slots is not None:  # _store_in_prefill: k / v and the cache in their types
+                kc, ks, vs = self.k_cache, self.k_scale_cache, self.v_scale_cache
+                quant = self.kv_cache_quant_mode in _QUANT_DTYPE
+                slots = store_slots.to(torch.int32).contiguous()
+                _lib.check(
+                    lib.nvs_varlen_attention_store(
+                        q.data_ptr(), q.stride(0), q.stride(1),
+                        k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
+                        slots.data_ptr(), kc.data_ptr(), self.v_cache.data_ptr(), _lib.nvs_dtype(kc.dtype),
+                        _lib.ptr(ks if quant else None), _lib.ptr(vs if quant else None), kc.shape[0], kc.shape[1],
+                        cu_q.data_ptr(), cu_k.data_ptr(), B, T, max_q, max_k,
+                        self.num_heads, self.num_kv_heads, self.head_dim, scale,
+                        out.data_ptr(), out.stride(0), out.stride(1), _lib.ptr(ws), ws_bytes, stream,
+                        _lib.nvs_dtype(compute),
+                    ),
+                    "varlen_attention_store",
+                )
+                return out if self.dtype == compute else out.to(self.dtype)
             _lib.check(
                 lib.nvs_varlen_attention_dtype(
                     q.data_ptr(), q.stride(0), q.stride(1),
@@ -466,6 +484,43 @@ class PagedAttention(nn.Module):
             and k.stride(-1) == 1 and v.stride(-1) == 1
         )
 
+    def _store_in_prefill(self, q, k, v, context) -> bool:
+        """True when the write of a batch with prefill rows can be part of
+        the attention call (its planning launch makes it where it is short):
+        the types and layouts that write_kv_cache and the attention method
+        both take as they are, and neither method replaced on this layer."""
+        cls = type(self)
+        attn_fn = "prefill_torch" if self.forward_backend == "torch" else "prefill_flashattn"
+        kc, vc, mode = self.k_cache, self.v_cache, self.kv_cache_quant_mode
+        compute = self.attention_compute_dtype
+        if kc is None or vc is None or compute not in _COMPUTE_DTYPES:
+            return False
+        if mode == "none":
+            cache_ok = kc.dtype == compute and vc.dtype == compute
+        elif mode in _QUANT_DTYPE:
+            ks, vs = self.k_scale_cache, self.v_scale_cache
+            cache_ok = (compute == torch.bfloat16 and kc.dtype == _QUANT_DTYPE[mode] and vc.dtype == kc.dtype
+                        and ks is not None and vs is not None
+                        and ks.dtype == torch.float32 and vs.dtype == torch.float32
+                        and ks.is_contiguous() and vs.is_contiguous())
+        else:
+            return False
+        return (
+            cache_ok
+            and "write_kv_cache" not in self.__dict__ and "store_kv_cache_torch" not in self.__dict__
+            and cls.write_kv_cache is PagedAttention.write_kv_cache
+            and cls.store_kv_cache_torch is PagedAttention.store_kv_cache_torch
+            and attn_fn not in self.__dict__ and getattr(cls, attn_fn) is getattr(PagedAttention, attn_fn)
+            and self.kv_writer_backend in ("torch", "hip")
+            and self.forward_backend in ("flashattn", "hip", "torch")
+            and (context.block_tables is None or int(context.max_seqlen_q) > 1)
+            and k.dtype == compute and v.dtype == compute and k.is_cuda and v.is_cuda and q.is_cuda
+            and kc.is_cuda and vc.is_cuda and context.slot_mapping is not None and context.slot_mapping.is_cuda
+            and kc.is_contiguous() and vc.is_contiguous() and k.stride(-1) == 1 and v.stride(-1) == 1
+            and k.shape == v.shape and q.shape[0] == k.shape[0] and k.shape[0] == context.slot_mapping.numel()
+            and tuple(kc.shape[2:]) == (self.num_kv_heads, self.head_dim) and k.shape[1:] == kc.shape[2:]
+        )
+
     def _decode_slots_private(self, context) -> bool:
         """Host check (one synchronisation) of what the one-call decode write
         relies on beyond what the kernel checks itself: no row of the batch
@@ -504,6 +559,8 @@ class PagedAttention(nn.Module):
         if not should_profile and self._store_in_decode(k, v, context) and (
                 not self.verify_decode_slots or self.in_cuda_graph_capture
                 or self._decode_slots_private(context)):
+            return self._attention(q, k, v, context, store_slots=context.slot_mapping)
+        if not should_profile and self._store_in_prefill(q, k, v, context):
             return self._attention(q, k, v, context, store_slots=context.slot_mapping)
         if should_profile:
             torch.cuda.synchronize()
