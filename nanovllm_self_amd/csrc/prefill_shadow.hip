@@ -59,51 +59,79 @@ __device__ __forceinline__ u32x4 dequant8(u32x2 w, float sc) {
   return o;
 }
 
+// The row of copy tile s: the largest b with base[b] <= s (base is
+// non-decreasing with base[B] = total > s, so that row has tiles).  Sixty-four
+// candidates a round, one a lane: a batch of up to 64 rows takes one load
+// round trip.
+__device__ __forceinline__ int row_of_tile(const int* base, int B, int s, int lane) {
+  int lo = 0, hi = B;
+  while (hi - lo > 1) {
+    const int step = (hi - lo + 63) / 64, i = lo + lane * step;
+    const int n = __popcll(__ballot(i < hi && base[min(i, hi - 1)] <= s));
+    lo += (n - 1) * step;
+    hi = min(lo + step, hi);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// A work-group dequantises a piece of a tile: its 64 keys, or, while the grid
+// holds them all, half, a quarter or an eighth of them.  Sixteen lanes take a
+// token row (eight codes each; 16-byte loads would store every other 16 bytes,
+// 10 % slower), two rows at a time a thread.  Bound by HBM in a long copy, by
+// latency in a short one (the tile's row, block and scales are loads that
+// wait for each other), which small pieces and few round trips shorten; more
+// work-groups than the CUs hold keep the stream dense.  Tiles of 8 heads,
+// fp8: 182 of them (71 MB) 23.5 -> 17.0 us, 504 39.2 -> 34.6, 717 51.7 ->
+// 47.6; 833 of int8 66.2 -> 56.0 (before: whole or half tiles, 1024
+// work-groups that loop, a row searched by halves).
+constexpr int kShadowRows = kShadowThreads / 16;  // token rows of a pass
+constexpr int kShadowPieces = 8;
+constexpr int kShadowUnroll = 2;
+
 template <int KV>
 __global__ __launch_bounds__(kShadowThreads) void shadow_fill_kernel(ShadowArgs a) {
   if (a.hdr->shadow_on == 0) return;
   const int total = a.hdr->shadow_tiles;
   const int j = threadIdx.x & 15;
   const int rows = kShadowTile * a.Hkv;  // token rows of a tile (token-major, then kv head)
-  // A copy whose half tiles (32 keys x Hkv token rows) all fit one pass of
-  // the grid is cut into them, so that it spreads over twice as many
-  // work-groups (mixed_32b's 504 tiles: 45.7 -> 38.3 us); a larger one keeps
-  // whole tiles (prefill_8b's 833 tiles as half tiles: 49.3 -> 53.5 us).
-  const int split = 2 * total <= (int)gridDim.x ? 2 : 1;
-  for (int u = blockIdx.x; u < split * total; u += gridDim.x) {
-    const int s = split == 2 ? u >> 1 : u, half = split == 2 ? u & 1 : 0;
-    // Row b of tile s: base[b] <= s < base[b + 1] (base is non-decreasing
-    // with base[B] = total > s, so the largest such b has tiles).
-    int lo = 0, hi = a.B;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (a.sh.base[mid] <= s) lo = mid; else hi = mid;
-    }
-    const int b = lo;
+  int log_pieces = 0;
+  while ((1 << log_pieces) < kShadowPieces && (int64_t)total << (log_pieces + 1) <= (int64_t)gridDim.x) ++log_pieces;
+  const int span = kShadowTile >> log_pieces;  // keys of a piece
+  for (int64_t u = blockIdx.x; u < (int64_t)total << log_pieces; u += gridDim.x) {
+    const int s = (int)(u >> log_pieces), piece = (int)u & ((1 << log_pieces) - 1);
+    const int b = row_of_tile(a.sh.base, a.B, s, threadIdx.x & 63);
     const int t = s - a.sh.base[b];  // < ST: the plan keeps a row's tiles within its table row
-    if (threadIdx.x == 0 && half == 0) a.sh.table[(int64_t)b * a.sh.ST + t] = s;
+    if (threadIdx.x == 0 && piece == 0) a.sh.table[(int64_t)b * a.sh.ST + t] = s;
     const int K = a.cu_k[b + 1] - a.cu_k[b];
     // The tile's keys lie in one block (block_size is a multiple of 64).
-    const int lb = kShadowTile * t / a.bs;
-    const int64_t nblk = min(((int64_t)K + a.bs - 1) / a.bs, a.bt_stride);
-    int blk = lb < nblk ? a.bt[(int64_t)b * a.bt_stride + lb] : -1;
+    const int lb = (int)((uint32_t)(kShadowTile * t) / (uint32_t)a.bs);
+    int blk = kShadowTile * (int64_t)t < K && lb < a.bt_stride ? a.bt[(int64_t)b * a.bt_stride + lb] : -1;
     if (blk >= a.NB) blk = -1;
-    const int64_t row0 = blk >= 0 ? ((int64_t)blk * a.bs + (kShadowTile * t) % a.bs) * a.Hkv : 0;
+    const int64_t row0 = blk >= 0 ? ((int64_t)blk * a.bs + (kShadowTile * t - lb * a.bs)) * a.Hkv : 0;
     const int keys = min(K - kShadowTile * t, kShadowTile);
     const int64_t out0 = (int64_t)s * rows;
-    const int span = kShadowTile / split;  // keys of the work item
-    const int r_end = min(keys, span * (half + 1)) * a.Hkv;
-    for (int r = span * half * a.Hkv + (threadIdx.x >> 4); r < r_end; r += kShadowThreads / 16) {
-      u32x4 ko = {0u, 0u, 0u, 0u}, vo = {0u, 0u, 0u, 0u};
-      if (blk >= 0) {
-        const int64_t cr = row0 + r;  // cache row (token, kv head)
-        const u32x2 kw = *reinterpret_cast<const u32x2*>(a.kc + cr * kHeadDim + 8 * j);
-        const u32x2 vw = *reinterpret_cast<const u32x2*>(a.vc + cr * kHeadDim + 8 * j);
-        ko = dequant8<KV>(kw, a.ks[cr]);
-        vo = dequant8<KV>(vw, a.vs[cr]);
+    const int r_end = min(keys, span * (piece + 1)) * a.Hkv;
+    for (int r0 = span * piece * a.Hkv + (int)(threadIdx.x >> 4); r0 < r_end; r0 += kShadowUnroll * kShadowRows) {
+      u32x2 kw[kShadowUnroll], vw[kShadowUnroll];
+      float ks[kShadowUnroll], vs[kShadowUnroll];
+#pragma unroll
+      for (int i = 0; i < kShadowUnroll; ++i) {
+        const int r = min(r0 + i * kShadowRows, r_end - 1);
+        const int64_t cr = row0 + (blk >= 0 ? r : 0);  // cache row (token, kv head)
+        kw[i] = *reinterpret_cast<const u32x2*>(a.kc + cr * kHeadDim + 8 * j);
+        vw[i] = *reinterpret_cast<const u32x2*>(a.vc + cr * kHeadDim + 8 * j);
+        ks[i] = a.ks[cr];
+        vs[i] = a.vs[cr];
       }
-      *reinterpret_cast<u32x4*>(a.sh.k + (out0 + r) * kHeadDim + 8 * j) = ko;
-      *reinterpret_cast<u32x4*>(a.sh.v + (out0 + r) * kHeadDim + 8 * j) = vo;
+#pragma unroll
+      for (int i = 0; i < kShadowUnroll; ++i) {
+        const int r = r0 + i * kShadowRows;
+        if (r >= r_end) break;
+        u32x4 ko = dequant8<KV>(kw[i], ks[i]), vo = dequant8<KV>(vw[i], vs[i]);
+        if (blk < 0) ko = vo = u32x4{0u, 0u, 0u, 0u};  // missing block: zeros
+        *reinterpret_cast<u32x4*>(a.sh.k + (out0 + r) * kHeadDim + 8 * j) = ko;
+        *reinterpret_cast<u32x4*>(a.sh.v + (out0 + r) * kHeadDim + 8 * j) = vo;
+      }
     }
   }
 }
@@ -126,8 +154,9 @@ int launch_shadow_fill(const AttnParams& P, const Plan& plan, const ShadowLayout
   a.hdr = plan.hdr;
   a.sh = sh;
   if (P.B <= 0 || sh.cap <= 0) return NVS_OK;
-  // Persistent: a few work-groups per CU, never more than the copy's half tiles.
-  const int wgs = (int)std::min<int64_t>(2 * (int64_t)sh.cap, (int64_t)device_slots(4));
+  // Up to four times the work-groups the CUs hold (8, 16, 32 and 64 a CU: 833
+  // tiles 61.6, 56.3, 56.0 and 55.6 us), never more than the copy's pieces.
+  const int wgs = (int)std::min<int64_t>(kShadowPieces * (int64_t)sh.cap, (int64_t)device_slots(32));
   dim3 grid((unsigned)std::max(1, wgs)), block(kShadowThreads);
   switch (P.cache_dtype) {
     case NVS_DTYPE_INT8:
