@@ -15,14 +15,21 @@
 // Each product and sum is rounded on its own (no fused multiply-add), as the
 // eager torch ops compute them.
 //
-// Work: one wave per token.  Its rows (units) are the Hq query heads, then
-// the Hkv key heads, then the Hkv value heads; the wave's four 16-lane groups
-// take rows g, g + 4, g + 8, ..., four passes at a time with every load of
-// the four issued before any is used.  Lane j holds elements 8 j .. 8 j + 7
-// of its head (head_dim 128) as one 16-byte load, its rotary partners
-// (elements +-64) sit in lane j ^ 8, and the norm's sum is a butterfly over
-// the row's 16 lanes.  The token's position, cos/sin and the two norm
-// weights are loaded once per wave.
+// Work: a token's rows (units) are the Hq query heads, then the Hkv key
+// heads, then the Hkv value heads, in rounds of eight rows (a key head and its
+// value head together); one wave, a work-group of its own, takes one round of
+// one token: its four 16-lane groups take rows g and g + 4, both loads issued
+// before either is used.  Lane j holds elements 8 j .. 8 j + 7 of its head
+// (head_dim 128) as one 16-byte load, its rotary partners (elements +-64) sit
+// in lane j ^ 8, and the norm's sum is a butterfly over the row's 16 lanes.
+// The token's position, cos/sin and the norm weight are loaded once per wave
+// (from the caches after a token's first).
+// A small step is bound by latency, which a wave per round keeps to one chain
+// (a wave per token walked a 32 / 8-head token's rounds one after the other:
+// 33 tokens 9.9 -> 4.0 us, 100 of 64 / 8 heads over int8 16.6 -> 5.4, 3768 over
+// fp8 24.1 -> 20.6), a long one by HBM, whose stream many short waves keep
+// dense (34 855 tokens 148.7 -> 141 us; in work-groups of four waves with the
+// round found by a division 148, looping over tokens 199).
 #include <algorithm>
 
 #include "nvs_common.h"
@@ -34,9 +41,9 @@ namespace {
 
 constexpr int kPrepD = 128;
 constexpr int kRowLanes = 16;  // lanes per head row, 8 elements each
-constexpr int kPrepThreads = 256;
-constexpr int kPrepTokens = kPrepThreads / 64;  // one wave per token
-constexpr int kPrepUnroll = 4;                  // passes whose loads are issued together
+constexpr int kPrepThreads = 64;  // one wave: a round of a token
+constexpr int kPrepUnroll = 2;    // rows of a lane group in a round, their loads issued together
+constexpr int64_t kPrepGridY = 65535;
 
 struct PrepArgs {
   const uint16_t* q;
@@ -61,6 +68,7 @@ struct PrepArgs {
   int64_t qo_ts, qo_hs;
   uint16_t* ko;  // may be null
   int64_t ko_ts, ko_hs;
+  int q_rounds;  // rounds of a token's q heads
 };
 
 // The 8 values rounded to bf16 in place, two per conversion; `bits` holds
@@ -184,6 +192,14 @@ struct PrepToken {
   uint16_t* ko;      // null: the rotated k is not returned
 };
 
+// Passes of a round of loads.
+template <int KIND>
+constexpr int kPrepPasses = KIND == 0 ? kPrepUnroll : kPrepUnroll / 2;
+template <int KIND>
+__host__ __device__ __forceinline__ int prep_rounds(int H) {
+  return ((H + 3) / 4 + kPrepPasses<KIND> - 1) / kPrepPasses<KIND>;
+}
+
 // The token's q heads (KIND 0) or its k and v heads (KIND 1), four rows a
 // pass (head g + 4 p on lane group g), the loads of kPrepUnroll rows issued
 // before any is used (KIND 1: the k and v rows of kPrepUnroll / 2 passes).
@@ -194,10 +210,10 @@ struct PrepToken {
 template <int KIND, int DST>
 __device__ __forceinline__ void prep_section(const PrepArgs& a, const PrepToken& tk, const uint16_t* src, int hs,
                                              const uint16_t* vsrc, int vhs, int H, const float (&w)[8], int g,
-                                             int j) {
-  constexpr int PER = KIND == 0 ? kPrepUnroll : kPrepUnroll / 2;  // passes per round of loads
-  const int passes = (H + 3) / 4;
-  for (int p0 = 0; p0 < passes; p0 += PER) {
+                                             int j, int round) {
+  constexpr int PER = kPrepPasses<KIND>;
+  const int passes = (H + 3) / 4, p0 = round * PER;
+  {
     u32x4 xw[kPrepUnroll];
 #pragma unroll
     for (int k = 0; k < kPrepUnroll; ++k) {
@@ -264,11 +280,10 @@ __device__ __forceinline__ void prep_section(const PrepArgs& a, const PrepToken&
 
 template <int DST>
 __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
-  // The token is wave-uniform (through readfirstlane, so its pointers are
-  // scalar); a lane adds a 32-bit offset for its head row and elements.
-  const int64_t t = (int64_t)blockIdx.x * kPrepTokens + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (t >= a.T) return;  // whole waves exit together
+  const int round = blockIdx.x;
   const int g = (threadIdx.x >> 4) & 3, j = threadIdx.x & (kRowLanes - 1);
+  const int64_t t = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
+  if (t >= a.T) return;
   PrepToken tk;
   const int64_t slot = a.slots[t];
   tk.ok = slot >= 0 && slot < a.total_slots;
@@ -293,8 +308,11 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
   for (int i = 0; i < 8; ++i) tk.s[i] = first ? -tk.s[i] : tk.s[i];
   tk.qo = a.qo + t * a.qo_ts;
   tk.ko = a.ko ? a.ko + t * a.ko_ts : nullptr;
-  prep_section<0, DST>(a, tk, a.q + t * a.q_ts, (int)a.q_hs, nullptr, 0, a.Hq, qw, g, j);
-  prep_section<1, DST>(a, tk, a.k + t * a.k_ts, (int)a.k_hs, a.v + t * a.v_ts, (int)a.v_hs, a.Hkv, kw, g, j);
+  if (round < a.q_rounds)
+    prep_section<0, DST>(a, tk, a.q + t * a.q_ts, (int)a.q_hs, nullptr, 0, a.Hq, qw, g, j, round);
+  else
+    prep_section<1, DST>(a, tk, a.k + t * a.k_ts, (int)a.k_hs, a.v + t * a.v_ts, (int)a.v_hs, a.Hkv, kw, g, j,
+                         round - a.q_rounds);
 }
 
 bool is_code_dtype(int dt) { return dt == NVS_DTYPE_INT8 || dt == NVS_DTYPE_FP8_E4M3; }
@@ -343,8 +361,7 @@ extern "C" int nvs_qk_norm_rope_store(const void* q, int64_t q_tok_stride, int64
                   k_out_tok_stride >= 0 && k_out_head_stride >= 0,
               NVS_ERR_INVALID, "%s: negative stride", who);
   if (num_tokens == 0) return NVS_OK;
-  const int64_t blocks = (num_tokens + kPrepTokens - 1) / kPrepTokens;
-  NVS_REQUIRE(blocks < (1ll << 31), NVS_ERR_INVALID, "%s: too many tokens (%lld)", who, (long long)num_tokens);
+  const int q_rounds = prep_rounds<0>(num_heads), rounds = q_rounds + prep_rounds<1>(num_kv_heads);
   PrepArgs a;
   a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
   a.q_ts = q_tok_stride; a.q_hs = q_head_stride; a.k_ts = k_tok_stride; a.k_hs = k_head_stride;
@@ -354,11 +371,13 @@ extern "C" int nvs_qk_norm_rope_store(const void* q, int64_t q_tok_stride, int64
   a.cs = cos_sin_cache; a.max_pos = max_position;
   a.slots = slot_mapping; a.total_slots = num_blocks * (int64_t)block_size;
   a.kc = k_cache; a.vc = v_cache; a.ks = k_scale; a.vs = v_scale;
-  a.Hq = num_heads; a.Hkv = num_kv_heads;
+  a.Hq = num_heads; a.Hkv = num_kv_heads; a.q_rounds = q_rounds;
   a.qo = (uint16_t*)q_out; a.qo_ts = q_out_tok_stride; a.qo_hs = q_out_head_stride;
   a.ko = (uint16_t*)k_out; a.ko_ts = k_out_tok_stride; a.ko_hs = k_out_head_stride;
   hipStream_t s = (hipStream_t)stream;
-  dim3 grid((unsigned)blocks), block(kPrepThreads);
+  const int64_t gy = std::min(num_tokens, kPrepGridY), gz = (num_tokens + gy - 1) / gy;
+  NVS_REQUIRE(gz <= kPrepGridY, NVS_ERR_INVALID, "%s: too many tokens (%lld)", who, (long long)num_tokens);
+  dim3 grid((unsigned)rounds, (unsigned)gy, (unsigned)gz), block(kPrepThreads);
   switch (cache_dtype) {
     case NVS_DTYPE_BF16: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_BF16>, grid, block, 0, s, a); break;
     case NVS_DTYPE_FP16: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_FP16>, grid, block, 0, s, a); break;

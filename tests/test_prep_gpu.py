@@ -213,3 +213,30 @@ def test_forward_fused_equals_forward_on_prepared_inputs(device, kv):
     plain = attn.forward(q_rot, k_rot, wl.v, ctx)
     torch.cuda.synchronize()
     assert torch.equal(fused, plain)
+
+
+@pytest.mark.parametrize("Hq,Hkv,kv", [(1, 1, "bf16"), (3, 1, "fp8"), (9, 5, "int8")])
+def test_rounds_past_the_grids_tokens(device, Hq, Hkv, kv):
+    """More tokens than one grid dimension holds (65 535), head counts that
+    leave rounds partly empty: the tokens around the edge equal those of a
+    call on them alone, outputs and cache rows bit for bit."""
+    T, edge = 65535 + 70, slice(65535 - 40, 65535 + 70)
+    NB, bs = (T + 255) // 256 + 1, 256
+    say(f"prep past the grid: Hq={Hq} Hkv={Hkv} cache={kv} T={T}")
+    q, k, v, qw, kw, pos, slots = (x.to(device) for x in _inputs(T, Hq, Hkv, 9, NB, bs))
+    table = torch.randn(MAX_POS, 1, D, generator=torch.Generator().manual_seed(1)).to(device)
+    outs = []
+    for part in (slice(0, T), edge):
+        attn = _layer(Hq, Hkv, kv, NB, bs, device)
+        attn.k_cache.view(torch.uint8).zero_()
+        attn.v_cache.view(torch.uint8).zero_()
+        qo, ko = attn.qk_norm_rope_store(q[part], k[part], v[part], pos[part], qw, kw, 1e-6, table, slots[part],
+                                         want_k=True)
+        torch.cuda.synchronize()
+        at = slots[edge][slots[edge] >= 0].long()
+        rows = [c.view(torch.uint8).reshape(NB * bs, -1)[at] for c in (attn.k_cache, attn.v_cache)]
+        if attn.k_scale_cache is not None:
+            rows += [c.reshape(NB * bs, -1)[at] for c in (attn.k_scale_cache, attn.v_scale_cache)]
+        outs.append([qo[-110:], ko[-110:], *rows])
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
