@@ -170,7 +170,12 @@ __global__ __launch_bounds__(kMxThreads) __attribute__((amdgpu_waves_per_eu(1, 1
   const int xcd = blockIdx.x & 7;
   int* counter = a.plan.hdr->prefill_next + xcd;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (number < 0) {  // streamed decode rows: joins late
+  // Beside decode rows a long list is claimed throughout: the work-groups that
+  // join late should not find the others' units dealt (2048 units beside 128
+  // rows 1744 against 1769 us dealt; 4416 units without decode rows 1125
+  // claimed, 1120 .. 1123 dealt).
+  if (units > kSplitMaxUnits && starters < (int)(gridDim.x >> 3)) starters = 0, number = -1;
+  if (number < 0) {  // or streamed decode rows: joins late
     if (threadIdx.x == 0)
       for (int i = 0; i < 3; ++i) s_claim[i] = 3 * starters + atomicAdd(counter, 1);
   } else if (threadIdx.x < 3) {
