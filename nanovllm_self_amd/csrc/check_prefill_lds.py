@@ -400,7 +400,9 @@ class Sim:
                 self.v[args[0]] = [self.records[idx][k] & M32 if voff[k] < nrec and k < 16 else 0 for k in range(64)]
             elif rs == G.S_RBT:
                 o = voff[0]
-                val = self.mem32.get(base + o, 0) if o + 4 <= nrec else 0
+                if o + 4 <= nrec and base + o not in self.mem32:
+                    self.fail("block id read outside the block table")
+                val = self.mem32[base + o] if o + 4 <= nrec else 0
                 self.v[args[0]] = [val & M32] * 64
             else:
                 raise NotImplementedError(ln)
@@ -413,13 +415,15 @@ class Sim:
         elif op in ("buffer_store_dwordx4", "buffer_store_dword"):
             r0 = self.check_rsrc(args[2])
             self.vmq.append({"pos": self.pos, "done": None, "region": None})
-            if self.s[r0 + 2] == G.PART_WAVE:  # a wave's part of a partial slot
+            base = self.s[r0] | ((self.s[r0 + 1] & 0xFFFF) << 32)
+            if 0 <= base - self.parts_base < self.parts_bytes:  # a wave's part of a partial slot
+                if self.s[r0 + 2] != G.PART_WAVE:
+                    self.fail("partial store: bytes of the slot")
                 size = 16 if op.endswith("x4") else 4
                 off = self.sget(args[3].split()[0]) + self.off(args)
                 voff = self.vget(args[1])
                 if voff != [size * x for x in range(64)]:
                     self.fail("partial store: lane offsets")
-                base = self.s[r0] | ((self.s[r0 + 1] & 0xFFFF) << 32)
                 self.parts.append((base, off, 64 * size))
         elif op == "global_atomic_add":
             self.vmq.append({"pos": self.pos, "done": None, "region": None})
@@ -472,13 +476,13 @@ def plan_records(seqs, pbm, ntq, paged, bs, bt_stride, Tk, cu_k0, rng, pe):
             step = bs // 64 if paged else 1
             starts = [0]
             if rng.random() < 0.5:
-                each = step * rng.randint(1, 4)
+                each = step * rng.randint(1, 6)
                 starts += [t for t in range(each, nt, each) if 64 * t <= p0 + off]
             for t0, t1 in zip(starts, starts[1:] + [nt]):
                 if paged:
                     k0c, kf = 0, K - 64 * t0
                     bto = 4 * (64 * t0 // bs)
-                    btb = 4 * min((K + bs - 1) // bs, bt_stride) - bto
+                    btb = max(0, 4 * min((K + bs - 1) // bs, bt_stride) - bto)
                     bb = tuple(tb(t0 + t) for t in range(3))
                 else:
                     c = min(max(k0, 0), Tk)
@@ -565,6 +569,8 @@ def check_case(rng, paged, slow_p):
         seqs.append((L, K, blks))
     ntq = max((L + pbm - 1) // pbm for L, _, _ in seqs)
     bt_stride = max(len(bl) for _, _, bl in seqs) + rng.randint(0, 3)
+    if rng.random() < 0.25:  # rows of more keys than the table has blocks for
+        bt_stride = rng.randint(1, bt_stride)
     Tk = sum(K for _, K, _ in seqs) - (rng.randint(0, 40) if not paged else 0)
     cu_k0, acc = [], 0
     for _, K, _ in seqs:
@@ -587,7 +593,7 @@ def check_case(rng, paged, slow_p):
     sim.mem32 = {}
     if paged:
         for b, (_, _, blks) in enumerate(seqs):
-            for k, x in enumerate(blks[:bt_stride]):
+            for k, x in enumerate((blks + [NB + 9] * bt_stride)[:bt_stride]):
                 sim.mem32[a["bt"] + b * bt_stride * 4 + 4 * k] = x & M32
     krow = Hkv * 256 if paged else a["k_ts"] * 2
     qrts = a["q_ts"] * 2
@@ -628,6 +634,7 @@ def check_case(rng, paged, slow_p):
     put64(23, a["bt"] if paged else 0)
     vals[25] = 4 * bt_stride if paged else 0
     parts = base()
+    sim.parts_base, sim.parts_bytes = parts, (len(recs) * pe + 1) * G.PART_BYTES
     put64(26, parts + w * G.PART_WAVE)
     for k, x in vals.items():
         bank[k] = x & M32

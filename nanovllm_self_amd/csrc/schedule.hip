@@ -204,7 +204,9 @@ __device__ __forceinline__ PlanRecord make_record(const PlanArgs& a, const RowFi
     rec.k0c = 0;
     rec.kf = r.K - 64 * t0;
     rec.bt_off = (int)(4 * (64 * (uint32_t)t0 / tbs));
-    rec.bt_bytes = (int)(4 * min(((uint32_t)max(r.K, 0) + tbs - 1) / tbs, tst)) - rec.bt_off;
+    // None of a part that starts past the table row (more keys than it has
+    // blocks for): they read as missing.
+    rec.bt_bytes = max(0, (int)(4 * min(((uint32_t)max(r.K, 0) + tbs - 1) / tbs, tst)) - rec.bt_off);
   } else {
     const int64_t k0c = min(max((int64_t)r.k0, (int64_t)0), a.Tk);
     rec.k0c = (int)k0c + 64 * t0;

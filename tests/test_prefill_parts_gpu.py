@@ -14,6 +14,7 @@ from nanovllm_self_amd.kv_cache import SeqSlice
 from nanovllm_self_amd.layers import attention as LA
 from oracle import attn_oracle as AO
 from tests.gpu_util import bf16_to_np, compare, oracle_seq_rows, say
+from tests.test_code_prefill_gpu import _oracle_with_holes
 
 pytestmark = pytest.mark.gpu
 N_SPLIT = 12  # the plan header's word
@@ -110,3 +111,28 @@ def test_parts_in_a_graph(device):
     need = LA._lib.load().nvs_attention_workspace_bytes(2, 30, 16384 + 30, 32, 8, 128, 0)
     assert ws.numel() < need or LA._workspaces[wl.q.device] is ws
     assert np.all(np.isfinite(bf16_to_np(eager)))
+
+
+@pytest.mark.parametrize("kv,bs", [("bf16", 64), ("bf16", 256), ("fp16", 64), ("fp8", 64), ("int8", 256)])
+def test_parts_over_missing_blocks(device, kv, bs):
+    """Parts whose tiles meet blocks that are missing (-1, outside the pool),
+    and rows of more keys than their block-table row has blocks for, whose
+    later parts start past its end: such blocks read as zero keys and values."""
+    spec = [(5120, 40), (4096, 70), (6144, 33)]
+    say(f"parts over missing blocks: {kv} block_size={bs}")
+    wl = _workload(device, spec, 2, 4, bs, kv, 17)
+    width = 2048 // bs  # every row has keys past it
+    bt = wl.context.block_tables[:, :width].contiguous()
+    bt[0, 512 // bs] = -1
+    bt[1, 1024 // bs] = wl.num_blocks + 3
+    wl.context.block_tables = bt
+    wl.context.max_seqlen_k = 2048
+    out = wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    header = LA._workspaces[wl.q.device][:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) > 0, "the batch was not split"
+    got = bf16_to_np(out)
+    for i in range(len(spec)):
+        row = [b if 0 <= b < wl.num_blocks else -1 for b in bt[i].tolist()]
+        ref, rows = _oracle_with_holes(wl, i, row + [-1] * (len(wl.seqs[i].block_table) - width))
+        compare(got[rows], ref, kv in ("int8", "fp8"), f"parts over missing blocks {kv} row {i}")
