@@ -30,6 +30,7 @@ _SERVED_CACHE_DTYPES = (torch.bfloat16, torch.float16, torch.int8, torch.float8_
 _QUANT_DTYPE = {"int8_mock": torch.int8, "fp8_e4m3": torch.float8_e4m3fn}
 
 _workspaces: dict = {}
+_no_room: dict = {}  # device -> bytes with the optional ones that it had no memory for
 _kept_workspaces: set = set()  # devices whose workspace was reserved or is in a captured graph
 
 
@@ -43,7 +44,9 @@ def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) ->
 
     `optional` bytes more are used where they are there: a buffer that lacks
     only them is not replaced once it was reserved or handed to a captured
-    graph.  Calls that share it must be ordered on one stream."""
+    graph, and a device that has no memory for them serves its calls without
+    (and is not asked again for as many until the next reserve call).  Calls
+    that share it must be ordered on one stream."""
     if nbytes <= 0:
         return None
     key = torch.device(device)
@@ -58,10 +61,23 @@ def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) ->
                     "reserve_attention_workspace(...) before capturing"
                 )
         elif have < nbytes or key not in _kept_workspaces:
-            buf = torch.empty(nbytes + optional, dtype=torch.uint8, device=key)
-            _workspaces[key] = buf
+            buf = _grow_workspace(key, buf, have, nbytes, optional)
     elif key not in _kept_workspaces and torch.cuda.is_current_stream_capturing():
         _kept_workspaces.add(key)
+    return buf
+
+
+def _grow_workspace(key, buf, have, nbytes, optional):
+    """A buffer of nbytes + optional, or, where there is no memory for the
+    optional bytes, the present one if it holds nbytes, else one of nbytes."""
+    if optional > 0 and nbytes + optional < _no_room.get(key, nbytes + optional + 1):
+        try:
+            _workspaces[key] = torch.empty(nbytes + optional, dtype=torch.uint8, device=key)
+            return _workspaces[key]
+        except torch.cuda.OutOfMemoryError:
+            _no_room[key] = nbytes + optional
+    if have < nbytes:
+        buf = _workspaces[key] = torch.empty(nbytes, dtype=torch.uint8, device=key)
     return buf
 
 
@@ -75,6 +91,7 @@ def reserve_attention_workspace(num_seqs: int, max_seqlen_q: int, max_seqlen_k: 
     n = lib.nvs_attention_workspace_bytes(num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, 128, 0)
     extra = lib.nvs_attention_split_bytes(num_seqs, 0, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads)
     if n > 0:
+        _no_room.pop(torch.device(device), None)
         attention_workspace(torch.device(device), int(n), int(extra))
         _kept_workspaces.add(torch.device(device))
 

@@ -1,0 +1,60 @@
+"""The per-device attention workspace: what is allocated, kept and given up,
+with the allocator stubbed (no GPU)."""
+import pytest
+import torch
+
+from nanovllm_self_amd.layers import attention as LA
+
+CPU = torch.device("cpu")
+
+
+class _Memory:
+    """torch.empty with at most `room` bytes a tensor; keeps the sizes asked for."""
+
+    def __init__(self, room):
+        self.room, self.asked, self.empty = room, [], torch.empty
+
+    def __call__(self, n, dtype, device):
+        self.asked.append(n)
+        if n > self.room:
+            raise torch.cuda.OutOfMemoryError("stub")
+        return self.empty(n, dtype=dtype, device=device)
+
+
+@pytest.fixture
+def memory(monkeypatch):
+    for name in ("_workspaces", "_no_room"):
+        monkeypatch.setattr(LA, name, {}, raising=False)
+    monkeypatch.setattr(LA, "_kept_workspaces", set())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    mem = _Memory(1 << 20)
+    monkeypatch.setattr(torch, "empty", mem)
+    return mem
+
+
+def test_no_memory_for_the_optional_bytes(memory):
+    """The call is served without them, by the buffer that is there or by one
+    of the bytes it cannot do without; as many are not asked for again."""
+    assert LA.attention_workspace(CPU, 1000, 1 << 20).numel() == 1000
+    assert memory.asked == [1000 + (1 << 20), 1000]
+    there = LA.attention_workspace(CPU, 1000)
+    assert LA.attention_workspace(CPU, 900, 2 << 20) is there
+    assert LA.attention_workspace(CPU, 1000, 1 << 20) is there
+    assert len(memory.asked) == 2
+    assert LA.attention_workspace(CPU, 1000, 500).numel() == 1500  # fewer: asked for, and there
+    assert LA.attention_workspace(CPU, 3000, 1 << 20).numel() == 3000
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        LA.attention_workspace(CPU, 2 << 20)
+    assert LA.attention_workspace(CPU, 3000).numel() == 3000
+
+
+def test_reserve_asks_for_the_optional_bytes_again(memory):
+    memory.room = 16 << 20
+    args = (6, 300, 16384, 32, CPU, 8)
+    LA.reserve_attention_workspace(*args)
+    without = LA._workspaces[CPU].numel()
+    assert memory.asked[0] > memory.room and memory.asked[1:] == [without]
+    memory.room = 1 << 30
+    LA._kept_workspaces.clear()
+    LA.reserve_attention_workspace(*args)
+    assert LA._workspaces[CPU].numel() == memory.asked[0]
