@@ -31,7 +31,7 @@ _QUANT_DTYPE = {"int8_mock": torch.int8, "fp8_e4m3": torch.float8_e4m3fn}
 
 _workspaces: dict = {}
 _no_room: dict = {}  # device -> bytes with the optional ones that it had no memory for
-_kept_workspaces: set = set()  # devices whose workspace was reserved or is in a captured graph
+_captured_workspaces: dict = {}  # device -> buffers that captured graphs use
 
 
 def _need_device(t: torch.Tensor, what: str) -> None:
@@ -42,28 +42,28 @@ def _need_device(t: torch.Tensor, what: str) -> None:
 def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) -> torch.Tensor | None:
     """Per-device split-K workspace, grown on demand (never inside graph capture).
 
-    `optional` bytes more are used where they are there: a buffer that lacks
-    only them is not replaced once it was reserved or handed to a captured
-    graph, and a device that has no memory for them serves its calls without
-    (and is not asked again for as many until the next reserve call).  Calls
-    that share it must be ordered on one stream."""
+    `optional` bytes more are used where they are there: a captured call takes
+    the buffer as it is, and a device that has no memory for them serves its
+    calls without (and is not asked again for as many until the next reserve
+    call).  A buffer that a captured graph holds the address of is kept for
+    good, beside the larger one that later calls may need.  Calls that share
+    it must be ordered on one stream."""
     if nbytes <= 0:
         return None
     key = torch.device(device)
     buf = _workspaces.get(key)
     have = buf.numel() if buf is not None else 0
-    if optional > 0 and have < nbytes + optional or have < nbytes:
-        if torch.cuda.is_current_stream_capturing():
-            _kept_workspaces.add(key)
-            if have < nbytes:
-                raise RuntimeError(
-                    "decode workspace too small inside graph capture; call "
-                    "reserve_attention_workspace(...) before capturing"
-                )
-        elif have < nbytes or key not in _kept_workspaces:
-            buf = _grow_workspace(key, buf, have, nbytes, optional)
-    elif key not in _kept_workspaces and torch.cuda.is_current_stream_capturing():
-        _kept_workspaces.add(key)
+    if torch.cuda.is_current_stream_capturing():
+        if have < nbytes:
+            raise RuntimeError(
+                "decode workspace too small inside graph capture; call "
+                "reserve_attention_workspace(...) before capturing"
+            )
+        held = _captured_workspaces.setdefault(key, [])
+        if not any(b is buf for b in held):
+            held.append(buf)
+    elif have < nbytes + optional:
+        buf = _grow_workspace(key, buf, have, nbytes, optional)
     return buf
 
 
@@ -93,7 +93,6 @@ def reserve_attention_workspace(num_seqs: int, max_seqlen_q: int, max_seqlen_k: 
     if n > 0:
         _no_room.pop(torch.device(device), None)
         attention_workspace(torch.device(device), int(n), int(extra))
-        _kept_workspaces.add(torch.device(device))
 
 
 def _quantize(x: torch.Tensor, code_dtype: torch.dtype):

@@ -136,3 +136,33 @@ def test_parts_over_missing_blocks(device, kv, bs):
         row = [b if 0 <= b < wl.num_blocks else -1 for b in bt[i].tolist()]
         ref, rows = _oracle_with_holes(wl, i, row + [-1] * (len(wl.seqs[i].block_table) - width))
         compare(got[rows], ref, kv in ("int8", "fp8"), f"parts over missing blocks {kv} row {i}")
+
+
+def test_parts_after_a_captured_decode(device, monkeypatch):
+    """Follow-up turns after decode was captured in a graph (its workspace
+    reserved for decode alone) are split all the same, and the graph replays
+    over its own workspace."""
+    for name in ("_workspaces", "_captured_workspaces"):
+        monkeypatch.setattr(LA, name, {}, raising=False)
+    say("parts after a captured decode")
+    dec = _workload(device, [(3000 + 11 * i, 1) for i in range(40)], 8, 4, 256, "bf16", 21)
+    LA.reserve_attention_workspace(40, 1, int(dec.context.max_seqlen_k), 32, device, 8)
+    args = (dec.q, dec.k, dec.v, dec.context)
+    dec.attn.forward(*args)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = dec.attn.forward(*args)
+    spec = [(4096, 40), (2048, 70), (8192, 30)]
+    turn = _workload(device, spec, 8, 4, 256, "bf16", 22)
+    for step in range(3):
+        got = turn.attn.forward(turn.q, turn.k, turn.v, turn.context)
+        torch.cuda.synchronize()
+        header = LA._workspaces[turn.q.device][:256].view(torch.int32).cpu()
+        assert int(header[N_SPLIT]) > 0, "the batch was not split"
+        if step == 0:
+            _check(turn, bf16_to_np(got), spec, False, "turn after a captured decode")
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = out.clone()
+        assert torch.equal(replayed, dec.attn.forward(*args)), f"replay {step} differs"

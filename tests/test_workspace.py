@@ -1,5 +1,7 @@
 """The per-device attention workspace: what is allocated, kept and given up,
 with the allocator stubbed (no GPU)."""
+import weakref
+
 import pytest
 import torch
 
@@ -23,9 +25,8 @@ class _Memory:
 
 @pytest.fixture
 def memory(monkeypatch):
-    for name in ("_workspaces", "_no_room"):
+    for name in ("_workspaces", "_no_room", "_captured_workspaces"):
         monkeypatch.setattr(LA, name, {}, raising=False)
-    monkeypatch.setattr(LA, "_kept_workspaces", set())
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     mem = _Memory(1 << 20)
     monkeypatch.setattr(torch, "empty", mem)
@@ -55,6 +56,36 @@ def test_reserve_asks_for_the_optional_bytes_again(memory):
     without = LA._workspaces[CPU].numel()
     assert memory.asked[0] > memory.room and memory.asked[1:] == [without]
     memory.room = 1 << 30
-    LA._kept_workspaces.clear()
     LA.reserve_attention_workspace(*args)
     assert LA._workspaces[CPU].numel() == memory.asked[0]
+
+
+def test_captured_buffers_stay_and_eager_calls_grow(memory, monkeypatch):
+    """A buffer that a captured call used outlives its replacement; calls
+    outside a capture get the optional bytes whatever was captured before."""
+    LA.attention_workspace(CPU, 1000)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    first = LA.attention_workspace(CPU, 800, 500)  # as it is, without the optional bytes
+    assert first.numel() == 1000
+    with pytest.raises(RuntimeError, match="too small inside graph capture"):
+        LA.attention_workspace(CPU, 1001)
+    assert LA.attention_workspace(CPU, 900) is first
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ref, address = weakref.ref(first), first.data_ptr()
+    del first
+    grown = LA.attention_workspace(CPU, 800, 500)
+    assert grown.numel() == 1300
+    assert ref() is not None and ref().data_ptr() == address
+    last = LA.attention_workspace(CPU, 2000)  # the grown one, captured by nobody, is given up
+    gone = weakref.ref(grown)
+    del grown
+    assert gone() is None and last.numel() == 2000
+
+
+def test_reserved_buffer_grows_for_the_optional_bytes(memory):
+    """A reservation for decode alone asks for no optional bytes; a prefill
+    call after it gets them."""
+    memory.room = 1 << 30
+    LA.reserve_attention_workspace(64, 1, 8192, 32, CPU, 8)
+    reserved = LA._workspaces[CPU].numel()
+    assert LA.attention_workspace(CPU, reserved, 4096).numel() == reserved + 4096
