@@ -72,12 +72,19 @@ def _grow_workspace(key, buf, have, nbytes, optional):
     optional bytes, the present one if it holds nbytes, else one of nbytes."""
     if optional > 0 and nbytes + optional < _no_room.get(key, nbytes + optional + 1):
         try:
-            _workspaces[key] = torch.empty(nbytes + optional, dtype=torch.uint8, device=key)
-            return _workspaces[key]
+            return _replace_workspace(key, buf, nbytes + optional)
         except torch.cuda.OutOfMemoryError:
             _no_room[key] = nbytes + optional
-    if have < nbytes:
-        buf = _workspaces[key] = torch.empty(nbytes, dtype=torch.uint8, device=key)
+    return buf if have >= nbytes else _replace_workspace(key, buf, nbytes)
+
+
+def _replace_workspace(key, old, nbytes):
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=key)
+    if old is not None and old.is_cuda:
+        # Calls still running may be on another stream than the one it was
+        # allocated on; the calling stream is ordered after all of them.
+        old.record_stream(torch.cuda.current_stream(key))
+    _workspaces[key] = buf
     return buf
 
 

@@ -635,3 +635,23 @@ def test_decode_store_shared_block_takes_store_path(device, monkeypatch):
     monkeypatch.setattr(lib, "nvs_store_kvcache", lambda *args: (calls.append(1), inner(*args))[1])
     _fused_vs_plain(a, b)
     assert len(calls) == 2, "the layer must run the store kernel (and b's write_kv_cache one more)"
+
+
+def test_replaced_workspace_waits_for_its_stream(device, monkeypatch):
+    """A workspace allocated on one stream, used on another and replaced there
+    while that stream is still busy is not handed out again before it is done."""
+    from nanovllm_self_amd.layers import attention as LA
+    for name in ("_workspaces", "_captured_workspaces"):
+        monkeypatch.setattr(LA, name, {})
+    say("a workspace replaced on a busy stream")
+    n = 3 << 20
+    old = LA.attention_workspace(device, n).data_ptr()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)  # about 0.1 s of a running call
+        LA.attention_workspace(device, 2 * n)
+    again = [torch.empty(n, dtype=torch.uint8, device=device) for _ in range(2)]
+    assert not side.query(), "the stream was not busy"
+    assert old not in [x.data_ptr() for x in again]
+    torch.cuda.synchronize()
