@@ -217,7 +217,8 @@ int64_t nvs_attention_workspace_bytes_cache(int num_seqs, int max_seqlen_q,
  * query tiles for the chip (a short new turn over a long cached prefix): the
  * parts' fp32 accumulators, at most 768 slots of 132 KiB.  0 where no split
  * can help.  Optional: a smaller workspace serves the call unsplit.
- * num_tokens <= 0: unknown (an upper bound); num_kv_heads <= 0: unknown.
+ * num_tokens <= 0: unknown (an upper bound for every batch of up to these
+ * sizes); num_kv_heads <= 0: unknown.
  */
 int64_t nvs_attention_split_bytes(int num_seqs, int64_t num_tokens,
                                   int max_seqlen_q, int max_seqlen_k,

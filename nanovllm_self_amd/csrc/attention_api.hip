@@ -126,12 +126,13 @@ static bool may_split(int num_seqs, int64_t num_tokens, int units, int pbm) {
 static SplitJob split_job(const AttnParams& P, const Plan& plan, int64_t offset, int wgs) {
   SplitJob job = {};
   const int units = prefill_mx_units(P.Hq, P.Hkv);
-  const int64_t slots = split_slots(P.B, plan.ntq, P.max_seqlen_k, units);
+  const int64_t entries = (int64_t)P.B * plan.ntq;
+  const int64_t slots = split_slots(entries, split_row_tiles(P.max_seqlen_k), units);
   offset = align256(offset);
   if (slots <= 0 || !may_split(P.B, P.T, units, plan.pbm) ||
-      P.ws_bytes < offset + split_bytes(P.B, plan.ntq, slots))
+      P.ws_bytes < offset + split_bytes(entries, slots))
     return job;
-  job.at = split_at((char*)P.ws + offset, P.B, plan.ntq);
+  job.at = split_at((char*)P.ws + offset, entries);
   job.slots = (int)slots;
   job.wgs = wgs;
   return job;
@@ -208,9 +209,13 @@ extern "C" int64_t nvs_attention_split_bytes(int num_seqs, int64_t num_tokens, i
   const int units = known ? prefill_mx_units(num_heads, num_kv_heads) : num_heads;
   const int pbm = known ? prefill_mx_positions(num_heads / num_kv_heads) : prefill_mx_positions(8);
   if (num_tokens > 0 && !may_split(num_seqs, num_tokens, units, pbm)) return 0;
-  const int ntq = prefill_tiles(max_seqlen_q, pbm);
-  const int64_t slots = split_slots(num_seqs, ntq, max_seqlen_k, units);
-  return slots > 0 ? 256 + split_bytes(num_seqs, ntq, slots) : 0;
+  int64_t entries = (int64_t)num_seqs * prefill_tiles(max_seqlen_q, pbm), tiles = split_row_tiles(max_seqlen_k);
+  if (num_tokens <= 0) {  // the bound covers the smaller batches, which may be split where the largest is not
+    entries = std::min(entries, kSplitMaxList);
+    tiles = std::min(tiles, kSplitMaxRowTiles);
+  }
+  const int64_t slots = split_slots(entries, tiles, units);
+  return slots > 0 ? 256 + split_bytes(entries, slots) : 0;
 }
 
 static int check_workspace(const AttnParams& P, const char* who) {

@@ -159,23 +159,25 @@ struct SplitLayout {
   char* slots;      // [kSplitSlots] of kPartBytes
 };
 
-// Slots a batch can use: none where no row can hold two parts.
-inline int64_t split_slots(int B, int ntq, int max_seqlen_k, int units_per_entry) {
-  const int64_t tiles = ((int64_t)max_seqlen_k + 63) / 64;
-  if (tiles < 2 * kSplitMinTiles || tiles > (1 << 20) || (int64_t)B * ntq > (1 << 16)) return 0;
-  const int64_t most = (int64_t)B * ntq * units_per_entry * (tiles / kSplitMinTiles);
+// Slots a batch of up to `entries` list entries can use: none where no row can
+// hold two parts, or past the sizes the plan's arithmetic is made for.
+constexpr int64_t kSplitMaxList = 1 << 16, kSplitMaxRowTiles = 1 << 20;
+inline int64_t split_row_tiles(int max_seqlen_k) { return ((int64_t)max_seqlen_k + 63) / 64; }
+inline int64_t split_slots(int64_t entries, int64_t tiles, int units_per_entry) {
+  if (tiles < 2 * kSplitMinTiles || tiles > kSplitMaxRowTiles || entries > kSplitMaxList) return 0;
+  const int64_t most = entries * units_per_entry * (tiles / kSplitMinTiles);
   return most < kSplitSlots ? most : kSplitSlots;
 }
-inline int64_t split_bytes(int B, int ntq, int64_t slots) {
+inline int64_t split_bytes(int64_t entries, int64_t slots) {
   if (slots <= 0) return 0;
-  return align256(((int64_t)B * ntq + kSplitSlots) * (int64_t)sizeof(PlanRecord)) +
+  return align256((entries + kSplitSlots) * (int64_t)sizeof(PlanRecord)) +
          align256(kSplitMaxEntries * (int64_t)sizeof(SplitRow)) + slots * kPartBytes;
 }
-inline SplitLayout split_at(void* p, int B, int ntq) {
+inline SplitLayout split_at(void* p, int64_t entries) {
   SplitLayout s;
   char* c = (char*)p;
   s.rec = (PlanRecord*)c;
-  c += align256(((int64_t)B * ntq + kSplitSlots) * (int64_t)sizeof(PlanRecord));
+  c += align256((entries + kSplitSlots) * (int64_t)sizeof(PlanRecord));
   s.rows = (SplitRow*)c;
   s.slots = c + align256(kSplitMaxEntries * (int64_t)sizeof(SplitRow));
   return s;

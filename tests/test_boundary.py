@@ -324,3 +324,22 @@ def test_workspace_unknown_kv_heads_is_upper_bound():
             for Hkv in (h for h in (1, 2, 4, 8, 16, 32, 64) if Hq % h == 0 and Hq // h <= 16):
                 need = lib.nvs_attention_workspace_bytes(B, max_q, max_k, Hq, Hkv, 128, 256)
                 assert bound >= need, (B, max_q, max_k, Hq, Hkv, bound, need)
+
+
+def test_split_bytes_unknown_tokens_is_upper_bound():
+    """Without a token count nvs_attention_split_bytes is a bound for every
+    batch of up to these sizes, also where the largest itself is never split."""
+    split = _lib.load().nvs_attention_split_bytes
+    for B, max_q, max_k in ((6, 300, 16384), (16, 4096, 20000), (256, 32768, 32768), (300, 65536, 131072),
+                            (4, 64, 80_000_000)):
+        for Hq, Hkv in ((16, 8), (32, 8), (64, 8), (8, 1), (32, 0)):
+            bound = split(B, 0, max_q, max_k, Hq, Hkv)
+            for b, q, k in ((B, max_q, max_k), (1, max_q, max_k), (B, 300, max_k), (min(B, 6), 300, 16384), (1, 64, 1024)):
+                if q > max_q or k > max_k:
+                    continue
+                for tokens in (0, b + 1, b * q // 2, b * q):
+                    for hk in (Hkv,) if Hkv else (1, 2, 4, 8):
+                        g = Hq // hk
+                        if g <= 16:
+                            need = split(b, tokens, q, k, Hq, hk)
+                            assert bound >= need, (B, max_q, max_k, b, tokens, q, k, Hq, hk, bound, need)
