@@ -122,7 +122,8 @@ static bool may_split(int num_seqs, int64_t num_tokens, int units, int pbm) {
 
 // Entries of a call served by the tile-loop kernel split along their keys,
 // if the workspace holds their slots after `offset` bytes; job->slots = 0 if
-// not.
+// not.  wgs: the launch's work-groups, or 0 for a launch of prefill rows alone,
+// which takes one for each unit that there can be with the parts.
 static SplitJob split_job(const AttnParams& P, const Plan& plan, int64_t offset, int wgs) {
   SplitJob job = {};
   const int units = prefill_mx_units(P.Hq, P.Hkv);
@@ -134,7 +135,7 @@ static SplitJob split_job(const AttnParams& P, const Plan& plan, int64_t offset,
     return job;
   job.at = split_at((char*)P.ws + offset, entries);
   job.slots = (int)slots;
-  job.wgs = wgs;
+  job.wgs = wgs > 0 ? wgs : prefill_mx_wgs(entries * units + slots);
   return job;
 }
 
@@ -493,7 +494,7 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
     return rc != NVS_OK ? rc : launch_prefill(P, plan, s);
   }
   const SplitJob split = split_job(P, plan, attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv),
-                                   prefill_mx_wgs(P, plan));
+                                   /*wgs=*/0);
   const SplitJob* sp = split.slots > 0 ? &split : nullptr;
   rc = launch_plan(P, plan, /*paged=*/false, s, nullptr, nullptr, nullptr, sp, store);
   if (rc != NVS_OK) return rc;

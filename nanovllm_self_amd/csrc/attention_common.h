@@ -366,7 +366,7 @@ int launch_prefill(const AttnParams& P, const Plan& plan, hipStream_t stream);
 bool prefill_mx_serves(const AttnParams& P);
 int prefill_mx_positions(int g);
 int prefill_mx_units(int Hq, int Hkv);  // units of a list entry
-int prefill_mx_wgs(const AttnParams& P, const Plan& plan);  // work-groups of a launch without decode rows
+int prefill_mx_wgs(int64_t units);  // work-groups of a launch without decode rows, for up to so many units
 // With `co`, the launch's first work-groups stream the call's decode rows
 // before they join the prefill (co->kv: the cache type of the decode rows,
 // which a code cache's prefill reads through its bf16 copy); the plan has

@@ -109,9 +109,8 @@ int prefill_mx_units(int Hq, int Hkv) {
   const int g = Hq / Hkv, hpi = mx_heads_per_item(g);
   return Hkv * ((g + hpi - 1) / hpi);
 }
-int prefill_mx_wgs(const AttnParams& P, const Plan& plan) {
-  const int64_t upper = (((int64_t)P.B * plan.ntq * prefill_mx_units(P.Hq, P.Hkv) + 7) / 8) * 8;
-  return (int)std::max<int64_t>(8, std::min<int64_t>(upper, (int64_t)device_slots(1)) & ~(int64_t)7);
+int prefill_mx_wgs(int64_t units) {
+  return (int)std::max<int64_t>(8, std::min<int64_t>((units + 7) & ~(int64_t)7, device_slots(1)) & ~(int64_t)7);
 }
 
 __device__ __forceinline__ int mx_swz(int key) { return ((key & 3) << 2) | ((key >> 2) & 3); }
@@ -358,7 +357,9 @@ int launch_prefill_mx(const AttnParams& P, const Plan& plan, hipStream_t stream,
     return NVS_ERR_INVALID;
   }
   // The plan sized the decode part, or the entries' parts, for as many.
-  const int64_t wgs = co ? co->wgs : split ? split->wgs : prefill_mx_wgs(P, plan);
+  const int64_t wgs = co      ? co->wgs
+                      : split ? split->wgs
+                              : prefill_mx_wgs((int64_t)P.B * plan.ntq * prefill_mx_units(P.Hq, P.Hkv));
   a.parts = split ? split->at.slots : nullptr;
   const PlanRecord* rec = split ? split->at.rec : plan.rec;
   const bool f16 = P.cache_dtype == NVS_DTYPE_FP16;
