@@ -396,7 +396,7 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     if (parts == 1) each = nt;
     ent.each[tid] = each;
     ent.parts[tid] = parts;
-    atomicMax(&ent.longest, each);
+    atomicMax(&ent.longest, max(each, nt - (parts - 1) * each));
     int slot = -1;
     if (parts > 1) {
       slot = atomicAdd(&ent.slots, parts) * a.units;
@@ -405,13 +405,18 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     ent.sees[tid] = slot;
   }
   __syncthreads();
-  // Places by part size, longest first, to a 64th of the longest.  Which of
-  // two entries of one bucket comes first, and the slots they take, change
-  // with the run; their outputs do not.
-  int bk = 0;
+  // Places by size, longest first, to a 64th of the longest; an entry's last
+  // part by its own size, as the cost has it.  Which of two parts of one bucket
+  // comes first, and the slots they take, change with the run; their outputs
+  // do not.
+  int bk = 0, bk_last = 0;
+  const int last = nt - (parts - 1) * each;
   if (tid < tot) {
-    bk = min(kPartBuckets - 1, (int)((float)(ent.longest - each) * ((float)kPartBuckets / (float)(ent.longest + 1))));
-    atomicAdd(&ent.bucket[bk], parts);
+    const float scale = (float)kPartBuckets / (float)(ent.longest + 1);
+    bk = min(kPartBuckets - 1, (int)((float)(ent.longest - each) * scale));
+    bk_last = min(kPartBuckets - 1, (int)((float)(ent.longest - last) * scale));
+    if (parts > 1) atomicAdd(&ent.bucket[bk], parts - 1);
+    atomicAdd(&ent.bucket[bk_last], 1);
   }
   __syncthreads();
   if (tid < kPartBuckets) {
@@ -424,9 +429,12 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
   }
   __syncthreads();
   if (tid < tot) {
-    const int at = atomicAdd(&ent.bucket[bk], parts);
+    if (parts > 1) {
+      const int at = atomicAdd(&ent.bucket[bk], parts - 1);
 #pragma unroll 1
-    for (int c = 0; c < parts; ++c) ent.place[at + c] = tid << 10 | c;
+      for (int c = 0; c < parts - 1; ++c) ent.place[at + c] = tid << 10 | c;
+    }
+    ent.place[atomicAdd(&ent.bucket[bk_last], 1)] = tid << 10 | (parts - 1);
   }
   __syncthreads();
   const int list = ent.list;

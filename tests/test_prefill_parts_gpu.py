@@ -166,3 +166,26 @@ def test_parts_after_a_captured_decode(device, monkeypatch):
         torch.cuda.synchronize()
         replayed = out.clone()
         assert torch.equal(replayed, dec.attn.forward(*args)), f"replay {step} differs"
+
+
+@pytest.mark.parametrize("spec,bs", [([(3072, 40 + i) for i in range(4)], 256), ([(4160, 70), (2752, 9)], 64)])
+def test_list_is_longest_first(device, spec, bs):
+    """The list's records run from the longest part to the shortest, to a
+    bucket of the plan's sort: each entry's short last part comes after the
+    others' whole ones."""
+    say(f"order of the parts {spec} block_size={bs}")
+    wl = _workload(device, spec, 8, 4, bs, "bf16", 6)
+    wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    ws = LA._workspaces[wl.q.device]
+    header = ws[:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) == len(spec) + sum(n > 64 for _, n in spec), "not every entry was split"
+    at = LA._lib.load().nvs_attention_workspace_bytes(
+        len(spec), max(n for _, n in spec), max(p + n for p, n in spec), 32, 8, 128, 0)
+    at = (at + 255) // 256 * 256
+    rec = ws[at:at + 64 * int(header[8])].view(torch.int32).cpu().reshape(-1, 16)
+    tiles = rec[:, 9].tolist()
+    assert sum(tiles) == sum((p + min(n, 64 * (t + 1)) + 63) // 64 for p, n in spec for t in range((n + 63) // 64))
+    slack = max(tiles) // 16 + 1
+    assert all(a + slack > b for a, b in zip(tiles, tiles[1:])), tiles
+    assert max(tiles) - min(tiles) > slack  # else every order would do
