@@ -269,52 +269,114 @@ struct PlanRows {
 // (then the first slot, -1: none), tiles of a part and parts; what the
 // buckets of part sizes hold, then their next place in the list; the list's
 // places (entry << 10 | part).
-constexpr int kPartBuckets = 64;
+constexpr int kPartBuckets = 16;
 struct PlanEntries {
   int row[kSplitMaxEntries], nt[kSplitMaxEntries], sees[kSplitMaxEntries];
   int each[kSplitMaxEntries], parts[kSplitMaxEntries];
   int place[kSplitMaxEntries + kSplitSlots];
   float cost[kPartChoices];
+  int tiles[kPlanWaves], deepest[kPlanWaves];  // of the waves' entries
+  float load[kPlanWaves];
   int bucket[kPartBuckets];
   int longest, list, slots, rows;
 };
 
-// Estimated time of the call's prefill with parts of at most C tiles, in key
-// tiles of one work-group (1.2 us, 1.6 with the whole chip busy), by one wave
+// Estimated times of the call's prefill, in key tiles of a work-group that runs
+// alone (1.06 us).  Two things bound it: the most tiles that one work-group
+// gets, each unit with kPartSetup tiles' worth of set-up and output, and what
+// the chip gets through, all the units' tiles at kPartBusy times an even
+// share (256 work-groups at once take 1.6 us a tile; half as many, 1.1).
+// Where the two are near each other each slows the other down (part_time).  A
+// part's slot is written and read once (132 KiB each way): kPartMerge.
+//
+// Fitted to 312 batches (8/1, 16/8, 32/8 and 64/8 heads, 1 .. 32 rows of 4 ..
+// 4000 tokens over 0 .. 16 K cached ones) with every choice of parts timed:
+// the mean error is 4 %.  Before, a tile cost the same however many
+// work-groups ran, and 123 of those batches were slower in their parts, or
+// sorted, than row by row (32 turns of 200 tokens over 3 K, 32/8 heads: 441
+// us, 362 row by row; 12 of 40 over 1.5 K: 64.7, 46.4).
+constexpr float kPartSetup = 5.2f;
+constexpr float kPartBusy = 1.54f;
+constexpr float kPartMerge = 0.036f;
+constexpr float kPartLaunch = 1.2f;
+__device__ __forceinline__ float part_time(float most, float chip) {
+  const float hi = fmaxf(most, chip), lo = fminf(most, chip);
+  return hi + 0.26f * lo * lo * lo * __builtin_amdgcn_rcpf(hi * hi);
+}
+
+// The choices are weighed (2.5 us more of the plan) where parts or another
+// order could bring a batch's time in row order down by more than kPartEarly
+// and a fiftieth of it, and the best of them is taken where it is kPartWorth
+// below the row order.
+constexpr float kPartEarly = 8.0f;
+constexpr float kPartWorth = 1.0f;
+
+// The estimate for whole entries in row order, what no choice gets below, and
+// (chip) the time of all tiles at the chip's rate; every thread calls it, after
+// a barrier that follows the entries' writes.  The first three rounds of units
+// are dealt by number (unit 8 k + x to work-group k of XCD x, back and forth);
+// past them, the even share and half of the deepest entry of the last round.
+__device__ __forceinline__ float row_order_cost(const PlanArgs& a, PlanEntries& ent, int entries, int wgs,
+                                                float& least, float& chip) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int units = entries * a.units, most = wgs >> 3;  // at most 128 work-groups of an XCD
+  const int j = lane & (kPlanWaves - 1);
+  const int of_wave = ent.tiles[j];
+  const int longest = wave_most(ent.deepest[j]);
+  const float tiles = (float)wave_total(lane < kPlanWaves ? of_wave : 0) * a.units;
+  const float each = __builtin_amdgcn_rcpf((float)wgs);
+  const float share = (tiles + kPartSetup * units) * each;
+  chip = kPartBusy * tiles * each;
+  float load = (float)longest + kPartSetup;
+  if (units > 8 * most) {
+    float mine = 0.0f;
+    if (tid < 8 * most) {
+      const int x = tid & 7, k = tid >> 3;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int unit = 8 * (i * most + (i == 1 ? most - 1 - k : k)) + x;
+        if (unit < units) mine += (float)ent.nt[ceil_div(unit + 1, a.units) - 1] + kPartSetup;
+      }
+    }
+    // Past three rounds: entries from `last` on are the last round's.
+    const int last = units > 24 * most ? entries - ceil_div(wgs, a.units) : entries;
+    if (tid >= last && tid < entries) mine = fmaxf(mine, share + 0.5f * ((float)ent.nt[tid] + kPartSetup));
+    mine = wave_most(mine);
+    if (lane == 0) ent.load[w] = mine;
+    __syncthreads();
+    load = wave_most(ent.load[j]);
+  }
+  least = part_time(fmaxf(share, (float)min(longest, kSplitMinTiles) + kPartSetup), chip);
+  return part_time(load, chip);
+}
+
+// The estimate for parts of at most C tiles, dealt longest first, by one wave
 // over all entries; infinite where the parts need more slots than there are.
-// Each unit has kPartSetup tiles' worth of set-up and output.  The units of
-// an XCD are dealt to its work-groups longest first, back and forth, three
-// rounds of them (prefill_mx_kernel's first claims): the most a work-group
-// gets is the estimate; past three rounds, the even share and some of the
-// longest.  A part's slot is written and read once (132 KiB each way):
-// kPartMerge.
-constexpr float kPartSetup = 7.0f;
+// Up to three rounds of units the deal is followed; past them, the even share
+// and some of the longest.
 constexpr float kPartUneven = 0.3f;
-constexpr float kPartMerge = 0.0125f;
-constexpr float kPartLaunch = 1.0f;
 __device__ __forceinline__ float part_cost(const PlanArgs& a, const PlanEntries& ent, int* hist, int entries, int C,
-                                           int step, int wgs, int lane) {
-  int units = 0, slots = 0, longest = 0, tiles = 0;
+                                           int step, int wgs, float chip, int lane) {
+  int units = 0, slots = 0, longest = 0;
 #pragma unroll 1
   for (int e = lane; e < entries; e += 64) {
     int parts;
     const int nt = ent.nt[e], each = part_tiles(nt, ent.sees[e], C, step, parts);
     units += parts;
     if (parts > 1) slots += parts;
-    tiles += nt;
     longest = max(longest, parts > 1 ? max(each, nt - (parts - 1) * each) : nt);
   }
   const int pieces = wave_total(units);
   units = pieces * a.units;
   slots = wave_total(slots) * a.units;
-  tiles = wave_total(tiles);
   longest = wave_most(longest);
   if (slots > a.split_slots) return INFINITY;
   const float merge = slots > 0 ? kPartLaunch + kPartMerge * slots : 0.0f;
   const int most = wgs >> 3;  // work-groups of an XCD
   if (units > 24 * most) {
     const float one = (float)longest + kPartSetup;
-    return merge + fmaxf(one, ((float)tiles * a.units + kPartSetup * units) / (float)wgs + kPartUneven * one);
+    const float share = chip * (1.0f / kPartBusy) + kPartSetup * units * __builtin_amdgcn_rcpf((float)wgs);
+    return merge + part_time(fmaxf(one, share + kPartUneven * one), chip);
   }
   // Pieces by size, longest first: 64 buckets, then how many there are up to
   // each (the wave's own LDS: its operations complete in order).
@@ -348,20 +410,21 @@ __device__ __forceinline__ float part_cost(const PlanArgs& a, const PlanEntries&
 #pragma unroll
   for (int i = 0; i < 3; ++i)
     if (piece[i] >= 0) load += (float)longest - (float)b[i] * (1.0f / 64.0f) * (float)(longest + 1) + kPartSetup;
-  return merge + wave_most(load);
+  return merge + part_time(wave_most(load), chip);
 }
 
+// The list of a batch of one step of rows (in `rows`, tot entries), longest
+// units first, its entries split along the keys where that ends sooner.
+// Returns the list's length, or -1, with nothing written, where the row order
+// is as good: neighbouring units of a row share its keys in L2.  Every thread
+// calls it.  A batch of more than kSplitMaxUnits units keeps the row order.
+//
 // Measured (the prefill kernel alone): six turns of 44 .. 294 tokens over
 // 2 .. 16 K cached ones (32 / 8 heads, 144 units of 33 .. 249 tiles) unsplit
 // 302 us, bound by the longest unit; in parts of up to 20, 28, 40, 56 and 92
 // tiles 135, 151, 136, 150 and 139 us, and 14, 12, 9, 6 and 4 us of merge.
 // Four prompts of 0.7 .. 1.2 K over up to 3.8 K cached (488 units of up to 75
-// tiles, fp8): row by row 194 us, longest first 178, in parts of 64 171.  A
-// batch of more than kSplitMaxUnits units keeps the row order: its tail is
-// short, and neighbouring units of a row share its keys in L2.
-// The list of a batch of one step of rows (in `rows`, tot entries), longest
-// units first, its entries split along the keys where that ends sooner.
-// Returns the list's length; every thread calls it.
+// tiles, fp8): row by row 194 us, longest first 178, in parts of 64 171.
 __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& ent, bool shadow, int tot, int wgs) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int step = (a.paged && !shadow) ? a.bs / 64 : 1;
@@ -378,11 +441,19 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     ent.nt[tid] = nt;
     ent.sees[tid] = sees;
   }
+  const int wave_tiles = wave_total(nt), wave_deepest = wave_most(nt);
+  if (lane == 0) {
+    ent.tiles[w] = wave_tiles;
+    ent.deepest[w] = wave_deepest;
+  }
   if (tid < kPartBuckets) ent.bucket[tid] = 0;
   if (tid == kPartBuckets) ent.longest = ent.slots = ent.rows = 0;
   __syncthreads();
+  float least, chip;
+  const float row_order = row_order_cost(a, ent, tot, wgs, least, chip);
+  if (0.98f * row_order <= least + kPartEarly) return -1;
   {
-    const float c = part_cost(a, ent, ent.place + 64 * w, tot, part_choice(w), step, wgs, lane);
+    const float c = part_cost(a, ent, ent.place + 64 * w, tot, part_choice(w), step, wgs, chip, lane);
     if (lane == 0) ent.cost[w] = c;
   }
   __syncthreads();
@@ -390,6 +461,7 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
   const float worth = 1.0f / (1.0f + (lane < kPartChoices ? ent.cost[lane] : INFINITY));
   const float top = wave_most(worth);
   const int best = 63 - __builtin_clzll(__ballot(lane < kPartChoices && worth == top));
+  if (row_order <= ent.cost[best] + kPartWorth) return -1;
   int parts = 0, each = 0;
   if (tid < tot) {
     each = part_tiles(nt, sees, part_choice(best), step, parts);
@@ -405,10 +477,12 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     ent.sees[tid] = slot;
   }
   __syncthreads();
-  // Places by size, longest first, to a 64th of the longest; an entry's last
-  // part by its own size, as the cost has it.  Which of two parts of one bucket
-  // comes first, and the slots they take, change with the run; their outputs
-  // do not.
+  // Places by size, longest first, to a 16th of the longest (finer, the tiles
+  // of a row lie further apart in the list, and its keys are read again: 32
+  // turns of 200 tokens over 3 K sorted to a 64th 445 us, to a 16th 370); an
+  // entry's last part by its own size, as the cost has it.  Which of two parts
+  // of one bucket comes first, and the slots they take, change with the run;
+  // their outputs do not.
   int bk = 0, bk_last = 0;
   const int last = nt - (parts - 1) * each;
   if (tid < tot) {
@@ -419,9 +493,9 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     atomicAdd(&ent.bucket[bk_last], 1);
   }
   __syncthreads();
-  if (tid < kPartBuckets) {
-    const int n = ent.bucket[tid], end = wave_scan_add(n);
-    ent.bucket[tid] = end - n;
+  if (tid < 64) {
+    const int n = tid < kPartBuckets ? ent.bucket[tid] : 0, end = wave_scan_add(n);
+    if (tid < kPartBuckets) ent.bucket[tid] = end - n;
     if (tid == kPartBuckets - 1) {
       ent.list = end;
       a.plan.hdr->n_split = ent.rows;
@@ -429,12 +503,11 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
   }
   __syncthreads();
   if (tid < tot) {
-    if (parts > 1) {
-      const int at = atomicAdd(&ent.bucket[bk], parts - 1);
+    const int at = parts > 1 ? atomicAdd(&ent.bucket[bk], parts - 1) : 0;
+    const int at_last = atomicAdd(&ent.bucket[bk_last], 1);
 #pragma unroll 1
-      for (int c = 0; c < parts - 1; ++c) ent.place[at + c] = tid << 10 | c;
-    }
-    ent.place[atomicAdd(&ent.bucket[bk_last], 1)] = tid << 10 | (parts - 1);
+    for (int c = 0; c < parts - 1; ++c) ent.place[at + c] = tid << 10 | c;
+    ent.place[at_last] = tid << 10 | (parts - 1);
   }
   __syncthreads();
   const int list = ent.list;
@@ -516,6 +589,25 @@ __device__ __forceinline__ void write_plan(const PlanArgs& a, PlanLds<PARTS>& ld
   // this thread's rows: decode rows and their tiles, prefill query-key pairs
   float dec_rows = 0.0f, dec_tiles = 0.0f, pairs = 0.0f;
   bool parted = false;
+  int entries = 0;
+  // The list entries of the rows in LDS (from row b0, tot entries), row by row.
+  const auto write_rows = [&](int b0, int tot) {
+#pragma unroll 1
+    for (int e = tid; e < tot; e += kPlanThreads) {
+      int lo = 0, hi = min(kPlanThreads, a.B - b0) - 1;  // the first row whose prefix passes e
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (rows.end[mid] > e) hi = mid; else lo = mid + 1;
+      }
+      const int r = lo, rb = b0 + r;
+      const int qt = rows.end[r] - 1 - e;  // the row's first entry is its deepest tile
+      const RowFields row = {rb, rows.q0[r], rows.L[r], rows.k0[r], rows.K[r]};
+      const int blk[3] = {rows.blk[0][r], rows.blk[1][r], rows.blk[2][r]};
+      int sees;
+      pl.plist[base + e] = rb * pl.ntq + qt;
+      a.rec[base + e] = make_record(a, row, shadow, blk, qt, 0, entry_tiles(a, row.L, row.K, qt, sees), -1);
+    }
+  };
   for (int b0 = 0; b0 < a.B; b0 += kPlanThreads) {
     bool dec;
     int np, q0, kl, tot;
@@ -546,25 +638,11 @@ __device__ __forceinline__ void write_plan(const PlanArgs& a, PlanLds<PARTS>& ld
       parted = a.B <= kPlanThreads && tot > 0 && tot <= kSplitMaxEntries && tot * a.units <= kSplitMaxUnits &&
                (!a.shadow_base || shadow);
       if (parted) {  // written below
-        base = tot;
+        entries = tot;
         break;
       }
     }
-#pragma unroll 1
-    for (int e = tid; e < tot; e += kPlanThreads) {
-      int lo = 0, hi = min(kPlanThreads, a.B - b0) - 1;  // the first row whose prefix passes e
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (rows.end[mid] > e) hi = mid; else lo = mid + 1;
-      }
-      const int r = lo, rb = b0 + r;
-      const int qt = rows.end[r] - 1 - e;  // the row's first entry is its deepest tile
-      const RowFields row = {rb, rows.q0[r], rows.L[r], rows.k0[r], rows.K[r]};
-      const int blk[3] = {rows.blk[0][r], rows.blk[1][r], rows.blk[2][r]};
-      int sees;
-      pl.plist[base + e] = rb * pl.ntq + qt;
-      a.rec[base + e] = make_record(a, row, shadow, blk, qt, 0, entry_tiles(a, row.L, row.K, qt, sees), -1);
-    }
+    write_rows(b0, tot);
     __syncthreads();  // the next step's rows overwrite the LDS
     base += tot;
   }
@@ -577,10 +655,16 @@ __device__ __forceinline__ void write_plan(const PlanArgs& a, PlanLds<PARTS>& ld
   }
   if constexpr (PARTS) {
     // The work-groups that stream decode rows join late.
-    if (parted)
-      base = plan_parts(a, rows, lds.entries, shadow, base, a.co_wgs > 0 ? max(8, a.co_wgs - dec_wgs) : a.split_wgs);
-    else if (tid == 0)
-      pl.hdr->n_split = 0;
+    if (parted) {
+      base = plan_parts(a, rows, lds.entries, shadow, entries, a.co_wgs > 0 ? max(8, a.co_wgs - dec_wgs) : a.split_wgs);
+      parted = base >= 0;
+      if (!parted) {
+        base = 0;
+        write_rows(0, entries);
+        base = entries;
+      }
+    }
+    if (!parted && tid == 0) pl.hdr->n_split = 0;
   }
   if (tid == 0) {
     pl.hdr->n_prefill = base;

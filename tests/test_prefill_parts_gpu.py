@@ -17,7 +17,7 @@ from tests.gpu_util import bf16_to_np, compare, oracle_seq_rows, say
 from tests.test_code_prefill_gpu import _oracle_with_holes
 
 pytestmark = pytest.mark.gpu
-N_SPLIT = 12  # the plan header's word
+N_LIST, N_SPLIT = 0, 12  # the plan header's words
 
 
 def _workload(device, spec, Hkv, g, bs, kv, seed):
@@ -183,9 +183,35 @@ def test_list_is_longest_first(device, spec, bs):
     at = LA._lib.load().nvs_attention_workspace_bytes(
         len(spec), max(n for _, n in spec), max(p + n for p, n in spec), 32, 8, 128, 0)
     at = (at + 255) // 256 * 256
-    rec = ws[at:at + 64 * int(header[8])].view(torch.int32).cpu().reshape(-1, 16)
+    rec = ws[at:at + 64 * int(header[N_LIST])].view(torch.int32).cpu().reshape(-1, 16)
     tiles = rec[:, 9].tolist()
     assert sum(tiles) == sum((p + min(n, 64 * (t + 1)) + 63) // 64 for p, n in spec for t in range((n + 63) // 64))
     slack = max(tiles) // 16 + 1
     assert all(a + slack > b for a, b in zip(tiles, tiles[1:])), tiles
     assert max(tiles) - min(tiles) > slack  # else every order would do
+
+
+@pytest.mark.parametrize("spec,Hkv,g", [
+    ([(1536, 40 + i) for i in range(12)], 8, 4),   # a unit on every third work-group, shallow
+    ([(1536, 200 + i) for i in range(24)], 1, 8),  # even rows, most work-groups busy
+    ([(2048, 200 + i) for i in range(20)], 2, 4),
+])
+def test_even_batches_keep_the_row_order(device, spec, Hkv, g):
+    """Batches whose rows are alike and keep the chip busy gain nothing by
+    parts or another order: whole entries, row by row, deepest first."""
+    say(f"row order: Hkv={Hkv} g={g} {len(spec)} rows from {spec[0]}")
+    wl = _workload(device, spec, Hkv, g, 256, "bf16", 8)
+    out = wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    ws = LA._workspaces[wl.q.device]
+    header = ws[:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) == 0
+    at = LA._lib.load().nvs_attention_workspace_bytes(
+        len(spec), max(n for _, n in spec), max(p + n for p, n in spec), g * Hkv, Hkv, 128, 0)
+    at = (at + 255) // 256 * 256
+    rec = ws[at:at + 64 * int(header[N_LIST])].view(torch.int32).cpu().reshape(-1, 16)
+    pos = 256 // (1 << min(3, g.bit_length() - 1))
+    want = [(b, pos * t) for b, (_, n) in enumerate(spec) for t in reversed(range((n + pos - 1) // pos))]
+    assert [(r[13], r[8]) for r in rec.tolist()] == want
+    assert all(r[0] == -1 for r in rec.tolist())
+    _check(wl, bf16_to_np(out), spec[:2] if len(spec) > 2 else spec, False, "row order")
