@@ -113,29 +113,58 @@ static bool shadow_serves(const AttnParams& P) {
   return prefill_mx_serves(C);
 }
 
-// The prefill tokens a batch holds at least (a row of one token may be a
-// decode row), as units of the tile-loop kernel: with kSplitMaxUnits of them
-// its entries are not split along the keys, and no room is asked for.
-static bool may_split(int num_seqs, int64_t num_tokens, int units, int pbm) {
-  return (num_tokens - num_seqs) / pbm * units < kSplitMaxUnits;
+// Whether the entries of a batch of `tiles` key tiles a row at most may gain
+// by parts or another order: not with kSplitMaxUnits units or more (the prefill
+// tokens there are at least, a row of one token being a decode row perhaps),
+// nor with rows of fewer than kSplitRowTiles tiles and no more than a unit a
+// CU, where weighing them costs what the parts save (32/8 heads, one turn of 40
+// tokens: over 1024 cached ones 34.0 us whole, 35.5 in parts, over 1536 42.6
+// and 36.4; 12 turns over 1024 38.3 and 45.5).
+static bool may_split(int num_seqs, int64_t num_tokens, int units, int pbm, int64_t tiles) {
+  const int64_t least = (num_tokens - num_seqs) / pbm * units;
+  return least < kSplitMaxUnits && (tiles >= kSplitRowTiles || least > kSplitRound);
 }
 
-// Entries of a call served by the tile-loop kernel split along their keys,
-// if the workspace holds their slots after `offset` bytes; job->slots = 0 if
-// not.  wgs: the launch's work-groups, or 0 for a launch of prefill rows alone,
-// which takes one for each unit that there can be with the parts.
+// Entries of a call served by the tile-loop kernel split along their keys or
+// taken longest first, if the workspace holds their slots after `offset`
+// bytes; job.wgs = 0 if not.  wgs: the launch's work-groups.
 static SplitJob split_job(const AttnParams& P, const Plan& plan, int64_t offset, int wgs) {
   SplitJob job = {};
   const int units = prefill_mx_units(P.Hq, P.Hkv);
-  const int64_t entries = (int64_t)P.B * plan.ntq;
-  const int64_t slots = split_slots(entries, split_row_tiles(P.max_seqlen_k), units);
+  const int64_t entries = (int64_t)P.B * plan.ntq, tiles = split_row_tiles(P.max_seqlen_k);
+  const int64_t slots = split_slots(entries, tiles, units);
   offset = align256(offset);
-  if (slots <= 0 || !may_split(P.B, P.T, units, plan.pbm) ||
-      P.ws_bytes < offset + split_bytes(entries, slots))
+  if (slots <= 0 || !may_split(P.B, P.T, units, plan.pbm, tiles) || P.ws_bytes < offset + split_bytes(entries, slots))
     return job;
   job.at = split_at((char*)P.ws + offset, entries);
   job.slots = (int)slots;
-  job.wgs = wgs > 0 ? wgs : prefill_mx_wgs(entries * units + slots);
+  job.wgs = wgs;
+  return job;
+}
+
+// The same for prompts with nothing cached, whose parts need a merge launch
+// that whole entries do not: parts only for few units of deep rows, on one
+// work-group for each unit that there can be with them; another order, which
+// needs neither slots nor that launch, for several rows of more than a round
+// of units.  One prompt of 8/1 heads (32 query positions an entry): 1500 tokens
+// 37.5 us whole, 36.9 in parts, 2000 46.4 and 42.8, 4000 82.9 and 65.4; 16/8
+// heads, 3000 72.9 and 66.9; 32/8 heads (more units), 1500 44.0 and 50.1, 3000
+// 89.4 and 95.5.  Eight of 1100 tokens, 16/8 heads: 99.8 us in row order, 82.7
+// longest first.
+static SplitJob local_split_job(const AttnParams& P, const Plan& plan, int64_t offset) {
+  const int units = prefill_mx_units(P.Hq, P.Hkv);
+  const int64_t entries = (int64_t)P.B * plan.ntq, tiles = split_row_tiles(P.max_seqlen_k);
+  const int64_t most = std::min(entries, P.T / plan.pbm + P.B) * units;
+  if (tiles >= kSplitLocalTiles && most <= kSplitLocalUnits) {
+    const int64_t slots = split_slots(entries, tiles, units);
+    return split_job(P, plan, offset, prefill_mx_wgs(most + slots));
+  }
+  SplitJob job = {};
+  if (P.B > 1 && tiles >= 2 * kSplitMinTiles && (P.T - P.B) / plan.pbm * units > kSplitRound &&
+      may_split(P.B, P.T, units, plan.pbm, tiles)) {
+    job.at.rec = plan.rec;
+    job.wgs = prefill_mx_wgs(entries * units);
+  }
   return job;
 }
 
@@ -209,7 +238,7 @@ extern "C" int64_t nvs_attention_split_bytes(int num_seqs, int64_t num_tokens, i
   const bool known = num_kv_heads > 0 && num_heads % num_kv_heads == 0;
   const int units = known ? prefill_mx_units(num_heads, num_kv_heads) : num_heads;
   const int pbm = known ? prefill_mx_positions(num_heads / num_kv_heads) : prefill_mx_positions(8);
-  if (num_tokens > 0 && !may_split(num_seqs, num_tokens, units, pbm)) return 0;
+  if (num_tokens > 0 && !may_split(num_seqs, num_tokens, units, pbm, split_row_tiles(max_seqlen_k))) return 0;
   int64_t entries = (int64_t)num_seqs * prefill_tiles(max_seqlen_q, pbm), tiles = split_row_tiles(max_seqlen_k);
   if (num_tokens <= 0) {  // the bound covers the smaller batches, which may be split where the largest is not
     entries = std::min(entries, kSplitMaxList);
@@ -313,7 +342,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
     const int64_t base = align256(attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv));
     const SplitJob split =
         split_job(P, plan, base + (shadow ? shadow_bytes(P.B, P.max_seqlen_k, P.Hkv) : 0), co_wgs);
-    const SplitJob* sp = split.slots > 0 ? &split : nullptr;
+    const SplitJob* sp = split.wgs > 0 ? &split : nullptr;
     if (!shadow) {
       rc = launch_plan(P, plan, /*paged=*/true, s, nullptr, nullptr, &co, sp, store);
       if (rc != NVS_OK) return rc;
@@ -493,14 +522,14 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
     rc = launch_plan(P, plan, /*paged=*/false, s);
     return rc != NVS_OK ? rc : launch_prefill(P, plan, s);
   }
-  const SplitJob split = split_job(P, plan, attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv),
-                                   /*wgs=*/0);
-  const SplitJob* sp = split.slots > 0 ? &split : nullptr;
+  const SplitJob split =
+      local_split_job(P, plan, attention_workspace_bytes(P.B, P.max_seqlen_q, P.max_seqlen_k, P.Hq, P.Hkv));
+  const SplitJob* sp = split.wgs > 0 ? &split : nullptr;
   rc = launch_plan(P, plan, /*paged=*/false, s, nullptr, nullptr, nullptr, sp, store);
   if (rc != NVS_OK) return rc;
   rc = launch_prefill_mx(P, plan, s, nullptr, sp);
   if (rc != NVS_OK) return rc;
-  return sp ? launch_decode_merge(DecodeArgs{}, 0, s, &P, &plan, sp) : NVS_OK;
+  return split.slots > 0 ? launch_decode_merge(DecodeArgs{}, 0, s, &P, &plan, sp) : NVS_OK;
 }
 
 extern "C" int nvs_varlen_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride,

@@ -144,6 +144,9 @@ constexpr int kSplitSlots = 768;        // partial slots at most: three rounds o
 constexpr int kSplitMaxUnits = 1024;    // units from which a batch fills the chip without parts
 constexpr int kSplitMaxEntries = 1024;  // list entries the plan weighs, one a thread
 constexpr int kSplitMinTiles = 8;       // fewest key tiles a part is given
+constexpr int kSplitRowTiles = 21;      // key tiles of a row from which a batch of up to kSplitRound units is weighed
+constexpr int kSplitRound = 256;        // a unit for every CU
+constexpr int kSplitLocalTiles = 28, kSplitLocalUnits = 200;  // prompts with nothing cached: parts from, up to
 constexpr int kPartWaveBytes = 33792;   // one wave's part of a slot: O (64 rows x 128), m, l in fp32
 constexpr int kPartBytes = 4 * kPartWaveBytes;
 
@@ -186,8 +189,8 @@ inline SplitLayout split_at(void* p, int64_t entries) {
 // What the plan, the prefill launch and the merge need of it.
 struct SplitJob {
   SplitLayout at;
-  int slots;  // 0: entries are not split
-  int wgs;    // work-groups of the prefill launch
+  int slots;  // 0: entries are not split, only put in order
+  int wgs;    // work-groups of the prefill launch (0: entries stay whole, in row order)
 };
 
 // Decode waves a call may use: Hkv per group, at most kDecodeMaxWaves in

@@ -36,7 +36,7 @@ struct PlanArgs {
   float dec_hbm_bps;     // decode bytes per second of the whole chip
   float pre_cu_flops;    // prefill FLOP per second of one CU
   float dec_finish;      // the decode should end by this fraction of the call
-  // Entries split along the keys (split_slots > 0: the slots there are).
+  // Entries split along the keys or put in order (split_slots: the slots there are).
   PlanRecord* rec;  // the list's records
   SplitRow* split_rows;
   int split_slots, split_wgs;
@@ -786,7 +786,7 @@ int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t s
     units = merge->units;
   }
   const int grid = 1 + (units > 0 ? merge_wgs(units, m.Hkv) : 0);
-  const bool parts = a.split_slots > 0;
+  const bool parts = split != nullptr;
   const dim3 one(1), block(kPlanThreads);
   if (store)
     parts ? launch_plan_store<true>(a, *store, stream) : launch_plan_store<false>(a, *store, stream);

@@ -343,3 +343,13 @@ def test_split_bytes_unknown_tokens_is_upper_bound():
                         if g <= 16:
                             need = split(b, tokens, q, k, Hq, hk)
                             assert bound >= need, (B, max_q, max_k, b, tokens, q, k, Hq, hk, bound, need)
+
+
+def test_split_bytes_short_rows():
+    """No room is asked for short rows of up to a unit a CU (weighing their
+    parts costs what they save), nor for a batch that fills the chip."""
+    split = _lib.load().nvs_attention_split_bytes
+    assert split(4, 4 * 200, 200, 1024 + 200, 32, 8) == 0
+    assert split(4, 4 * 200, 200, 1280 + 200, 32, 8) > 0
+    assert split(40, 40 * 200, 200, 1024 + 200, 32, 8) > 0  # 976 units at least: their order may matter
+    assert split(50, 50 * 200, 200, 8192, 32, 8) == 0       # 1216

@@ -215,3 +215,26 @@ def test_even_batches_keep_the_row_order(device, spec, Hkv, g):
     assert [(r[13], r[8]) for r in rec.tolist()] == want
     assert all(r[0] == -1 for r in rec.tolist())
     _check(wl, bf16_to_np(out), spec[:2] if len(spec) > 2 else spec, False, "row order")
+
+
+def test_local_prompts_in_order_without_parts(device):
+    """Several prompts of more than a round of units, nothing cached: put
+    longest first, whole (no slots, no merge launch)."""
+    lens = [150, 90] * 6 + [2700, 2400, 2600]
+    say(f"local prompts longest first {lens}")
+    wl = _workload(device, [(0, n) for n in lens], 8, 1, 64, "bf16", 12)
+    assert wl.context.block_tables is None
+    out = wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    ws = LA._workspaces[wl.q.device]
+    header = ws[:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) == 0
+    n = sum((x + 255) // 256 for x in lens)
+    assert int(header[N_LIST]) == n
+    at = 256 + (4 * len(lens) * ((max(lens) + 255) // 256) + 255) // 256 * 256  # behind the header and the list
+    tiles = ws[at:at + 64 * n].view(torch.int32).cpu().reshape(-1, 16)[:, 9].tolist()
+    assert sorted(tiles) == sorted((min(x, 256 * (t + 1)) + 63) // 64 for x in lens for t in range((x + 255) // 256))
+    assert all(a + max(tiles) // 16 + 1 > b for a, b in zip(tiles, tiles[1:])), tiles
+    ref = AO.attention_local(*(torch.from_numpy(bf16_to_np(x)) for x in (wl.q, wl.k, wl.v)),
+                             wl.context.cu_seqlens_q.cpu(), 8, 8, 128)
+    compare(bf16_to_np(out), ref.numpy(), False, "local prompts longest first")
