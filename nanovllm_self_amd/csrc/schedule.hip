@@ -269,7 +269,7 @@ struct PlanRows {
 // (then the first slot, -1: none), tiles of a part and parts; what the
 // buckets of part sizes hold, then their next place in the list; the list's
 // places (entry << 10 | part).
-constexpr int kPartBuckets = 16;
+constexpr int kPartBuckets = 64;
 struct PlanEntries {
   int row[kSplitMaxEntries], nt[kSplitMaxEntries], sees[kSplitMaxEntries];
   int each[kSplitMaxEntries], parts[kSplitMaxEntries];
@@ -477,12 +477,10 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     ent.sees[tid] = slot;
   }
   __syncthreads();
-  // Places by size, longest first, to a 16th of the longest (finer, the tiles
-  // of a row lie further apart in the list, and its keys are read again: 32
-  // turns of 200 tokens over 3 K sorted to a 64th 445 us, to a 16th 370); an
-  // entry's last part by its own size, as the cost has it.  Which of two parts
-  // of one bucket comes first, and the slots they take, change with the run;
-  // their outputs do not.
+  // Places by size, longest first, to a 64th of the longest (a 16th: 0.2 %
+  // slower over the batches); an entry's last part by its own size, as the cost
+  // has it.  Which of two parts of one bucket comes first, and the slots they
+  // take, change with the run; their outputs do not.
   int bk = 0, bk_last = 0;
   const int last = nt - (parts - 1) * each;
   if (tid < tot) {
@@ -493,9 +491,9 @@ __device__ int plan_parts(const PlanArgs& a, const PlanRows& rows, PlanEntries& 
     atomicAdd(&ent.bucket[bk_last], 1);
   }
   __syncthreads();
-  if (tid < 64) {
-    const int n = tid < kPartBuckets ? ent.bucket[tid] : 0, end = wave_scan_add(n);
-    if (tid < kPartBuckets) ent.bucket[tid] = end - n;
+  if (tid < kPartBuckets) {
+    const int n = ent.bucket[tid], end = wave_scan_add(n);
+    ent.bucket[tid] = end - n;
     if (tid == kPartBuckets - 1) {
       ent.list = end;
       a.plan.hdr->n_split = ent.rows;
