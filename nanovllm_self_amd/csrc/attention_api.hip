@@ -348,7 +348,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
       if (rc != NVS_OK) return rc;
       rc = launch_prefill_mx(P, plan, s, &co, sp);
       if (rc != NVS_OK) return rc;
-      return launch_decode_merge(co.a, co.groups, s, &P, &plan, sp);
+      return launch_decode_merge(co.a, co.groups, P.max_seqlen_k, s, &P, &plan, sp);
     }
     // Code cache: the prefill reads the bf16 copy, the decode waves the
     // codes; they run whichever prefill kernel the plan lets serve.
@@ -369,7 +369,7 @@ static int paged_attention_impl(AttnParams& P, const void* q, int64_t q_tok_stri
       rc = launch_prefill(F, plan, s);
       if (rc != NVS_OK) return rc;
     }
-    return launch_decode_merge(co.a, co.groups, s, &P, &plan, sp);
+    return launch_decode_merge(co.a, co.groups, P.max_seqlen_k, s, &P, &plan, sp);
   }
   // With prefill rows the plan launch also merges the split decode rows.
   MergeJob merge;
@@ -529,7 +529,7 @@ static int varlen_attention_impl(const void* q, int64_t q_tok_stride, int64_t q_
   if (rc != NVS_OK) return rc;
   rc = launch_prefill_mx(P, plan, s, nullptr, sp);
   if (rc != NVS_OK) return rc;
-  return split.slots > 0 ? launch_decode_merge(DecodeArgs{}, 0, s, &P, &plan, sp) : NVS_OK;
+  return split.slots > 0 ? launch_decode_merge(DecodeArgs{}, 0, 0, s, &P, &plan, sp) : NVS_OK;
 }
 
 extern "C" int nvs_varlen_attention(const void* q, int64_t q_tok_stride, int64_t q_head_stride,

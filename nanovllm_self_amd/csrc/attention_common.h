@@ -360,8 +360,8 @@ int launch_decode(const AttnParams& P, int max_waves, int waves, void* partials,
 struct DecodeArgs;
 DecodeArgs decode_args(const AttnParams& P, int max_waves, void* partials);
 // With `split`, the same launch merges the prefill rows' parts.
-int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream, const AttnParams* P = nullptr,
-                        const Plan* plan = nullptr, const SplitJob* split = nullptr);
+int launch_decode_merge(const DecodeArgs& a, int groups, int max_seqlen_k, hipStream_t stream,
+                        const AttnParams* P = nullptr, const Plan* plan = nullptr, const SplitJob* split = nullptr);
 int launch_prefill(const AttnParams& P, const Plan& plan, hipStream_t stream);
 // The MFMA tile-loop prefill kernel (paged_prefill_mx.hip): whether it serves
 // a call, its query positions per work item for a group of g query heads,

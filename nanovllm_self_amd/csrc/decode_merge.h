@@ -171,6 +171,14 @@ struct MergeLds {
   f32x4 o[kMergeWaves][2][64];
 };
 
+// Whether a row of up to max_seqlen_k keys may have more partials than its wave
+// merges alone: its tiles, over groups of kDecodeMinUnits or more, from the
+// last tile of one on.
+inline bool merge_teams(int max_seqlen_k, int group) {
+  const int64_t tiles = ((int64_t)max_seqlen_k + kDecodeTile - 1) / kDecodeTile;
+  return (tiles + kDecodeMinUnits - 2) / kDecodeMinUnits + 1 > (group <= 4 ? kMergeAlone<1> : kMergeAlone<2>);
+}
+
 // Work-groups of a merge launch of `units` groups and kv heads.
 inline int merge_wgs(int units, int Hkv) { return (units / Hkv + kMergeWaves - 1) / kMergeWaves * Hkv; }
 
@@ -243,26 +251,31 @@ __device__ __forceinline__ MergeRow merge_row(const DecodeArgs& a, int unit, int
 // head passes) stay with one wave (33 rows of up to 14 partials: 8.0 us
 // alone, 9.5 with teams from nine on; 64 rows of about 5: 7.3, 12.5 with
 // teams from five on; the 48 rows: 16.0 with teams only from thirteen on).
-template <int NH>
-__device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units, int wg, MergeLds& lds) {
+//
+// A launch whose rows cannot have more partials than a wave merges alone
+// (merge_teams) runs without TEAMS: no LDS, no barrier (eight rows of 128 ..
+// 1024 keys, the whole call 18.2 us with both, 17.6 without).
+template <int NH, bool TEAMS>
+__device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units, int wg, MergeLds* lds) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int k = wg / a.Hkv * kMergeWaves + w;
   MergeRow r = merge_row(a, k * a.Hkv + wg % a.Hkv, units);
-  if (r.k_last >= 0 && r.k_last - r.k < kMergeAlone<NH>) {
+  if (r.k_last >= 0 && (!TEAMS || r.k_last - r.k < kMergeAlone<NH>)) {
     for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_heads<NH>(a, r, c0, lane);
     r.k_last = -1;
   }
-  if (lane == 0) lds.rows[w] = r;
+  if constexpr (!TEAMS) return;
+  if (lane == 0) lds->rows[w] = r;
   __syncthreads();
   // The longer rows, the same for every wave: one bit a unit.
-  uint32_t rest = (uint32_t)__ballot(lane < kMergeWaves && lds.rows[lane & (kMergeWaves - 1)].k_last >= 0);
+  uint32_t rest = (uint32_t)__ballot(lane < kMergeWaves && lds->rows[lane & (kMergeWaves - 1)].k_last >= 0);
   while (rest) {
     const int n = __popc(rest);
     const int waves = n == 1 ? kMergeWaves : n == 2 ? kMergeWaves / 2 : kMergeWaves / kMergeTeams;
     const int team = w / waves;
     MergeRow x = {0, 0, -1, 0, 0};
     for (int t = 0; t < kMergeWaves / waves && rest; ++t) {
-      if (t == team) x = lds.rows[__ffs(rest) - 1];
+      if (t == team) x = lds->rows[__ffs(rest) - 1];
       rest &= rest - 1;
     }
     x.k = __builtin_amdgcn_readfirstlane(x.k);
@@ -270,7 +283,7 @@ __device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units,
     x.k_last = __builtin_amdgcn_readfirstlane(x.k_last);
     x.slot_k = __builtin_amdgcn_readfirstlane(x.slot_k);
     x.q_row = __builtin_amdgcn_readfirstlane(x.q_row);
-    for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_pass<NH>(a, x, w, w % waves, waves, c0, lane, lds);
+    for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_pass<NH>(a, x, w, w % waves, waves, c0, lane, *lds);
   }
 }
 

@@ -37,6 +37,7 @@
 // checked for on the device and written, before any load, by every wave that
 // reads the cache (see write_nonconforming).
 #include <algorithm>
+#include <type_traits>
 
 #include "nvs_common.h"
 #include "attention_common.h"
@@ -80,16 +81,21 @@ void paged_decode_kernel(DecodeArgs a, const int32_t* __restrict__ bt, const int
 // (merge_split_rows).
 // Sixteen merge waves a work-group: a launch of a few large work-groups
 // is dispatched sooner than one of many single-wave ones.
-// The work-groups after the first `wgs` merge the parts of prefill entries
-// split along the keys.
-template <int NH>
+// With PARTS, the work-groups after the first `wgs` merge the parts of prefill
+// entries split along the keys.
+template <int NH, bool TEAMS, bool PARTS>
 __global__ __launch_bounds__(64 * kMergeWaves) void decode_merge_kernel(DecodeArgs a, int units, int wgs,
-                                                                        PartMergeArgs parts) {
-  __shared__ MergeLds lds;
-  if ((int)blockIdx.x < wgs)
-    merge_split_rows<NH>(a, units, (int)blockIdx.x, lds);
-  else
+                                                                        std::conditional_t<PARTS, PartMergeArgs, int> parts) {
+  if (!PARTS || (int)blockIdx.x < wgs) {
+    if constexpr (TEAMS) {
+      __shared__ MergeLds lds;
+      merge_split_rows<NH, true>(a, units, (int)blockIdx.x, &lds);
+    } else {
+      merge_split_rows<NH, false>(a, units, (int)blockIdx.x, nullptr);
+    }
+  } else if constexpr (PARTS) {
     merge_parts(parts, (int)blockIdx.x - wgs);
+  }
 }
 
 int64_t decode_workspace_bytes(int max_waves, int group) {
@@ -118,8 +124,8 @@ DecodeArgs decode_args(const AttnParams& P, int max_waves, void* partials) {
   return a;
 }
 
-int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream, const AttnParams* P, const Plan* plan,
-                        const SplitJob* split) {
+int launch_decode_merge(const DecodeArgs& a, int groups, int max_seqlen_k, hipStream_t stream, const AttnParams* P,
+                        const Plan* plan, const SplitJob* split) {
   PartMergeArgs parts = {};
   if (split && split->slots > 0) {
     parts.hdr = plan->hdr;
@@ -140,10 +146,18 @@ int launch_decode_merge(const DecodeArgs& a, int groups, hipStream_t stream, con
   const int wgs = units > 0 ? merge_wgs(units, a.Hkv) : 0;
   if (wgs + parts.wgs == 0) return NVS_OK;
   const dim3 grid(wgs + parts.wgs), block(64 * kMergeWaves);
+  const auto launch = [&](auto nh, auto teams) {
+    if (parts.wgs > 0)
+      hipLaunchKernelGGL((decode_merge_kernel<nh(), teams(), true>), grid, block, 0, stream, a, units, wgs, parts);
+    else
+      hipLaunchKernelGGL((decode_merge_kernel<nh(), teams(), false>), grid, block, 0, stream, a, units, wgs, 0);
+  };
+  using std::integral_constant;
+  const bool teams = units > 0 && merge_teams(max_seqlen_k, a.g);
   if (a.g <= 4)
-    hipLaunchKernelGGL(decode_merge_kernel<1>, grid, block, 0, stream, a, units, wgs, parts);
+    teams ? launch(integral_constant<int, 1>{}, std::true_type{}) : launch(integral_constant<int, 1>{}, std::false_type{});
   else
-    hipLaunchKernelGGL(decode_merge_kernel<2>, grid, block, 0, stream, a, units, wgs, parts);
+    teams ? launch(integral_constant<int, 2>{}, std::true_type{}) : launch(integral_constant<int, 2>{}, std::false_type{});
   return check_launch("decode_merge");
 }
 
@@ -181,7 +195,7 @@ int launch_decode(const AttnParams& P, int max_waves, int waves, void* partials,
     defer->units = groups > 1 ? (groups - 1) * P.Hkv : 0;
     return NVS_OK;
   }
-  return launch_decode_merge(a, groups, stream);
+  return launch_decode_merge(a, groups, P.max_seqlen_k, stream);
 }
 
 }  // namespace nvs

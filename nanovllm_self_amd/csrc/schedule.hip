@@ -679,7 +679,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeAr
     MergeLds merge;
   } lds;
   if (blockIdx.x > 0)
-    merge_split_rows<2>(m, merge_units, (int)blockIdx.x - 1, lds.merge);
+    merge_split_rows<2, true>(m, merge_units, (int)blockIdx.x - 1, &lds.merge);
   else
     write_plan<false>(a, lds.plan);
 }

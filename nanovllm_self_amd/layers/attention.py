@@ -50,7 +50,7 @@ def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) ->
     it must be ordered on one stream."""
     if nbytes <= 0:
         return None
-    key = torch.device(device)
+    key = device if isinstance(device, torch.device) else torch.device(device)
     buf = _workspaces.get(key)
     have = buf.numel() if buf is not None else 0
     if torch.cuda.is_current_stream_capturing():

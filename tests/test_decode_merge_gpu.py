@@ -22,6 +22,8 @@ _ROWS = {
     "three": [5000, 7003, 6500, 130, 0],
     "some": [1300 + 7 * i for i in range(24)],
     "few": [300 + 11 * i for i in range(60)],
+    # the longest rows that a launch without teams serves, and a tile more
+    "edge_one_pass": [1951, 5, 1951], "past_one_pass": [1952, 1980], "edge_two_passes": [927, 927], "past_two_passes": [928],
 }
 
 
