@@ -39,6 +39,11 @@ def _need_device(t: torch.Tensor, what: str) -> None:
         raise RuntimeError(f"{what} must be a GPU tensor for the HIP kernels (got {t.device})")
 
 
+def _int32(t: torch.Tensor) -> torch.Tensor:
+    """t as contiguous int32 (itself where it is, without a call into torch)."""
+    return t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
+
+
 def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) -> torch.Tensor | None:
     """Per-device split-K workspace, grown on demand (never inside graph capture).
 
@@ -331,8 +336,8 @@ class PagedAttention(nn.Module):
             q = q.contiguous()
         T = q.shape[0]
         out = torch.empty(T, self.num_heads, self.head_dim, dtype=compute, device=q.device)
-        cu_q = context.cu_seqlens_q.to(torch.int32).contiguous()
-        cu_k = context.cu_seqlens_k.to(torch.int32).contiguous()
+        cu_q = _int32(context.cu_seqlens_q)
+        cu_k = _int32(context.cu_seqlens_k)
         B = cu_q.numel() - 1
         scale = 1.0 / math.sqrt(self.head_dim)
         lib = _lib.load()
@@ -368,7 +373,7 @@ class PagedAttention(nn.Module):
             if store_slots is not None:  # _store_in_prefill: k / v and the cache in their types
                 kc, ks, vs = self.k_cache, self.k_scale_cache, self.v_scale_cache
                 quant = self.kv_cache_quant_mode in _QUANT_DTYPE
-                slots = store_slots.to(torch.int32).contiguous()
+                slots = _int32(store_slots)
                 _lib.check(
                     lib.nvs_varlen_attention_store(
                         q.data_ptr(), q.stride(0), q.stride(1),
@@ -406,9 +411,7 @@ class PagedAttention(nn.Module):
             vs = self.v_scale_cache if quant else None
             if quant and (ks is None or vs is None):
                 raise RuntimeError("quantised KV cache needs k_scale_cache / v_scale_cache")
-            bt = context.block_tables
-            if bt.dtype != torch.int32 or not bt.is_contiguous():
-                bt = bt.to(torch.int32).contiguous()
+            bt = _int32(context.block_tables)
             num_blocks, block_size = kc.shape[0], kc.shape[1]
             if store_slots is None:
                 _lib.check(
@@ -423,7 +426,7 @@ class PagedAttention(nn.Module):
                     "paged_attention",
                 )
             else:
-                slots = store_slots.to(torch.int32).contiguous()
+                slots = _int32(store_slots)
                 _lib.check(
                     lib.nvs_paged_attention_store(
                         q.data_ptr(), q.stride(0), q.stride(1),
