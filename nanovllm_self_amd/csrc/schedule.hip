@@ -673,13 +673,14 @@ __device__ __forceinline__ void write_plan(const PlanArgs& a, PlanLds<PARTS>& ld
 // Work-group 0 writes the plan; the others (a paged call whose decode
 // launch left its merge to this one) merge the decode rows split across
 // groups, one merge wave per wave.
+template <int NH>
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a, DecodeArgs m, int merge_units) {
   __shared__ union Lds {
     PlanLds<false> plan;
     MergeLds merge;
   } lds;
   if (blockIdx.x > 0)
-    merge_split_rows<2, true>(m, merge_units, (int)blockIdx.x - 1, &lds.merge);
+    merge_split_rows<NH, true>(m, merge_units, (int)blockIdx.x - 1, &lds.merge);
   else
     write_plan<false>(a, lds.plan);
 }
@@ -791,7 +792,7 @@ int launch_plan(const AttnParams& P, const Plan& plan, bool paged, hipStream_t s
   else if (parts)
     hipLaunchKernelGGL(plan_only_kernel<true>, one, block, 0, stream, a);
   else if (units > 0)
-    hipLaunchKernelGGL(plan_kernel, dim3(grid), block, 0, stream, a, m, units);
+    hipLaunchKernelGGL(m.g <= 4 ? plan_kernel<1> : plan_kernel<2>, dim3(grid), block, 0, stream, a, m, units);
   else
     hipLaunchKernelGGL(plan_only_kernel<false>, one, block, 0, stream, a);
   return check_launch("plan");
