@@ -693,9 +693,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_only_kernel(PlanArgs a) {
 
 // The plan by work-group 0 and the write of the step's k / v by the others:
 // neither reads what the other writes, and a small step's write (5 us) and
-// plan (4 .. 13 us) are each mostly latency.  Chosen for writes of up to two
-// work-groups a CU; a long one is bound by HBM and keeps its own launch,
-// whose small work-groups stream faster.
+// plan (4 .. 13 us) are each mostly latency.  Chosen for writes of up to four
+// work-groups a CU (the whole call, 32/8 heads, prompts of 250 tokens; a launch
+// of its own and here: 250 tokens 19.0 and 16.8 us, 4000 (500 work-groups) 38.7
+// and 35.0, 8000 (1000) 64.4 and 59.0; over fp8 4000 41.3 and 37.5, 8000 64.9
+// and 63.1, 12 000 88.0 and 88.6).
 template <bool PARTS, int SRC, int DST>
 __global__ __launch_bounds__(kPlanThreads) void plan_store_kernel(PlanArgs a, StoreArgs st) {
   __shared__ PlanLds<PARTS> lds;
@@ -714,7 +716,7 @@ static bool plan_stores(const StoreJob& job) {
 static int64_t store_wgs(const StoreJob& job) {
   return ((job.a.rows << job.a.lpr_log2) + kPlanThreads - 1) / kPlanThreads;
 }
-bool plan_launch_stores(const StoreJob& job) { return plan_stores(job) && store_wgs(job) <= device_slots(2); }
+bool plan_launch_stores(const StoreJob& job) { return plan_stores(job) && store_wgs(job) <= device_slots(4); }
 
 template <bool PARTS>
 static void launch_plan_store(const PlanArgs& a, const StoreJob& job, hipStream_t stream) {
