@@ -64,6 +64,8 @@ def test_parts_match_oracle(device, monkeypatch, Hkv, g, bs, kv, spec):
     monkeypatch.setattr(LA._lib.load(), "nvs_attention_split_bytes", lambda *a: 0)
     whole = wl.attn.prefill_flashattn(wl.q, wl.k, wl.v, wl.context)
     torch.cuda.synchronize()
+    header = LA._workspaces[wl.q.device][:256].view(torch.int32).cpu()
+    assert int(header[N_SPLIT]) == 0, "the batch was split without room"
     compare(got, bf16_to_np(whole), kv in ("int8", "fp8"), "parts vs whole")
 
 
@@ -110,6 +112,7 @@ def test_parts_in_a_graph(device):
     torch.cuda.synchronize()
     need = LA._lib.load().nvs_attention_workspace_bytes(2, 30, 16384 + 30, 32, 8, 128, 0)
     assert ws.numel() < need or LA._workspaces[wl.q.device] is ws
+    assert any(b is ws for b in LA._captured_workspaces[wl.q.device])
     assert np.all(np.isfinite(bf16_to_np(eager)))
 
 
@@ -238,3 +241,32 @@ def test_local_prompts_in_order_without_parts(device):
     ref = AO.attention_local(*(torch.from_numpy(bf16_to_np(x)) for x in (wl.q, wl.k, wl.v)),
                              wl.context.cu_seqlens_q.cpu(), 8, 8, 128)
     compare(bf16_to_np(out), ref.numpy(), False, "local prompts longest first")
+
+
+@pytest.mark.parametrize("Hkv,g,kv", [(8, 4, "bf16"), (2, 16, "fp16"), (1, 4, "int8")])
+def test_parts_into_a_strided_output(device, Hkv, g, kv):
+    """Split entries and decode rows into output rows and heads further apart
+    than they are long: the values of a contiguous output, nothing beside them."""
+    from nanovllm_self_amd import _lib
+    spec = [(6144, 67), (5000, 1), (4096, 20)]
+    say(f"parts into a strided output: heads {g * Hkv}/{Hkv} cache={kv}")
+    wl = _workload(device, spec, Hkv, g, 256, kv, 14)
+    want = wl.attn.forward(wl.q, wl.k, wl.v, wl.context)
+    torch.cuda.synchronize()
+    ws = LA._workspaces[wl.q.device]
+    assert int(ws[:256].view(torch.int32).cpu()[N_SPLIT]) > 0, "the batch was not split"
+    Hq, T, ctx, attn = g * Hkv, wl.q.shape[0], wl.context, wl.attn
+    room = torch.full((T, Hq + 3, 144), 7.0, dtype=wl.q.dtype, device=device)
+    out = room[:, 1:Hq + 1, :128]
+    _lib.check(_lib.load().nvs_paged_attention(
+        wl.q.data_ptr(), wl.q.stride(0), wl.q.stride(1), attn.k_cache.data_ptr(), attn.v_cache.data_ptr(),
+        _lib.nvs_dtype(attn.k_cache.dtype), _lib.ptr(attn.k_scale_cache), _lib.ptr(attn.v_scale_cache),
+        ctx.cu_seqlens_q.data_ptr(), ctx.cu_seqlens_k.data_ptr(), ctx.block_tables.data_ptr(), ctx.block_tables.size(1),
+        len(spec), T, int(ctx.max_seqlen_q), int(ctx.max_seqlen_k), Hq, Hkv, 128, 256, wl.num_blocks, 128 ** -0.5,
+        out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(), ws.numel(), _lib.stream_of(wl.q)),
+        "paged_attention")
+    torch.cuda.synchronize()
+    assert int(ws[:256].view(torch.int32).cpu()[N_SPLIT]) > 0, "the batch was not split"
+    assert torch.equal(out, want)
+    room[:, 1:Hq + 1, :128] = 7.0
+    assert bool((room == 7.0).all()), "written outside the output"
