@@ -44,6 +44,15 @@ def _int32(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
 
 
+def _device_key(device) -> torch.device:
+    """The device as tensors on it name it ("cuda" is the current one)."""
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
+    if device.type == "cuda" and device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    return device
+
+
 def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) -> torch.Tensor | None:
     """Per-device split-K workspace, grown on demand (never inside graph capture).
 
@@ -55,7 +64,7 @@ def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) ->
     it must be ordered on one stream."""
     if nbytes <= 0:
         return None
-    key = device if isinstance(device, torch.device) else torch.device(device)
+    key = _device_key(device)
     buf = _workspaces.get(key)
     have = buf.numel() if buf is not None else 0
     if torch.cuda.is_current_stream_capturing():
@@ -103,8 +112,8 @@ def reserve_attention_workspace(num_seqs: int, max_seqlen_q: int, max_seqlen_k: 
     n = lib.nvs_attention_workspace_bytes(num_seqs, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads, 128, 0)
     extra = lib.nvs_attention_split_bytes(num_seqs, 0, max_seqlen_q, max_seqlen_k, num_heads, num_kv_heads)
     if n > 0:
-        _no_room.pop(torch.device(device), None)
-        attention_workspace(torch.device(device), int(n), int(extra))
+        _no_room.pop(_device_key(device), None)
+        attention_workspace(device, int(n), int(extra))
 
 
 def _quantize(x: torch.Tensor, code_dtype: torch.dtype):

@@ -89,3 +89,13 @@ def test_reserved_buffer_grows_for_the_optional_bytes(memory):
     LA.reserve_attention_workspace(64, 1, 8192, 32, CPU, 8)
     reserved = LA._workspaces[CPU].numel()
     assert LA.attention_workspace(CPU, reserved, 4096).numel() == reserved + 4096
+
+
+def test_device_without_an_index_is_the_current_one(memory, monkeypatch):
+    """reserve_attention_workspace(..., "cuda") reserves what calls on tensors
+    of "cuda:1", the current device, look up."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(torch, "empty", lambda n, dtype, device: torch.zeros(n, dtype=dtype))
+    LA.reserve_attention_workspace(4, 1, 512, 16, "cuda", 8)
+    assert list(LA._workspaces) == [torch.device("cuda:1")]
+    assert LA.attention_workspace(torch.device("cuda:1"), 100) is LA._workspaces[torch.device("cuda:1")]
