@@ -64,8 +64,10 @@ def attention_workspace(device: torch.device, nbytes: int, optional: int = 0) ->
     it must be ordered on one stream."""
     if nbytes <= 0:
         return None
-    key = _device_key(device)
-    buf = _workspaces.get(key)
+    key, buf = device, _workspaces.get(device)
+    if buf is None:
+        key = _device_key(device)
+        buf = _workspaces.get(key)
     have = buf.numel() if buf is not None else 0
     if torch.cuda.is_current_stream_capturing():
         if have < nbytes:
