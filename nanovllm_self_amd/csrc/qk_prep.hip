@@ -17,19 +17,23 @@
 //
 // Work: a token's rows (units) are the Hq query heads, then the Hkv key
 // heads, then the Hkv value heads, in rounds of eight rows (a key head and its
-// value head together); one wave, a work-group of its own, takes one round of
-// one token: its four 16-lane groups take rows g and g + 4, both loads issued
-// before either is used.  Lane j holds elements 8 j .. 8 j + 7 of its head
-// (head_dim 128) as one 16-byte load, its rotary partners (elements +-64) sit
-// in lane j ^ 8, and the norm's sum is a butterfly over the row's 16 lanes.
-// The token's position, cos/sin and the norm weight are loaded once per wave
-// (from the caches after a token's first).
-// A small step is bound by latency, which a wave per round keeps to one chain
-// (a wave per token walked a 32 / 8-head token's rounds one after the other:
-// 33 tokens 9.9 -> 4.0 us, 100 of 64 / 8 heads over int8 16.6 -> 5.4, 3768 over
-// fp8 24.1 -> 20.6), a long one by HBM, whose stream many short waves keep
-// dense (34 855 tokens 148.7 -> 141 us; in work-groups of four waves with the
-// round found by a division 148, looping over tokens 199).
+// value head together): a wave's four 16-lane groups take rows g and g + 4,
+// both loads issued before either is used.  Lane j holds elements 8 j .. 8 j + 7
+// of its head (head_dim 128) as one 16-byte load, its rotary partners (elements
+// +-64) sit in lane j ^ 8, and the norm's sum is a butterfly over the row's 16
+// lanes.  The token's position, cos/sin and the norm weight are loaded once per
+// wave (from the caches after a token's first).
+//
+// A small step is bound by latency, which a wave per round
+// keeps to one chain: a wave per token walked a 32 / 8-head token's
+// rounds one after the other (33 tokens 9.9 -> 4.0 us, 100 of 64 / 8 heads over
+// int8 16.6 -> 5.4, 3768 over fp8 24.1 -> 20.6).  A long step is bound by HBM,
+// and the rounds of a token, on different XCDs, each read its rotary row: with
+// few rounds a token, and over codes (whose stores are short) with up to six,
+// a wave a token is faster again, one a work-group, in rounds of sixteen query
+// rows where there are as many heads (prep_by_token; 8 / 1 heads, 60 000 tokens
+// 69 -> 59 us, fp8 81 -> 76; 16 / 8 heads, 25 000 tokens 72 -> 68, fp8 78 -> 72;
+// 32 / 8 heads stay: 60 000 tokens 239 by round, 245 by token; fp8 254 and 238).
 #include <algorithm>
 
 #include "nvs_common.h"
@@ -41,9 +45,8 @@ namespace {
 
 constexpr int kPrepD = 128;
 constexpr int kRowLanes = 16;  // lanes per head row, 8 elements each
-constexpr int kPrepThreads = 64;  // one wave: a round of a token
-constexpr int kPrepUnroll = 2;    // rows of a lane group in a round, their loads issued together
-constexpr int64_t kPrepGridY = 65535;
+constexpr int kPrepUnroll = 2;  // rows of a lane group in a round, their loads issued together
+constexpr int64_t kPrepGridYZ = 65535;
 
 struct PrepArgs {
   const uint16_t* q;
@@ -68,7 +71,6 @@ struct PrepArgs {
   int64_t qo_ts, qo_hs;
   uint16_t* ko;  // may be null
   int64_t ko_ts, ko_hs;
-  int q_rounds;  // rounds of a token's q heads
 };
 
 // The 8 values rounded to bf16 in place, two per conversion; `bits` holds
@@ -193,36 +195,36 @@ struct PrepToken {
 };
 
 // Passes of a round of loads.
-template <int KIND>
-constexpr int kPrepPasses = KIND == 0 ? kPrepUnroll : kPrepUnroll / 2;
-template <int KIND>
+template <int KIND, int U>
+constexpr int kPrepPasses = KIND == 0 ? U : U / 2;
+template <int KIND, int U>
 __host__ __device__ __forceinline__ int prep_rounds(int H) {
-  return ((H + 3) / 4 + kPrepPasses<KIND> - 1) / kPrepPasses<KIND>;
+  return ((H + 3) / 4 + kPrepPasses<KIND, U> - 1) / kPrepPasses<KIND, U>;
 }
 
 // The token's q heads (KIND 0) or its k and v heads (KIND 1), four rows a
-// pass (head g + 4 p on lane group g), the loads of kPrepUnroll rows issued
-// before any is used (KIND 1: the k and v rows of kPrepUnroll / 2 passes).
+// pass (head g + 4 p on lane group g), the loads of U rows issued before
+// any is used (KIND 1: the k and v rows of U / 2 passes).
 // Rows past the heads re-read the last one and write nothing.  q and k rows:
 // RMSNorm (mean of squares over the 128 elements, division by 128 exact),
 // rounding to bf16, rotation, rounding to bf16; q goes to q_out, k to k_out
 // and the cache; v rows go to the cache as they are (cast or quantised).
-template <int KIND, int DST>
+template <int KIND, int DST, int U>
 __device__ __forceinline__ void prep_section(const PrepArgs& a, const PrepToken& tk, const uint16_t* src, int hs,
                                              const uint16_t* vsrc, int vhs, int H, const float (&w)[8], int g,
                                              int j, int round) {
-  constexpr int PER = kPrepPasses<KIND>;
+  constexpr int PER = kPrepPasses<KIND, U>;
   const int passes = (H + 3) / 4, p0 = round * PER;
   {
-    u32x4 xw[kPrepUnroll];
+    u32x4 xw[U];
 #pragma unroll
-    for (int k = 0; k < kPrepUnroll; ++k) {
+    for (int k = 0; k < U; ++k) {
       const bool isv = KIND == 1 && k >= PER;
       const int h = min(g + 4 * (p0 + k % PER), H - 1);
       xw[k] = prep_load(reinterpret_cast<const u32x4*>((isv ? vsrc : src) + (uint32_t)(h * (isv ? vhs : hs) + 8 * j)));
     }
 #pragma unroll
-    for (int k = 0; k < kPrepUnroll; ++k) {
+    for (int k = 0; k < U; ++k) {
       if (p0 + k % PER >= passes) continue;
       const int h = g + 4 * (p0 + k % PER);
       if (h >= H) continue;
@@ -278,11 +280,13 @@ __device__ __forceinline__ void prep_section(const PrepArgs& a, const PrepToken&
   }
 }
 
-template <int DST>
-__global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
-  const int round = blockIdx.x;
+// A wave takes round blockIdx.x of one token, TOKENS of them a work-group, or
+// all rounds of a token.
+template <int DST, int TOKENS, bool BY_TOKEN, int U>
+__global__ __launch_bounds__(64 * TOKENS) void qk_prep_kernel(PrepArgs a) {
   const int g = (threadIdx.x >> 4) & 3, j = threadIdx.x & (kRowLanes - 1);
-  const int64_t t = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
+  const int64_t t = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * TOKENS +
+                    __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (t >= a.T) return;
   PrepToken tk;
   const int64_t slot = a.slots[t];
@@ -308,11 +312,52 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
   for (int i = 0; i < 8; ++i) tk.s[i] = first ? -tk.s[i] : tk.s[i];
   tk.qo = a.qo + t * a.qo_ts;
   tk.ko = a.ko ? a.ko + t * a.ko_ts : nullptr;
-  if (round < a.q_rounds)
-    prep_section<0, DST>(a, tk, a.q + t * a.q_ts, (int)a.q_hs, nullptr, 0, a.Hq, qw, g, j, round);
+  const auto q_round = [&](int r) {
+    prep_section<0, DST, U>(a, tk, a.q + t * a.q_ts, (int)a.q_hs, nullptr, 0, a.Hq, qw, g, j, r);
+  };
+  const auto kv_round = [&](int r) {
+    prep_section<1, DST, U>(a, tk, a.k + t * a.k_ts, (int)a.k_hs, a.v + t * a.v_ts, (int)a.v_hs, a.Hkv, kw, g, j, r);
+  };
+  const int q_rounds = prep_rounds<0, U>(a.Hq);
+  if constexpr (BY_TOKEN) {
+    for (int r = 0; r < q_rounds; ++r) q_round(r);
+    for (int r = 0; r < prep_rounds<1, U>(a.Hkv); ++r) kv_round(r);
+  } else {
+    const int r = blockIdx.x;
+    if (r < q_rounds)
+      q_round(r);
+    else
+      kv_round(r - q_rounds);
+  }
+}
+
+// Whether a wave takes a whole token: long steps of few rounds (from 6000 tokens
+// by token 0 .. 25 % faster with up to four, from 12 000 over codes 1 .. 6 %
+// with up to six, slower or equal otherwise).
+bool prep_by_token(int64_t tokens, int rounds, bool codes) {
+  return rounds <= 4 ? tokens >= 6000 : codes && rounds <= 6 && tokens >= 12000;
+}
+
+template <int DST, int TOKENS, bool BY_TOKEN, int U>
+void launch_prep_as(const PrepArgs& a, int rounds, hipStream_t s) {
+  const int64_t groups = (a.T + TOKENS - 1) / TOKENS;
+  const int64_t gz = (groups + kPrepGridYZ - 1) / kPrepGridYZ, gy = (groups + gz - 1) / gz;
+  hipLaunchKernelGGL((qk_prep_kernel<DST, TOKENS, BY_TOKEN, U>), dim3((unsigned)rounds, (unsigned)gy, (unsigned)gz),
+                     dim3(64 * TOKENS), 0, s, a);
+}
+
+// A work-group takes a round of four tokens from 256 on (3000 tokens of 3 / 1
+// heads 6.4 us, 5.5 with four), of one below (64 over fp8 4.8, 5.6 with four).
+template <int DST>
+void launch_prep(const PrepArgs& a, bool by_token, int rounds, hipStream_t s) {
+  if (by_token && a.Hq >= 16)
+    launch_prep_as<DST, 1, true, 2 * kPrepUnroll>(a, 1, s);
+  else if (by_token)
+    launch_prep_as<DST, 1, true, kPrepUnroll>(a, 1, s);
+  else if (a.T >= 256)
+    launch_prep_as<DST, 4, false, kPrepUnroll>(a, rounds, s);
   else
-    prep_section<1, DST>(a, tk, a.k + t * a.k_ts, (int)a.k_hs, a.v + t * a.v_ts, (int)a.v_hs, a.Hkv, kw, g, j,
-                         round - a.q_rounds);
+    launch_prep_as<DST, 1, false, kPrepUnroll>(a, rounds, s);
 }
 
 bool is_code_dtype(int dt) { return dt == NVS_DTYPE_INT8 || dt == NVS_DTYPE_FP8_E4M3; }
@@ -361,7 +406,7 @@ extern "C" int nvs_qk_norm_rope_store(const void* q, int64_t q_tok_stride, int64
                   k_out_tok_stride >= 0 && k_out_head_stride >= 0,
               NVS_ERR_INVALID, "%s: negative stride", who);
   if (num_tokens == 0) return NVS_OK;
-  const int q_rounds = prep_rounds<0>(num_heads), rounds = q_rounds + prep_rounds<1>(num_kv_heads);
+  const int rounds = prep_rounds<0, kPrepUnroll>(num_heads) + prep_rounds<1, kPrepUnroll>(num_kv_heads);
   PrepArgs a;
   a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
   a.q_ts = q_tok_stride; a.q_hs = q_head_stride; a.k_ts = k_tok_stride; a.k_hs = k_head_stride;
@@ -371,19 +416,19 @@ extern "C" int nvs_qk_norm_rope_store(const void* q, int64_t q_tok_stride, int64
   a.cs = cos_sin_cache; a.max_pos = max_position;
   a.slots = slot_mapping; a.total_slots = num_blocks * (int64_t)block_size;
   a.kc = k_cache; a.vc = v_cache; a.ks = k_scale; a.vs = v_scale;
-  a.Hq = num_heads; a.Hkv = num_kv_heads; a.q_rounds = q_rounds;
+  a.Hq = num_heads; a.Hkv = num_kv_heads;
   a.qo = (uint16_t*)q_out; a.qo_ts = q_out_tok_stride; a.qo_hs = q_out_head_stride;
   a.ko = (uint16_t*)k_out; a.ko_ts = k_out_tok_stride; a.ko_hs = k_out_head_stride;
   hipStream_t s = (hipStream_t)stream;
-  const int64_t gy = std::min(num_tokens, kPrepGridY), gz = (num_tokens + gy - 1) / gy;
-  NVS_REQUIRE(gz <= kPrepGridY, NVS_ERR_INVALID, "%s: too many tokens (%lld)", who, (long long)num_tokens);
-  dim3 grid((unsigned)rounds, (unsigned)gy, (unsigned)gz), block(kPrepThreads);
+  const bool by_token = prep_by_token(num_tokens, rounds, is_code_dtype(cache_dtype));
+  NVS_REQUIRE(num_tokens <= kPrepGridYZ * kPrepGridYZ, NVS_ERR_INVALID, "%s: too many tokens (%lld)", who,
+              (long long)num_tokens);
   switch (cache_dtype) {
-    case NVS_DTYPE_BF16: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_BF16>, grid, block, 0, s, a); break;
-    case NVS_DTYPE_FP16: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_FP16>, grid, block, 0, s, a); break;
-    case NVS_DTYPE_FP32: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_FP32>, grid, block, 0, s, a); break;
-    case NVS_DTYPE_INT8: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_INT8>, grid, block, 0, s, a); break;
-    default: hipLaunchKernelGGL(qk_prep_kernel<NVS_DTYPE_FP8_E4M3>, grid, block, 0, s, a); break;
+    case NVS_DTYPE_BF16: launch_prep<NVS_DTYPE_BF16>(a, by_token, rounds, s); break;
+    case NVS_DTYPE_FP16: launch_prep<NVS_DTYPE_FP16>(a, by_token, rounds, s); break;
+    case NVS_DTYPE_FP32: launch_prep<NVS_DTYPE_FP32>(a, by_token, rounds, s); break;
+    case NVS_DTYPE_INT8: launch_prep<NVS_DTYPE_INT8>(a, by_token, rounds, s); break;
+    default: launch_prep<NVS_DTYPE_FP8_E4M3>(a, by_token, rounds, s); break;
   }
   return check_launch(who);
 }

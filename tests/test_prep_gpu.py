@@ -240,3 +240,31 @@ def test_rounds_past_the_grids_tokens(device, Hq, Hkv, kv):
         outs.append([qo[-110:], ko[-110:], *rows])
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T", [257, 5999, 6001, 12003])
+@pytest.mark.parametrize("Hq,Hkv,kv", [(3, 1, "bf16"), (16, 8, "fp8"), (20, 4, "int8"), (24, 8, "fp8"), (24, 8, "bf16")])
+def test_long_steps_equal_short_ones(device, Hq, Hkv, kv, T):
+    """The routes of a long step (four tokens a work-group, a wave a token, two
+    or four passes a round): its last tokens equal those of a call on them
+    alone, outputs and cache rows bit for bit."""
+    edge = slice(T - 41, T)
+    NB, bs = (T + 255) // 256 + 1, 256
+    say(f"prep routes: Hq={Hq} Hkv={Hkv} cache={kv} T={T}")
+    q, k, v, qw, kw, pos, slots = (x.to(device) for x in _inputs(T, Hq, Hkv, 10, NB, bs))
+    table = torch.randn(MAX_POS, 1, D, generator=torch.Generator().manual_seed(1)).to(device)
+    outs = []
+    for part in (slice(0, T), edge):
+        attn = _layer(Hq, Hkv, kv, NB, bs, device)
+        attn.k_cache.view(torch.uint8).zero_()
+        attn.v_cache.view(torch.uint8).zero_()
+        qo, ko = attn.qk_norm_rope_store(q[part], k[part], v[part], pos[part], qw, kw, 1e-6, table, slots[part],
+                                         want_k=True)
+        torch.cuda.synchronize()
+        at = slots[edge][slots[edge] >= 0].long()
+        rows = [c.view(torch.uint8).reshape(NB * bs, -1)[at] for c in (attn.k_cache, attn.v_cache)]
+        if attn.k_scale_cache is not None:
+            rows += [c.reshape(NB * bs, -1)[at] for c in (attn.k_scale_cache, attn.v_scale_cache)]
+        outs.append([qo[-41:], ko[-41:], *rows])
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
