@@ -157,12 +157,21 @@ __device__ __forceinline__ void merge_heads(const DecodeArgs& a, const MergeRow&
 }
 
 // A merge work-group is sixteen waves, one unit each.  A row of up to
-// kMergeAlone partials is merged by its wave; the longer
-// ones by teams of waves, the work-group's waves shared evenly among up to
-// kMergeTeams of them at a time.
+// kMergeAlone partials is merged by its wave; longer ones may be merged by
+// teams of waves, the work-group's waves shared evenly among up to kMergeTeams
+// of them at a time.
 constexpr int kMergeWaves = 16;
 template <int NH>
 constexpr int kMergeAlone = 16 / NH;
+
+// The most of sixteen lanes' values (>= 0), the same in each row of sixteen.
+__device__ __forceinline__ int most_of_16(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false));  // row_ror 8, 4, 2, 1
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x121, 0xf, 0xf, false));
+  return __builtin_amdgcn_readfirstlane(x);
+}
 constexpr int kMergeTeams = 4;
 
 struct MergeLds {
@@ -171,12 +180,18 @@ struct MergeLds {
   f32x4 o[kMergeWaves][2][64];
 };
 
-// Whether a row of up to max_seqlen_k keys may have more partials than its wave
-// merges alone: its tiles, over groups of kDecodeMinUnits or more, from the
-// last tile of one on.
+// Runs of partials that a row must have more of than a team's share of it for
+// the team to pay.
+template <int NH>
+constexpr int kTeamRuns = 4 - NH;
+
+// Whether a row of up to max_seqlen_k keys may have so many partials that a
+// team merges it (more than 16, with two head passes 12): its tiles, over
+// groups of kDecodeMinUnits or more, from the last tile of one on.
 inline bool merge_teams(int max_seqlen_k, int group) {
   const int64_t tiles = ((int64_t)max_seqlen_k + kDecodeTile - 1) / kDecodeTile;
-  return (tiles + kDecodeMinUnits - 2) / kDecodeMinUnits + 1 > (group <= 4 ? kMergeAlone<1> : kMergeAlone<2>);
+  return (tiles + kDecodeMinUnits - 2) / kDecodeMinUnits + 1 >
+         kMergeRun * (1 + (group <= 4 ? kTeamRuns<1> : kTeamRuns<2>));
 }
 
 // Work-groups of a merge launch of `units` groups and kv heads.
@@ -242,33 +257,45 @@ __device__ __forceinline__ MergeRow merge_row(const DecodeArgs& a, int unit, int
 // serves head 4 p + l / 16 of the group (pass p) and head_dim elements
 // 8 (l % 16) .. + 7; a pass over the partials keeps a running max, sum and
 // output, for NH head passes together (two for groups of more than four).
-// What bounds it is the chain of dependent loads, about 0.7 us a run of four
-// partials (1.3 us with two head passes).  With one wave a row throughout, a
-// single conversation of 20 011 keys, whose row is split across all 156
-// groups, took 62.8 us here (now 9.0), 48 rows of 256 .. 32 768 keys with 8
-// heads a group 14.1 us (13.2).  A team costs about 2 us (barriers, the
-// states' way through LDS): rows of up to sixteen partials (eight with two
-// head passes) stay with one wave (33 rows of up to 14 partials: 8.0 us
-// alone, 9.5 with teams from nine on; 64 rows of about 5: 7.3, 12.5 with
-// teams from five on; the 48 rows: 16.0 with teams only from thirteen on).
+// What bounds it is the chain of dependent loads, 0.7 .. 1.5 us a run of four
+// partials (1.3 .. 1.8 us with two head passes).  With one wave a row
+// throughout, a single conversation of 20 011 keys, whose row is split across
+// all 156 groups, took 62.8 us here (now 8.8).  A team costs as much as a few
+// runs (barriers, the states' way through LDS), and the work-group's shorter
+// rows come before it: each work-group takes teams where its longest row is
+// longer than all that (kTeamRuns), and rows of up to sixteen partials (eight
+// with two head passes) stay with one wave in any case (33 rows of up to 14
+// partials: 8.0 us alone, 9.5 with teams from nine on; 64 rows of about 5: 7.3,
+// 12.5 with teams from five on).  With teams for every row past those, whole
+// calls of rows of 17 partials beside ones of 16 were 10 .. 19 % slower than one
+// wave a row (6 rows of 2000 keys, 32/8 heads 25.9 us, 23.0 alone), of 9 beside
+// 8 with two head passes 20 .. 45 % (12 rows of 1000 keys, 32/2 heads 30.5, 21.4).
 //
-// A launch whose rows cannot have more partials than a wave merges alone
-// (merge_teams) runs without TEAMS: no LDS, no barrier (eight rows of 128 ..
-// 1024 keys, the whole call 18.2 us with both, 17.6 without).
+// A launch whose rows cannot have enough partials for a team (merge_teams) runs without TEAMS: no LDS, no barrier (eight rows of 128 ..
+// 1024 keys, GPU time of the call 15.85 us with both, 15.50 without).
 template <int NH, bool TEAMS>
 __device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units, int wg, MergeLds* lds) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int k = wg / a.Hkv * kMergeWaves + w;
-  MergeRow r = merge_row(a, k * a.Hkv + wg % a.Hkv, units);
-  if (r.k_last >= 0 && (!TEAMS || r.k_last - r.k < kMergeAlone<NH>)) {
-    for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_heads<NH>(a, r, c0, lane);
-    r.k_last = -1;
+  const MergeRow r = merge_row(a, k * a.Hkv + wg % a.Hkv, units);
+  uint32_t rest = 0;  // the rows for teams, one bit a unit, the same for every wave
+  if constexpr (TEAMS) {
+    if (lane == 0) lds->rows[w] = r;
+    __syncthreads();
+    const MergeRow& y = lds->rows[lane & (kMergeWaves - 1)];
+    const int partials = y.k_last >= 0 ? y.k_last - y.k + 1 : 0;
+    rest = (uint32_t)__ballot(lane < kMergeWaves && partials > kMergeAlone<NH>);
+    if (rest) {
+      const int n = __popc(rest), waves = n == 1 ? kMergeWaves : n == 2 ? kMergeWaves / 2 : kMergeWaves / kMergeTeams;
+      const int runs = (most_of_16(partials) + kMergeRun - 1) / kMergeRun;
+      const int before = (most_of_16(partials > kMergeAlone<NH> ? 0 : partials) + kMergeRun - 1) / kMergeRun;
+      const int rounds = (n + kMergeTeams - 1) / kMergeTeams;
+      if (runs <= before + rounds * (kTeamRuns<NH> + (runs + waves - 1) / waves)) rest = 0;
+    }
   }
+  if (r.k_last >= 0 && !(rest >> w & 1))
+    for (int c0 = 0; c0 < a.g; c0 += 4 * NH) merge_heads<NH>(a, r, c0, lane);
   if constexpr (!TEAMS) return;
-  if (lane == 0) lds->rows[w] = r;
-  __syncthreads();
-  // The longer rows, the same for every wave: one bit a unit.
-  uint32_t rest = (uint32_t)__ballot(lane < kMergeWaves && lds->rows[lane & (kMergeWaves - 1)].k_last >= 0);
   while (rest) {
     const int n = __popc(rest);
     const int waves = n == 1 ? kMergeWaves : n == 2 ? kMergeWaves / 2 : kMergeWaves / kMergeTeams;

@@ -23,7 +23,10 @@ _ROWS = {
     "some": [1300 + 7 * i for i in range(24)],
     "few": [300 + 11 * i for i in range(60)],
     # the longest rows that a launch without teams serves, and a tile more
-    "edge_one_pass": [1951, 5, 1951], "past_one_pass": [1952, 1980], "edge_two_passes": [927, 927], "past_two_passes": [928],
+    "edge_one_pass": [1951, 5, 1951], "past_one_pass": [1952, 1980],
+    # rows just past a wave's own beside shorter ones
+    "mixed_2000": [2000 + 7 * i for i in range(6)], "mixed_1000": [1000 + 7 * i for i in range(12)],
+    "edge_two_passes": [1471, 927], "past_two_passes": [1472, 1500],
 }
 
 
