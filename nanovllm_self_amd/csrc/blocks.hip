@@ -12,16 +12,18 @@
 // other (distinct destination blocks, source and destination regions
 // disjoint): the work-groups run in no particular order.
 //
-// Bound by HBM.  One wave a work-group copies 1 KiB, one 16-byte load and
-// store a lane, both non-temporal: the dispatcher hands out the next KiB as
-// soon as a wave ends, so the stream stays dense and in address order
-// (72 planes x 16 blocks of 512 KiB, 604 MB each way: 184 us, 6.55 TB/s read
-// and written).  Measured beside it: 256 threads with four loads each, 8192
-// work-groups that loop, plain stores (before) 232 / 237 us gathering /
-// scattering; the same with non-temporal stores 211 / 223; one load a
-// thread, a work-group per chunk 195 / 195 (256 threads) and 193 / 192 (128);
-// one wave with the item split by divisions instead of the grid's dimensions
-// 195 / 195, with two loads a lane 189 / 192.
+// Bound by HBM.  A work-group copies one 16-byte load and store a lane, both
+// non-temporal: the dispatcher hands out the next chunk as soon as one ends, so
+// the stream stays dense and in address order.  One wave a work-group for large
+// blocks (72 planes x 16 blocks of 512 KiB, 604 MB each way: 184 us, 6.55 TB/s
+// read and written; 195 with four waves), four for blocks of up to 256 KiB, of
+// which one-wave chunks wait for the dispatcher (72 planes x 32 blocks of 8 KiB,
+// what a code cache's scales are: 11.6 us, 9.4 with four waves, 9.8 before; of
+// 128 KiB 106 and 104, 116 before).  Measured beside it at 512 KiB, gathering /
+// scattering: 256 threads with four loads each, 8192 work-groups that loop,
+// plain stores (before) 232 / 237 us; the same with non-temporal stores 211 /
+// 223; two waves a chunk 193 / 192; one wave with the item split by divisions
+// instead of the grid's dimensions 195 / 195, with two loads a lane 189 / 192.
 #include <algorithm>
 
 #include "nvs_common.h"
@@ -29,8 +31,7 @@
 namespace nvs {
 namespace {
 
-constexpr int kCopyThreads = 64;
-constexpr int64_t kChunk = kCopyThreads * 16;
+constexpr int64_t kCopySmallBlock = 256 << 10;  // blocks of up to so many bytes are copied by four waves a chunk
 // Largest grid dimensions; the kernel loops over what lies beyond.
 constexpr int64_t kGridX = 1 << 24, kGridYZ = 65535;
 
@@ -47,7 +48,8 @@ struct CopyArgs {
 };
 
 // Work-group (chunk, copy, plane).
-__global__ __launch_bounds__(kCopyThreads) void copy_blocks_kernel(CopyArgs a) {
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void copy_blocks_kernel(CopyArgs a) {
   for (int64_t plane = blockIdx.z; plane < a.planes; plane += gridDim.z) {
     for (int64_t i = blockIdx.y; i < a.copies; i += gridDim.y) {
       const int64_t s = a.src_ids ? a.src_ids[i] : i;
@@ -56,7 +58,7 @@ __global__ __launch_bounds__(kCopyThreads) void copy_blocks_kernel(CopyArgs a) {
       const char* from = a.src + (plane * a.src_nb + s) * a.block_bytes;
       char* to = a.dst + (plane * a.dst_nb + d) * a.block_bytes;
       for (int64_t chunk = blockIdx.x; chunk < a.chunks; chunk += gridDim.x) {
-        const int64_t off = chunk * kChunk + threadIdx.x * 16;
+        const int64_t off = (chunk * THREADS + threadIdx.x) * 16;
         if (off < a.block_bytes)
           __builtin_nontemporal_store(__builtin_nontemporal_load((const u32x4*)(from + off)), (u32x4*)(to + off));
       }
@@ -84,7 +86,8 @@ extern "C" int nvs_copy_blocks(const void* src, int64_t src_num_blocks, const in
   NVS_REQUIRE(dst_block_ids || num_copies <= dst_num_blocks, NVS_ERR_INVALID,
               "%s: %lld copies into a %lld-block destination without ids", who, (long long)num_copies,
               (long long)dst_num_blocks);
-  const int64_t chunks = (block_bytes + kChunk - 1) / kChunk;
+  const int threads = block_bytes <= kCopySmallBlock ? 256 : 64;
+  const int64_t chunks = (block_bytes + threads * 16 - 1) / (threads * 16);
   if (num_planes == 0 || num_copies == 0) return NVS_OK;
   NVS_REQUIRE(src && dst, NVS_ERR_INVALID, "%s: null pointer argument", who);
   NVS_REQUIRE(((uintptr_t)src % 16) == 0 && ((uintptr_t)dst % 16) == 0, NVS_ERR_INVALID,
@@ -96,6 +99,7 @@ extern "C" int nvs_copy_blocks(const void* src, int64_t src_num_blocks, const in
   a.block_bytes = block_bytes; a.chunks = chunks; a.copies = num_copies; a.planes = num_planes;
   const dim3 grid((unsigned)std::min(chunks, kGridX), (unsigned)std::min(num_copies, kGridYZ),
                   (unsigned)std::min(num_planes, kGridYZ));
-  hipLaunchKernelGGL(copy_blocks_kernel, grid, dim3(kCopyThreads), 0, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(threads == 256 ? copy_blocks_kernel<256> : copy_blocks_kernel<64>, grid, dim3(threads), 0,
+                     (hipStream_t)stream, a);
   return check_launch(who);
 }

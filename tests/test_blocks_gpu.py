@@ -91,6 +91,7 @@ def test_round_trip_and_errors(device):
 @pytest.mark.parametrize("planes,nb,copies,block_bytes", [
     (2, 9, 5, 16), (3, 4, 4, 1008), (2, 3, 2, 1024 + 16), (1, 2, 2, 5 * 1024 - 16),  # remainders of a 1 KiB chunk
     (1, 70001, 70001, 16), (65537, 1, 1, 16),  # past the grid's copies and planes
+    (2, 3, 2, 4096 - 16), (2, 3, 2, 4096 + 16), (1, 3, 2, 256 * 1024), (1, 3, 2, 256 * 1024 + 16),  # either chunk's edge
 ])
 def test_copy_blocks_sizes(device, planes, nb, copies, block_bytes):
     from nanovllm_self_amd import _lib
