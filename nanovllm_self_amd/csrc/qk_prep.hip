@@ -285,8 +285,8 @@ __device__ __forceinline__ void prep_section(const PrepArgs& a, const PrepToken&
 template <int DST, int TOKENS, bool BY_TOKEN, int U>
 __global__ __launch_bounds__(64 * TOKENS) void qk_prep_kernel(PrepArgs a) {
   const int g = (threadIdx.x >> 4) & 3, j = threadIdx.x & (kRowLanes - 1);
-  const int64_t t = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * TOKENS +
-                    __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int64_t t = (int64_t)blockIdx.z * gridDim.y + blockIdx.y;
+  if constexpr (TOKENS > 1) t = t * TOKENS + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (t >= a.T) return;
   PrepToken tk;
   const int64_t slot = a.slots[t];
@@ -347,14 +347,17 @@ void launch_prep_as(const PrepArgs& a, int rounds, hipStream_t s) {
 }
 
 // A work-group takes a round of four tokens from 256 on (3000 tokens of 3 / 1
-// heads 6.4 us, 5.5 with four), of one below (64 over fp8 4.8, 5.6 with four).
+// heads 6.4 us, 5.5 with four), of one below (64 over fp8 4.8, 5.6 with four)
+// and from 12 000 on: 32 / 8 heads over bf16 148.4 us with one, 151.6 with four
+// at 36 864 tokens (238.9, 241.0 at 60 000; medians of three runs a side in
+// turn); fewer heads and fp8 are the same either way within their spread.
 template <int DST>
 void launch_prep(const PrepArgs& a, bool by_token, int rounds, hipStream_t s) {
   if (by_token && a.Hq >= 16)
     launch_prep_as<DST, 1, true, 2 * kPrepUnroll>(a, 1, s);
   else if (by_token)
     launch_prep_as<DST, 1, true, kPrepUnroll>(a, 1, s);
-  else if (a.T >= 256)
+  else if (a.T >= 256 && a.T < 12000)
     launch_prep_as<DST, 4, false, kPrepUnroll>(a, rounds, s);
   else
     launch_prep_as<DST, 1, false, kPrepUnroll>(a, rounds, s);
