@@ -271,8 +271,9 @@ __device__ __forceinline__ MergeRow merge_row(const DecodeArgs& a, int unit, int
 // wave a row (6 rows of 2000 keys, 32/8 heads 25.9 us, 23.0 alone), of 9 beside
 // 8 with two head passes 20 .. 45 % (12 rows of 1000 keys, 32/2 heads 30.5, 21.4).
 //
-// A launch whose rows cannot have enough partials for a team (merge_teams) runs without TEAMS: no LDS, no barrier (eight rows of 128 ..
-// 1024 keys, GPU time of the call 15.85 us with both, 15.50 without).
+// A launch whose rows cannot have enough partials for a team (merge_teams) runs
+// without TEAMS: no LDS, no barrier (eight rows of 128 .. 1024 keys, GPU time of
+// the call 15.85 us with both, 15.50 without).
 template <int NH, bool TEAMS>
 __device__ __forceinline__ void merge_split_rows(const DecodeArgs& a, int units, int wg, MergeLds* lds) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));

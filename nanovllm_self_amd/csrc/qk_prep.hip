@@ -331,6 +331,8 @@ __global__ __launch_bounds__(64 * TOKENS) void qk_prep_kernel(PrepArgs a) {
   }
 }
 
+bool is_code_dtype(int dt) { return dt == NVS_DTYPE_INT8 || dt == NVS_DTYPE_FP8_E4M3; }
+
 // Whether a wave takes a whole token: long steps of few rounds (from 6000 tokens
 // by token 0 .. 25 % faster with up to four, from 12 000 over codes 1 .. 6 %
 // with up to six, slower or equal otherwise).
@@ -347,23 +349,24 @@ void launch_prep_as(const PrepArgs& a, int rounds, hipStream_t s) {
 }
 
 // A work-group takes a round of four tokens from 256 on (3000 tokens of 3 / 1
-// heads 6.4 us, 5.5 with four), of one below (64 over fp8 4.8, 5.6 with four)
-// and from 12 000 on: 32 / 8 heads over bf16 148.4 us with one, 151.6 with four
-// at 36 864 tokens (238.9, 241.0 at 60 000; medians of three runs a side in
-// turn); fewer heads and fp8 are the same either way within their spread.
+// heads 6.4 us with one, 5.4 with four), of one below (64 over fp8 4.8, 5.6 with
+// four) and where the launch has waves to fill the chip over and over, which
+// lies lower over codes: their waves last longer.  One and four, medians of
+// three runs a side: bf16 32 / 8 heads 2000 tokens (12 000 waves) 12.3, 11.8;
+// 48 / 8 6000 tokens (48 000) 35.7, 36.3; 32 / 8 36 864 tokens 148.4, 151.6.
+// fp8 32 / 8 1200 tokens (7200) 10.0, 9.2; 2000 (12 000) 13.6, 14.0; 64 / 8
+// 7500 (75 000) 55.5, 57.9.  The other way: 16 / 8 bf16 3000 (12 000) 12.2, 12.5.
 template <int DST>
 void launch_prep(const PrepArgs& a, bool by_token, int rounds, hipStream_t s) {
   if (by_token && a.Hq >= 16)
     launch_prep_as<DST, 1, true, 2 * kPrepUnroll>(a, 1, s);
   else if (by_token)
     launch_prep_as<DST, 1, true, kPrepUnroll>(a, 1, s);
-  else if (a.T >= 256 && a.T < 12000)
+  else if (a.T >= 256 && a.T * rounds < (is_code_dtype(DST) ? 10000 : 24000))
     launch_prep_as<DST, 4, false, kPrepUnroll>(a, rounds, s);
   else
     launch_prep_as<DST, 1, false, kPrepUnroll>(a, rounds, s);
 }
-
-bool is_code_dtype(int dt) { return dt == NVS_DTYPE_INT8 || dt == NVS_DTYPE_FP8_E4M3; }
 
 }  // namespace
 }  // namespace nvs
